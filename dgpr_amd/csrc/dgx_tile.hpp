@@ -17,7 +17,11 @@
 //   * the trace records of the new state are produced the same way.
 // LDS per face point: the tangential dual-consistency fluxes (8 doubles),
 // then the projected face term and the normal flux (9 doubles), in one
-// 64 x 9 region shared with the volume divergence and the trace exchange.
+// 9 x 64 region shared with the volume divergence and the trace exchange.
+// The exchanges are stored by component ([component][lane]): consecutive lanes
+// hit consecutive banks, where 8 and 4 doubles per lane gave 4-way conflicts
+// (32^3 p = 3 cube, per RK4 stage: 225 against 231 us; FP32-MFMA form 206
+// against 214 us).
 // Included by dgx_stage.hpp inside namespace dgx, after stage_body and its
 // helpers.
 #pragma once
@@ -169,9 +173,9 @@ __device__ __forceinline__ void tile_face_subpass(
 #pragma unroll
     for (int r = 0; r < 4; ++r)
     {
-      hn[r]              = hc[D][r];
-      sR[tid * 8 + r]     = hc[T1][r];
-      sR[tid * 8 + 4 + r] = hc[T2][r];
+      hn[r]                  = hc[D][r];
+      sR[r * 64 + tid]       = hc[T1][r];
+      sR[(4 + r) * 64 + tid] = hc[T2][r];
     }
   }
   __syncthreads();
@@ -185,8 +189,8 @@ __device__ __forceinline__ void tile_face_subpass(
 #pragma unroll
       for (int m = 0; m < N; ++m)
       {
-        t -= pt.Dg[m][a] * sR[(fbase + m + N * b) * 8 + (r - 1)];
-        t -= pt.Dg[m][b] * sR[(fbase + a + N * m) * 8 + 4 + (r - 1)];
+        t -= pt.Dg[m][a] * sR[(r - 1) * 64 + fbase + m + N * b];
+        t -= pt.Dg[m][b] * sR[(3 + r) * 64 + fbase + a + N * m];
       }
       G[r] = t;
     }
@@ -196,10 +200,10 @@ __device__ __forceinline__ void tile_face_subpass(
   {
 #pragma unroll
     for (int r = 0; r < 5; ++r)
-      sR[tid * 9 + r] = G[r];
+      sR[r * 64 + tid] = G[r];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      sR[tid * 9 + 5 + r] = hn[r];
+      sR[(5 + r) * 64 + tid] = hn[r];
   }
   __syncthreads();
   // gather: each node takes its element's low and high face of direction D
@@ -220,10 +224,10 @@ __device__ __forceinline__ void tile_face_subpass(
         if (gg / FPS != sp)
           continue;
         const int fp = (gg % FPS) * NF + idx[T2] * N + idx[T1];
-        acc[rr][0] += pt.L[h][m] * sR[fp * 9];
+        acc[rr][0] += pt.L[h][m] * sR[fp];
 #pragma unroll
         for (int r = 1; r < 5; ++r)
-          acc[rr][r] += pt.L[h][m] * sR[fp * 9 + r] - pt.Ld[h][m] * sR[fp * 9 + 4 + r];
+          acc[rr][r] += pt.L[h][m] * sR[r * 64 + fp] - pt.Ld[h][m] * sR[(4 + r) * 64 + fp];
       }
     }
   }
@@ -276,8 +280,8 @@ __device__ __forceinline__ void tile_trace_subpass(
       U[r] = v;
       if (r < 4)
       {
-        dn[r]           = dv;
-        sR[tid * 4 + r] = v;
+        dn[r]            = dv;
+        sR[r * 64 + tid] = v;
       }
     }
   }
@@ -298,8 +302,8 @@ __device__ __forceinline__ void tile_trace_subpass(
 #pragma unroll
       for (int m = 0; m < N; ++m)
       {
-        d1 += pt.Dg[a][m] * sR[(fbase + m + N * b) * 4 + r];
-        d2 += pt.Dg[b][m] * sR[(fbase + a + N * m) * 4 + r];
+        d1 += pt.Dg[a][m] * sR[r * 64 + fbase + m + N * b];
+        d2 += pt.Dg[b][m] * sR[r * 64 + fbase + a + N * m];
       }
       gr[D][r]  = dn[r];
       gr[T1][r] = d1;
