@@ -119,17 +119,17 @@ hipError_t stage(dgx_ctx* c, const Phys& ph, const double* Vin, const double* Ti
 // one RK4 step of the context's state (the dgx_step path)
 hipError_t step_ctx(dgx_ctx* c, double dt)
 {
-  hipError_t e = ensure_traces(c);
+  hipError_t e = ensure_stage_inputs(c);
   if (e != hipSuccess)
     return e;
-  c->tu_valid = false;
+  drop_traces(c);
   StageArgs sa[4];
   int ns = stage_plan(c, DGX_RK4, dt, sa);
   for (int k = 0; k < ns && e == hipSuccess; ++k)
     e = rhs_dispatch(c->p, c->q, mesh_args(c), c->phys, sa[k], c->lam, c->status,
                      c->stage_waves, c->stream, c->stage_tile);
   if (e == hipSuccess)
-    c->tu_valid = true;
+    stage_outputs_valid(c);
   return e;
 }
 
@@ -461,7 +461,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
     if (st != DGX_OK)
       return st;
     AHIP(c, copy_state(c, c->U, final_state.p));
-    c->tu_valid = false;
+    drop_traces(c);
   }
   else
   {
@@ -478,7 +478,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
         if (st != DGX_OK)
           return st;
         AHIP(c, copy_state(c, c->U, final_state.p));
-        c->tu_valid = false;
+        drop_traces(c);
         break;
       }
       AHIP(c, step_ctx(c, dt));
@@ -537,7 +537,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
     {
       const uint64_t s0 = sg * K, s1 = (s0 + K < nsteps) ? s0 + K : nsteps;
       AHIP(c, copy_state(c, c->U, chk[sg].p));
-      c->tu_valid = false;
+      drop_traces(c);
       for (uint64_t s = s0; s < s1; ++s)
       {
         AHIP(c, copy_state(c, seg[s - s0].p, c->U));
@@ -579,7 +579,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   }
   // the context ends at the final state, as after dgx_step
   AHIP(c, copy_state(c, c->U, final_state.p));
-  c->tu_valid = false;
+  drop_traces(c);
   AHIP(c, hipStreamSynchronize(c->stream));
   int h = 0;
   AHIP(c, hipMemcpy(&h, c->status, sizeof(int), hipMemcpyDeviceToHost));

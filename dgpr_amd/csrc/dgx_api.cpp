@@ -44,11 +44,31 @@ static dgx_status fail(dgx_ctx* c, dgx_status st, const char* fmt, ...)
       return fail((ctx), DGX_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));      \
   } while (0)
 
-// Occupancy target per (p, q): 3 waves/SIMD where the stage kernel fits the
-// 168-register budget without spilling (p=3, q=1), 2 elsewhere.
+// Occupancy target of the record-reading kernels per (p, q): 3 waves/SIMD
+// where the stage kernel fits the 168-register budget without spilling (p=3,
+// q=1), 2 elsewhere.
 int dgx::default_stage_waves(int p, int q)
 {
   return (p == 3 && q == 1) ? 3 : 2;
+}
+
+// Stage kernel and occupancy target of a context, where the caller has not
+// chosen them.  q = 1 in FP64: the state-reading tiled kernel at p = 1 and 3, at
+// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1313
+// against 2166 us per RK4 stage on the 64^3 p = 3 cube, 299 against 437 us on
+// the 64^3 p = 1 cube, 146 against 195 us on a 61x37x43 p = 1 channel.  The
+// mixed forms: the record-reading tiled kernel at p = 3, q = 1 (3 waves per
+// SIMD on affine meshes, 2 on curved ones, where 3 spills).  The general-order
+// kernel (tile 2) outside 1 <= p, q <= 3, the one-row kernel elsewhere.
+static void apply_defaults(dgx_ctx* c)
+{
+  const bool fp64 = c->prec == DGX_PREC_FP64;
+  if (!c->tile_chosen)
+    c->stage_tile = general_order(c->p, c->q) ? 2
+                  : (c->q == 1 && (c->p == 3 || (c->p == 1 && fp64))) ? 1 : 0;
+  if (!c->waves_chosen)
+    c->stage_waves = c->stage_tile != 1 ? default_stage_waves(c->p, c->q)
+                                        : (!fp64 && c->p == 3 && c->affine ? 3 : 2);
 }
 
 static void derive_phys(const dgx_params& p, Phys& ph)
@@ -83,6 +103,7 @@ MeshArgs dgx::mesh_args(const dgx_ctx* c)
     m.bounds[i] = c->bounds[i];
   m.affine = c->affine;
   m.lamf   = c->lamf;
+  m.arec   = c->arec;
   return m;
 }
 
@@ -147,6 +168,8 @@ static dgx_status ensure_tables(int device)
     built = true;
   }
   hipError_t e = upload_tables(pt, qt);
+  if (e == hipSuccess)
+    e = upload_tables_tile(pt, qt);
   if (e == hipSuccess)
     e = upload_tables_ensemble(pt, qt);
   if (e == hipSuccess)
@@ -278,16 +301,12 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   for (int i = 0; i < 3; ++i)
     if ((e = hipMalloc(tbufs[i], tb)) != hipSuccess)
       return bail("hipMalloc(traces)", e);
-  c->tu_valid = false;
-  // the tiled kernel at p = 3, q = 1 (measured 14 % faster than the one-row
-  // kernel on the 64^3 cube at 3 waves per SIMD, 7 % on the curved channel
-  // at 2, where 3 spills); the one-row kernel at the other orders of
-  // 1..3; the general-order kernel (tile 2) outside them
-  c->stage_tile  = general_order(c->p, c->q) ? 2 : ((c->p == 3 && c->q == 1) ? 1 : 0);
-  c->stage_waves = c->stage_tile == 1 ? (c->affine ? 3 : 2) : default_stage_waves(c->p, c->q);
+  drop_traces(c);
   c->prec = DGX_PREC_FP64;
+  apply_defaults(c);
   c->bytes = 5 * sb + 3 * tb +
-             (nn + nlam + (c->affine ? (size_t)c->nelem * 6 : 0) + (size_t)c->npartial +
+             (nn + nlam +
+              (c->affine ? (size_t)c->nelem * 6 + affine_record_doubles(c->nelem) : 0) + (size_t)c->npartial +
               sum_scratch(c->npartial)) * sizeof(double) + 16;
   if ((e = hipMemcpyAsync(c->nodes, mesh->nodes, nn * sizeof(double), hipMemcpyHostToDevice,
                           c->stream)) != hipSuccess)
@@ -302,6 +321,10 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
       return bail("hipMalloc(lamf)", e);
     if ((e = lift_face_dispatch(c->p, c->lam, c->nelem, c->lamf, c->stream)) != hipSuccess)
       return bail("face lifting coefficients", e);
+    if ((e = hipMalloc(&c->arec, affine_record_doubles(c->nelem) * sizeof(double))) != hipSuccess)
+      return bail("hipMalloc(arec)", e);
+    if ((e = affine_record_dispatch(c->nodes, c->nelem, c->arec, c->stream)) != hipSuccess)
+      return bail("affine records", e);
   }
   if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);
@@ -317,8 +340,8 @@ dgx_status dgx_destroy(dgx_ctx* c)
     return DGX_OK;
   if (c->stream)
     (void)hipStreamSynchronize(c->stream);
-  double* bufs[14] = {c->U,   c->Ua,  c->Ub,  c->acc, c->fs,  c->nodes, c->partial,
-                      c->sum, c->lam, c->lamf, c->TU, c->TUa, c->TUb, c->mean};
+  double* bufs[15] = {c->U,   c->Ua,  c->Ub,   c->acc, c->fs,  c->nodes, c->partial, c->sum,
+                      c->lam, c->lamf, c->arec, c->TU, c->TUa, c->TUb,   c->mean};
   for (double* b : bufs)
     if (b)
       (void)hipFree(b);
@@ -340,7 +363,7 @@ dgx_status dgx_set_params(dgx_ctx* c, const dgx_params* params)
     return fail(c, DGX_ERR_INVALID, "invalid reference state");
   c->params = *params;
   derive_phys(*params, c->phys);
-  c->tu_valid = false;  // the gradient tractions scale with mu
+  drop_traces(c);  // the gradient tractions scale with mu
   return DGX_OK;
 }
 
@@ -376,7 +399,7 @@ dgx_status dgx_set_state_device(dgx_ctx* c, const double* U_dev)
   if (!c || !U_dev)
     return DGX_ERR_INVALID;
   HIPCHK(c, basis_dispatch(c->p, U_dev, c->U, c->nelem, 0, c->stream));
-  c->tu_valid = false;
+  drop_traces(c);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return DGX_OK;
 }
@@ -397,7 +420,7 @@ dgx_status dgx_set_state(dgx_ctx* c, const double* U_host)
   HIPCHK(c, hipMemcpyAsync(c->Ua, U_host, c->nstate * sizeof(double), hipMemcpyHostToDevice,
                            c->stream));
   HIPCHK(c, basis_dispatch(c->p, c->Ua, c->U, c->nelem, 0, c->stream));
-  c->tu_valid = false;
+  drop_traces(c);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return DGX_OK;
 }
@@ -433,6 +456,7 @@ static hipError_t rhs(dgx_ctx* c, const double* Vin, const double* Tin, const do
   sa.accmode = accmode;
   sa.trace32 = c->prec != DGX_PREC_FP64;
   sa.ctype   = c->prec == DGX_PREC_MIXED ? 1 : (c->prec == DGX_PREC_MIXED_BF16 ? 2 : 0);
+  sa.records = !reads_states(c);
   return rhs_dispatch(c->p, c->q, mesh_args(c), c->phys, sa, c->lam, c->status, c->stage_waves,
                       c->stream, c->stage_tile);
 }
@@ -447,7 +471,23 @@ hipError_t dgx::ensure_traces(dgx_ctx* c)
   hipError_t e = trace_dispatch(c->p, c->q, mesh_args(c), c->phys, c->U, c->TU, c->status,
                                 c->stream, c->prec != DGX_PREC_FP64);
   if (e == hipSuccess)
-    c->tu_valid = true;
+    c->tu_valid = c->tb_valid = true;
+  return e;
+}
+
+hipError_t dgx::ensure_stage_inputs(dgx_ctx* c)
+{
+  return reads_states(c) ? ensure_boundary(c) : ensure_traces(c);
+}
+
+// Boundary states of U (q = 1), recomputed when U was set from outside.
+hipError_t dgx::ensure_boundary(dgx_ctx* c)
+{
+  if (c->tb_valid)
+    return hipSuccess;
+  hipError_t e = boundary_dispatch(c->p, mesh_args(c), c->phys, c->U, c->TU, c->status, c->stream);
+  if (e == hipSuccess)
+    c->tb_valid = true;
   return e;
 }
 
@@ -471,8 +511,12 @@ dgx_status dgx_residual_device(dgx_ctx* c, const double* U_dev, double* R_dev, d
   if (!c || !U_dev || !f_dev)
     return DGX_ERR_INVALID;
   HIPCHK(c, basis_dispatch(c->p, U_dev, c->Ua, c->nelem, 0, c->stream));
-  HIPCHK(c, trace_dispatch(c->p, c->q, mesh_args(c), c->phys, c->Ua, c->TUa, c->status,
-                           c->stream, c->prec != DGX_PREC_FP64));
+  const bool t32 = c->prec != DGX_PREC_FP64;
+  if (reads_states(c))
+    HIPCHK(c, boundary_dispatch(c->p, mesh_args(c), c->phys, c->Ua, c->TUa, c->status, c->stream));
+  else
+    HIPCHK(c, trace_dispatch(c->p, c->q, mesh_args(c), c->phys, c->Ua, c->TUa, c->status,
+                             c->stream, t32));
   HIPCHK(c, rhs(c, c->Ua, c->TUa, nullptr, nullptr, nullptr, nullptr, c->fs, 0, 0, 0, 0));
   HIPCHK(c, resid_out_dispatch(c->p, c->q, mesh_args(c), c->fs, f_dev, R_dev, nullptr,
                                c->stream));
@@ -483,7 +527,7 @@ dgx_status dgx_residual(dgx_ctx* c, double* R_host, double* f_host)
 {
   if (!c || !f_host)
     return DGX_ERR_INVALID;
-  HIPCHK(c, ensure_traces(c));
+  HIPCHK(c, ensure_stage_inputs(c));
   HIPCHK(c, rhs(c, c->U, c->TU, nullptr, nullptr, nullptr, nullptr, c->fs, 0, 0, 0, 0));
   HIPCHK(c, resid_out_dispatch(c->p, c->q, mesh_args(c), c->fs, c->Ua, R_host ? c->Ub : nullptr,
                                nullptr, c->stream));
@@ -504,7 +548,8 @@ int dgx::stage_plan(const dgx_ctx* c, int scheme, double dt, StageArgs sa[4])
 {
   const int t32 = c->prec != DGX_PREC_FP64;
   const int ct  = c->prec == DGX_PREC_MIXED ? 1 : (c->prec == DGX_PREC_MIXED_BF16 ? 2 : 0);
-  auto set = [t32, ct](StageArgs& a, const double* Vin, const double* Tin, const double* Vbase,
+  const int rec = !reads_states(c);
+  auto set = [t32, ct, rec](StageArgs& a, const double* Vin, const double* Tin, const double* Vbase,
                    double* acc, double* Vout, double* Tout, double ca, double cb, double cf,
                    int accmode) {
     a.Vin = Vin;
@@ -520,6 +565,7 @@ int dgx::stage_plan(const dgx_ctx* c, int scheme, double dt, StageArgs sa[4])
     a.accmode = accmode;
     a.trace32 = t32;
     a.ctype   = ct;
+    a.records = rec;
   };
   // the first stage's base is its own input: cb = 1 takes it from the LDS
   // copy the kernel already holds instead of reading U from HBM again
@@ -549,9 +595,9 @@ static hipError_t launch_step(dgx_ctx* c, int scheme, double dt, bool want_norm,
                               double* norm_dev = nullptr)
 {
   hipError_t e;
-  if ((e = ensure_traces(c)) != hipSuccess)
+  if ((e = ensure_stage_inputs(c)) != hipSuccess)
     return e;
-  c->tu_valid = false;  // until the last stage has rewritten them
+  drop_traces(c);  // until the last stage has rewritten them
   StageArgs sa[4];
   int ns = stage_plan(c, scheme, dt, sa);
   const bool fused = want_norm && c->stage_tile == 1;
@@ -577,7 +623,7 @@ static hipError_t launch_step(dgx_ctx* c, int scheme, double dt, bool want_norm,
         return e;
     }
   }
-  c->tu_valid = true;
+  stage_outputs_valid(c);
   return hipSuccess;
 }
 
@@ -641,7 +687,8 @@ dgx_status dgx_set_precision(dgx_ctx* c, int precision)
   if (precision != c->prec)
   {
     c->prec = precision;
-    c->tu_valid = false;
+    apply_defaults(c);
+    drop_traces(c);
   }
   return DGX_OK;
 }
@@ -658,7 +705,8 @@ dgx_status dgx_set_tuning(dgx_ctx* c, int stage_waves)
 {
   if (!c || stage_waves < 1 || stage_waves > 3 || !tile_valid(c->p, c->q, c->stage_tile, stage_waves))
     return DGX_ERR_INVALID;
-  c->stage_waves = stage_waves;
+  c->stage_waves  = stage_waves;
+  c->waves_chosen = true;
   return DGX_OK;
 }
 
@@ -677,7 +725,9 @@ dgx_status dgx_set_tile(dgx_ctx* c, int tile)
   if (!tile_valid(c->p, c->q, tile, 2))
     return fail(c, DGX_ERR_UNSUPPORTED, "no stage kernel of tile %d for p = %d, q = %d", tile,
                 c->p, c->q);
-  c->stage_tile = tile;
+  c->stage_tile  = tile;
+  c->tile_chosen = true;
+  apply_defaults(c);
   if (!tile_valid(c->p, c->q, tile, c->stage_waves))
     c->stage_waves = 2;  // the tiled kernels are compiled for 2 and 3 waves per SIMD
   return DGX_OK;
@@ -698,7 +748,7 @@ dgx_status dgx_autotune(dgx_ctx* c, int reps, int* chosen, double us_out[3])
 {
   if (!c || reps < 1)
     return DGX_ERR_INVALID;
-  HIPCHK(c, ensure_traces(c));
+  HIPCHK(c, ensure_stage_inputs(c));
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
@@ -745,6 +795,8 @@ dgx_status dgx_autotune(dgx_ctx* c, int reps, int* chosen, double us_out[3])
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   c->stage_waves = (st == DGX_OK) ? best : keep;
+  if (st == DGX_OK)
+    c->waves_chosen = true;
   if (chosen)
     *chosen = c->stage_waves;
   if (st != DGX_OK)
@@ -792,6 +844,7 @@ dgx_status dgx_autotune_tiles(dgx_ctx* c, int reps, int* tile_out, int* waves_ou
   }
   c->stage_tile  = best_tile;
   c->stage_waves = best_waves;
+  c->tile_chosen = true;
   if (tile_out)
     *tile_out = best_tile;
   if (waves_out)

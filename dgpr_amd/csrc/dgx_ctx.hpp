@@ -29,12 +29,15 @@ struct dgx_ctx
   double* sum;      // reduced sum
   double* lam;      // BR2 lifting coefficients [e][6][(p+1)^2]
   double* lamf;     // affine meshes: one coefficient per element face [e][6]
+  double* arec;     // affine meshes: each element's constant geometry
   double* TU;       // face trace records of U, Ua, Ub [e][6][8][(p+1)^2]
   double* TUa;
   double* TUb;
   bool tu_valid;    // TU holds the traces of the current U
+  bool tb_valid;    // TU holds its boundary states (all the tiled kernel reads)
   int stage_waves;  // occupancy target of the stage kernel (1..3)
   int stage_tile;   // 0: one-row stage kernel, 1: tiled stage kernel
+  bool tile_chosen, waves_chosen;  // by the caller (else the defaults)
   int prec;         // DGX_PREC_* (float trace records in the mixed forms)
   int affine;       // q = 1 and every element a parallelepiped
   double* mean;     // running mean (Gauss-nodal), allocated on first use
@@ -53,6 +56,26 @@ namespace dgx
 MeshArgs mesh_args(const dgx_ctx* c);
 // trace records of U, recomputed when U was set from outside
 hipError_t ensure_traces(dgx_ctx* c);
+// what a stage of the context's kernel reads besides U: the boundary states
+// (tiled kernel) or the trace records
+hipError_t ensure_stage_inputs(dgx_ctx* c);
+hipError_t ensure_boundary(dgx_ctx* c);
+// whether the context's stages read states instead of trace records
+inline bool reads_states(const dgx_ctx* c)
+{
+  return c->stage_tile == 1 && c->prec == DGX_PREC_FP64;
+}
+// the last stage of a step has written U and what the next stage reads
+inline void stage_outputs_valid(dgx_ctx* c)
+{
+  c->tb_valid = true;
+  c->tu_valid = !reads_states(c);  // such stages write no records
+}
+// U was set or changed from outside: nothing stored belongs to it
+inline void drop_traces(dgx_ctx* c)
+{
+  c->tu_valid = c->tb_valid = false;
+}
 // StageArgs of the stages of one step without a norm (returns the number of
 // stages: 4 for RK4, 3 for TVD-RK3); the last stage writes U and its traces
 int stage_plan(const dgx_ctx* c, int scheme, double dt, StageArgs sa[4]);

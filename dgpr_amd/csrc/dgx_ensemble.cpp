@@ -153,6 +153,7 @@ static dgx_status plan(dgx_ensemble* en, int scheme, const double* dt)
         it.mesh = mesh_args(c);
         it.ph = c->phys;
         it.sa = sa[s];
+        it.sa.records = !(g.unit_grid && g.tile == 1);
         it.lam = c->lam;
         it.block0 = block0;
         it.p = c->p;
@@ -224,13 +225,25 @@ static hipError_t enqueue_step(dgx_ensemble* en)
   return hipSuccess;
 }
 
-// Trace records of members whose state was set from outside; every member
-// stream is idle afterwards.
-static dgx_status prepare_members(dgx_ensemble* en)
+// Whether the active group of member i runs the tiled kernel (which reads and
+// writes boundary states, no trace records).
+static bool member_tiled(const dgx_ensemble* en, int i)
 {
-  for (dgx_ctx* c : en->ctx)
+  for (const EnsGroup& g : en->groups)
+    if (active(en, g) && std::find(g.members.begin(), g.members.end(), i) != g.members.end())
+      return g.unit_grid && g.tile == 1;
+  return false;
+}
+
+// What the next stage reads besides the state of members whose state was set
+// from outside (all: the trace records of every member); every member stream
+// is idle afterwards.
+static dgx_status prepare_members(dgx_ensemble* en, bool all)
+{
+  for (size_t i = 0; i < en->ctx.size(); ++i)
   {
-    EHIP(en, ensure_traces(c));
+    dgx_ctx* c = en->ctx[i];
+    EHIP(en, !all && member_tiled(en, (int)i) ? ensure_boundary(c) : ensure_traces(c));
     EHIP(en, hipStreamSynchronize(c->stream));
   }
   return DGX_OK;
@@ -367,10 +380,10 @@ dgx_status dgx_ensemble_step(dgx_ensemble* en, int scheme, const double* dt, uin
   dgx_status st = plan(en, scheme, dt);
   if (st != DGX_OK)
     return st;
-  if ((st = prepare_members(en)) != DGX_OK)
+  if ((st = prepare_members(en, false)) != DGX_OK)
     return st;
   for (dgx_ctx* c : en->ctx)
-    c->tu_valid = false;
+    drop_traces(c);
   if (use_graph && !en->graph_ready && nsteps > 0)
   {
     EHIP(en, hipStreamBeginCapture(en->stream, hipStreamCaptureModeThreadLocal));
@@ -402,8 +415,11 @@ dgx_status dgx_ensemble_step(dgx_ensemble* en, int scheme, const double* dt, uin
     else
       EHIP(en, enqueue_step(en));
   }
-  for (dgx_ctx* c : en->ctx)
-    c->tu_valid = true;
+  for (size_t i = 0; i < en->ctx.size(); ++i)
+  {
+    en->ctx[i]->tb_valid = true;
+    en->ctx[i]->tu_valid = !member_tiled(en, (int)i);
+  }
   return DGX_OK;
 }
 
@@ -441,7 +457,7 @@ dgx_status dgx_ensemble_autotune(dgx_ensemble* en, int scheme, const double* dt,
   dgx_status st = plan(en, scheme, dt);
   if (st != DGX_OK)
     return st;
-  if ((st = prepare_members(en)) != DGX_OK)
+  if ((st = prepare_members(en, true)) != DGX_OK)
     return st;
   drop_graph(en);
   hipEvent_t e0, e1;

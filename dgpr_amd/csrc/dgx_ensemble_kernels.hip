@@ -21,20 +21,20 @@
 namespace dgx
 {
 
-template <int P, int TILE>
+template <int P, int TILE, bool AFF>
 constexpr size_t ens_body_bytes()
 {
   if constexpr (TILE == 1)
-    return TileLds<P, 1, tile_rows(P)>::bytes;
+    return StateLds<P, 1, tile_rows(P), AFF>::bytes;
   else
     return StageLds<P, 1>::bytes;
 }
 
-template <int TILE>
+template <int TILE, bool AFF>
 constexpr size_t ens_lds_bytes()
 {
-  constexpr size_t a = ens_body_bytes<1, TILE>(), b = ens_body_bytes<2, TILE>(),
-                   c = ens_body_bytes<3, TILE>();
+  constexpr size_t a = ens_body_bytes<1, TILE, AFF>(), b = ens_body_bytes<2, TILE, AFF>(),
+                   c = ens_body_bytes<3, TILE, AFF>();
   return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
@@ -43,8 +43,7 @@ __device__ __forceinline__ void ens_body(const BatchItem& it, int unit, int* sta
                                          unsigned char* lds)
 {
   if constexpr (TILE == 1)
-    tile_body_lds<P, 1, tile_rows(P), double, AFF>(it.mesh, it.ph, it.sa, it.lam, status,
-                                                       unit, lds);
+    state_body<P, 1, tile_rows(P), AFF, false>(it.mesh, it.ph, it.sa, it.lam, status, unit, lds);
   else
     stage_body_lds<P, 1, double, AFF>(it.mesh, it.ph, it.sa, it.lam, status, unit, lds);
 }
@@ -55,7 +54,8 @@ template <int W, int TILE, bool AFF, int PS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
 void dgx_ens_stage_kernel(const BatchItem* __restrict__ items, int nitems, int* status)
 {
-  constexpr size_t LDS = PS ? ens_body_bytes<(PS ? PS : 1), TILE>() : ens_lds_bytes<TILE>();
+  constexpr size_t LDS = PS ? ens_body_bytes<(PS ? PS : 1), TILE, AFF>()
+                            : ens_lds_bytes<TILE, AFF>();
   __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
   const int u = blockIdx.x;
   int lo = 0, hi = nitems - 1;

@@ -6,8 +6,6 @@
 #include "dgx_dual.hpp"
 #include "dgx_dd.hpp"
 
-#include <type_traits>
-
 namespace dgx
 {
 
@@ -509,53 +507,10 @@ __global__ __launch_bounds__(256) void dgx_mean_kernel(const double* __restrict_
 
 // ---- launch helpers (host) -----------------------------------------------
 
-template <int P, int Q, typename TT, bool AFF, int CT>
-hipError_t launch_tile_ct(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
-                          const double* lam, int* status, int waves, hipStream_t st)
-{
-  constexpr int R = tile_rows(P);
-  constexpr int E = TileDims<P, R>::E;
-  int nblk = (m.nelem + E - 1) / E;
-  const bool norm = sa.normp != nullptr;
-  if (waves == 2 && norm)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT, true>), dim3(nblk),
-                       dim3(64), 0, st, m, ph, sa, lam, status);
-  else if (waves == 2)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
-                       st, m, ph, sa, lam, status);
-  else if (waves == 3 && norm)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT, true>), dim3(nblk),
-                       dim3(64), 0, st, m, ph, sa, lam, status);
-  else if (waves == 3)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
-                       st, m, ph, sa, lam, status);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-// the matrix-core contraction forms exist for p = 3 with FP32 trace records
-template <int P, int Q, typename TT, bool AFF>
-hipError_t launch_tile_t(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
-                         const double* lam, int* status, int waves, hipStream_t st)
-{
-  if constexpr (P == 3 && std::is_same<TT, float>::value)
-  {
-    if (sa.ctype == 1)
-      return launch_tile_ct<P, Q, TT, AFF, 1>(m, ph, sa, lam, status, waves, st);
-    if (sa.ctype == 2)
-      return launch_tile_ct<P, Q, TT, AFF, 2>(m, ph, sa, lam, status, waves, st);
-  }
-  return launch_tile_ct<P, Q, TT, AFF, 0>(m, ph, sa, lam, status, waves, st);
-}
-
 template <int P, int Q, typename TT, bool AFF>
 hipError_t launch_rhs_t(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
-                        int* status, int waves, int tile, hipStream_t st)
+                        int* status, int waves, hipStream_t st)
 {
-  if constexpr (Q == 1)
-    if (tile)
-      return launch_tile_t<P, Q, TT, AFF>(m, ph, sa, lam, status, waves, st);
   constexpr int EPW = Dims<P, Q>::EPW;
   int nblk = (m.nelem + EPW - 1) / EPW;
   if (waves == 1)
@@ -575,21 +530,21 @@ hipError_t launch_rhs_t(const MeshArgs& m, const Phys& ph, const StageArgs& sa, 
 // affine q = 1 meshes take the constant-Jacobian instantiation
 template <int P, int Q, typename TT>
 hipError_t launch_rhs_a(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
-                        int* status, int waves, int tile, hipStream_t st)
+                        int* status, int waves, hipStream_t st)
 {
   if constexpr (Q == 1)
     if (m.affine)
-      return launch_rhs_t<P, Q, TT, true>(m, ph, sa, lam, status, waves, tile, st);
-  return launch_rhs_t<P, Q, TT, false>(m, ph, sa, lam, status, waves, tile, st);
+      return launch_rhs_t<P, Q, TT, true>(m, ph, sa, lam, status, waves, st);
+  return launch_rhs_t<P, Q, TT, false>(m, ph, sa, lam, status, waves, st);
 }
 
 template <int P, int Q>
 hipError_t launch_rhs(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
-                      int* status, int waves, int tile, hipStream_t st)
+                      int* status, int waves, hipStream_t st)
 {
   if (sa.trace32)
-    return launch_rhs_a<P, Q, float>(m, ph, sa, lam, status, waves, tile, st);
-  return launch_rhs_a<P, Q, double>(m, ph, sa, lam, status, waves, tile, st);
+    return launch_rhs_a<P, Q, float>(m, ph, sa, lam, status, waves, st);
+  return launch_rhs_a<P, Q, double>(m, ph, sa, lam, status, waves, st);
 }
 
 template <int P, int Q, bool AFF>
@@ -726,7 +681,9 @@ hipError_t rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, const S
     return hipErrorInvalidValue;
   if (tile == 2)
     return gen_rhs_dispatch(p, q, m, ph, sa, lam, status, st);
-#define CALL_RHS(P, Q) launch_rhs<P, Q>(m, ph, sa, lam, status, waves, tile, st)
+  if (tile == 1)
+    return tile_rhs_dispatch(p, m, ph, sa, lam, status, waves, st);
+#define CALL_RHS(P, Q) launch_rhs<P, Q>(m, ph, sa, lam, status, waves, st)
   DGX_DISPATCH_PQ(p, q, CALL_RHS)
 #undef CALL_RHS
 }
@@ -805,6 +762,28 @@ hipError_t lift_face_dispatch(int p, const double* lam, int nelem, double* lamf,
   const size_t n = (size_t)nelem * 6;
   hipLaunchKernelGGL(dgx_lift_face_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, lam,
                      (p + 1) * (p + 1), n, lamf);
+  return hipGetLastError();
+}
+
+// arec[e][GREC]: the constant geometry of every element of an affine mesh
+// (affine_record), computed once per context.
+__global__ __launch_bounds__(64) void dgx_affine_record_kernel(const double* __restrict__ nodes,
+                                                              int nelem, double* __restrict__ arec)
+{
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  if (e < nelem)
+    affine_record(nodes, e, nelem, arec + (size_t)e * GREC);
+}
+
+size_t affine_record_doubles(int nelem)
+{
+  return (size_t)nelem * GREC;
+}
+
+hipError_t affine_record_dispatch(const double* nodes, int nelem, double* arec, hipStream_t st)
+{
+  hipLaunchKernelGGL(dgx_affine_record_kernel, dim3((unsigned)((nelem + 63) / 64)), dim3(64), 0, st,
+                     nodes, nelem, arec);
   return hipGetLastError();
 }
 

@@ -71,6 +71,9 @@ struct MeshArgs
   // constant over a parallelepiped's face (fJ / det J times a table sum);
   // null otherwise
   const double* lamf;
+  // affine meshes: each element's constant geometry [e][GREC] (affine_record
+  // in dgx_stage.hpp); null otherwise
+  const double* arec;
 };
 
 // Epilogue of one right-hand-side evaluation:
@@ -101,6 +104,10 @@ struct StageArgs
   // sum of R^2, R = -B3^T W f (the residual norm of this stage's f), for
   // tile_blocks(p, nelem) blocks
   double* normp = nullptr;
+  // FP64 tiled kernel only: 0 writes just the boundary states of Vout's
+  // domain-boundary faces to Tout (all that its next stage reads); the other
+  // kernels, and the adjoint, read the trace records of every face
+  int records = 1;
 };
 
 // One member of a batched stage launch: its mesh, physics, stage arguments
@@ -125,6 +132,18 @@ struct BatchItem
 hipError_t rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
                         const double* lam, int* status, int waves, hipStream_t st, int tile = 0);
 bool tile_valid(int p, int q, int tile, int waves);
+// the tiled kernel (tile 1) of q = 1 meshes (dgx_tile_kernels.hip): in FP64 it
+// reads both sides' states, and of Tin only the boundary states of Vin
+hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                             const double* lam, int* status, int waves, hipStream_t st);
+// boundary states of V (q = 1) into the boundary section of the record set
+// Tout; nothing to do on periodic meshes
+hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
+                             double* Tout, int* status, hipStream_t st);
+hipError_t upload_tables_tile(const PTab* pt, const QTab* qt);
+// affine meshes: arec (affine_record_doubles(nelem)) of every element
+size_t affine_record_doubles(int nelem);
+hipError_t affine_record_dispatch(const double* nodes, int nelem, double* arec, hipStream_t st);
 // one stage of several meshes of the same (p, q): items_dev (device memory,
 // sorted by block0) covers nblocks blocks in total; affine: every member is
 // an affine q = 1 mesh (MeshArgs::affine)

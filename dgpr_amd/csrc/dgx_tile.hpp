@@ -679,11 +679,3 @@ __device__ __forceinline__ void tile_body_lds(const MeshArgs& mesh, const Phys& 
     atomicOr(status, 1);
 }
 
-template <int P, int Q, int R, int W, typename TT, bool AFF, int CT = 0, bool NORM = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
-void dgx_tile_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
-                           int* status)
-{
-  __shared__ __attribute__((aligned(16))) unsigned char lds[TileLds<P, Q, R>::bytes];
-  tile_body_lds<P, Q, R, TT, AFF, CT, NORM>(mesh, ph, sa, lam, status, blockIdx.x, lds);
-}

@@ -1,0 +1,166 @@
+// dgx_tile_kernels.hip -- the tiled stage kernel of q = 1 meshes (dgx_tile.hpp)
+// and the boundary states it starts from, with their host launch helpers.
+#include "dgx_stage.hpp"
+
+#include <type_traits>
+
+namespace dgx
+{
+
+// Boundary states (bound_states.cpp:24-130) of every domain-boundary face
+// point of the Gauss-nodal state V, into the boundary section of a trace
+// record set: what a tiled stage reads besides V itself, after V was set from
+// outside.  One thread per boundary face point (sides in the order of
+// bface_index); the points of periodic sides are not read and not written.
+template <int P, bool AFF>
+__global__ __launch_bounds__(64) void dgx_boundary_kernel(MeshArgs mesh, Phys ph,
+                                                          const double* __restrict__ V,
+                                                          double* __restrict__ Tout, int* status)
+{
+  constexpr int N = P + 1, NF = N * N, NB = N * N * N;
+  const size_t t = (size_t)blockIdx.x * 64 + threadIdx.x;
+  if (t >= boundary_faces(mesh.nx, mesh.ny, mesh.nz) * NF)
+    return;
+  const int fpt = (int)(t % NF), bf = (int)(t / NF);
+  const int sx = mesh.ny * mesh.nz, sy = mesh.nx * mesh.nz, sz = mesh.nx * mesh.ny;
+  const int nd = bf < 2 * sx ? 0 : (bf < 2 * (sx + sy) ? 1 : 2);
+  const int in = bf - (nd == 0 ? 0 : (nd == 1 ? 2 * sx : 2 * (sx + sy)));
+  const int s  = nd == 0 ? sx : (nd == 1 ? sy : sz);
+  const int hi = in >= s, c = in - hi * s, f = 2 * nd + hi;
+  const int n1 = nd == 0 ? mesh.ny : mesh.nx;  // first tangential element count
+  const int i1 = c % n1, i2 = c / n1;
+  const int far = (nd == 0 ? mesh.nx : (nd == 1 ? mesh.ny : mesh.nz)) - 1;
+  const int i0 = hi ? far : 0;
+  const int ci = nd == 0 ? i0 : i1, cj = nd == 1 ? i0 : (nd == 0 ? i1 : i2), ck = nd == 2 ? i0 : i2;
+  int bt;
+  if (neighbour(mesh, ci, cj, ck, f, &bt) >= 0)
+    return;
+  const size_t e = ((size_t)ck * mesh.ny + cj) * mesh.nx + ci;
+  const PTab& pt = c_ptab[P - 1];
+  const int a = fpt % N, b = fpt / N;
+  double U[5];
+#pragma unroll
+  for (int r = 0; r < 5; ++r)
+  {
+    double v = 0.0;
+#pragma unroll
+    for (int m = 0; m < N; ++m)
+      v += pt.L[hi][m] * V[(e * 5 + r) * NB + line_node<N>(nd, m, a, b)];
+    U[r] = v;
+  }
+  double Ji[3][3], nv[3], Ub[5];
+  const int gi0 = (nd == 0) ? 0 : a;
+  const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
+  const int gi2 = (nd == 2) ? 0 : b;
+  face_geometry<1, AFF>(c_qtab[P - 1][0], mesh.nodes + e * 24, AFF ? mesh.arec + e * GREC : nullptr,
+                        nd, hi, gi0, gi1, gi2, Ji, nv);
+  if (!boundary_state(bt, U, nv, ph, Ub))
+    atomicOr(status, 1);
+  double* B = Tout + (size_t)mesh.nelem * 6 * 8 * NF + (size_t)bf * 5 * NF + fpt;
+#pragma unroll
+  for (int r = 0; r < 5; ++r)
+    B[r * NF] = Ub[r];
+}
+
+template <int P>
+static hipError_t launch_boundary(const MeshArgs& m, const Phys& ph, const double* V, double* Tout,
+                                  int* status, hipStream_t st)
+{
+  const size_t n = boundary_faces(m.nx, m.ny, m.nz) * (size_t)((P + 1) * (P + 1));
+  const dim3 grid((unsigned)((n + 63) / 64)), block(64);
+  if (m.affine)
+    hipLaunchKernelGGL((dgx_boundary_kernel<P, true>), grid, block, 0, st, m, ph, V, Tout, status);
+  else
+    hipLaunchKernelGGL((dgx_boundary_kernel<P, false>), grid, block, 0, st, m, ph, V, Tout, status);
+  return hipGetLastError();
+}
+
+hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
+                             double* Tout, int* status, hipStream_t st)
+{
+  bool walls = false;
+  for (int i = 0; i < 6; ++i)
+    walls = walls || m.bounds[i] != -2;
+  if (!walls)
+    return hipSuccess;
+  switch (p)
+  {
+    case 1: return launch_boundary<1>(m, ph, V, Tout, status, st);
+    case 2: return launch_boundary<2>(m, ph, V, Tout, status, st);
+    case 3: return launch_boundary<3>(m, ph, V, Tout, status, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <int P, int Q, typename TT, bool AFF, int CT>
+static hipError_t launch_tile_ct(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                          const double* lam, int* status, int waves, hipStream_t st)
+{
+  constexpr int R = tile_rows(P);
+  constexpr int E = TileDims<P, R>::E;
+  int nblk = (m.nelem + E - 1) / E;
+  const bool norm = sa.normp != nullptr;
+  if (waves == 2 && norm)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT, true>), dim3(nblk),
+                       dim3(64), 0, st, m, ph, sa, lam, status);
+  else if (waves == 2)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
+                       st, m, ph, sa, lam, status);
+  else if (waves == 3 && norm)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT, true>), dim3(nblk),
+                       dim3(64), 0, st, m, ph, sa, lam, status);
+  else if (waves == 3)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
+                       st, m, ph, sa, lam, status);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+// the matrix-core contraction forms exist for p = 3 with FP32 trace records
+template <int P, int Q, typename TT, bool AFF>
+static hipError_t launch_tile_t(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                         const double* lam, int* status, int waves, hipStream_t st)
+{
+  if constexpr (P == 3 && std::is_same<TT, float>::value)
+  {
+    if (sa.ctype == 1)
+      return launch_tile_ct<P, Q, TT, AFF, 1>(m, ph, sa, lam, status, waves, st);
+    if (sa.ctype == 2)
+      return launch_tile_ct<P, Q, TT, AFF, 2>(m, ph, sa, lam, status, waves, st);
+  }
+  return launch_tile_ct<P, Q, TT, AFF, 0>(m, ph, sa, lam, status, waves, st);
+}
+
+template <int P>
+static hipError_t launch_tile(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                              const double* lam, int* status, int waves, hipStream_t st)
+{
+  if (sa.trace32)
+    return m.affine ? launch_tile_t<P, 1, float, true>(m, ph, sa, lam, status, waves, st)
+                    : launch_tile_t<P, 1, float, false>(m, ph, sa, lam, status, waves, st);
+  return m.affine ? launch_tile_t<P, 1, double, true>(m, ph, sa, lam, status, waves, st)
+                  : launch_tile_t<P, 1, double, false>(m, ph, sa, lam, status, waves, st);
+}
+
+hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                             const double* lam, int* status, int waves, hipStream_t st)
+{
+  switch (p)
+  {
+    case 1: return launch_tile<1>(m, ph, sa, lam, status, waves, st);
+    case 2: return launch_tile<2>(m, ph, sa, lam, status, waves, st);
+    case 3: return launch_tile<3>(m, ph, sa, lam, status, waves, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t upload_tables_tile(const PTab* pt, const QTab* qt)
+{
+  hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_ptab), pt, sizeof(PTab) * 3);
+  if (e != hipSuccess)
+    return e;
+  return hipMemcpyToSymbol(HIP_SYMBOL(c_qtab), qt, sizeof(QTab) * 9);
+}
+
+}  // namespace dgx
