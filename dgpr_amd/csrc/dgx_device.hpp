@@ -29,6 +29,23 @@ __device__ __forceinline__ double rcp(double x)
   return __builtin_fma(r, e, r);
 }
 
+// 1/sqrt(x) for x > 0 well inside the normal range: the hardware estimate
+// refined by two Newton-Raphson steps y <- y + y (1 - x y^2) / 2, within about
+// one ulp.  sqrt(x) is x times it: 10 instructions and one transcendental for
+// both, where the IEEE square root and reciprocal take about 30 and two.
+__device__ __forceinline__ double rsq(double x)
+{
+#ifdef __HIP__
+  double y = __builtin_amdgcn_rsq(x);
+#else
+  double y = 1.0 / sqrt(x);
+#endif
+  double e = __builtin_fma(-(x * y), y, 1.0);
+  y = __builtin_fma(0.5 * y, e, y);
+  e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(0.5 * y, e, y);
+}
+
 // Euler flux F[d][r] of conserved state U.
 __device__ __forceinline__ void euler_flux(const double* U, double gamma,
                                            double F[3][5])
@@ -117,6 +134,65 @@ __device__ __forceinline__ void roe_flux(const T* Ul, const T* Ur, const double*
   f[3] = 0.5 * ((mnl * wl + pl * n[2]) + (mnr * wr + pr * n[2])) -
          0.5 * (al3 * dzm + C1 * w + C2 * n[2]);
   f[4] = 0.5 * ((mnl * Hl) + (mnr * Hr)) - 0.5 * (al3 * drE + C1 * H + C2 * un);
+}
+
+// roe_flux with fewer operations, for the FP64 kernels (the mixed forms and
+// the dual numbers keep the form above, whose last bits their stored FP32
+// records and tests follow).  ul, ur are the velocities and irl, irr the
+// reciprocal densities of the two states, which the caller needs too.  The Roe
+// weights come from one square root, wr = s / (1 + s) with s = sqrt(rr / rl); c and 1/c
+// from one reciprocal square root; 1/(2 eps) is 10/c.  Also returns the jumps
+// d = Ur - Ul.
+__device__ __forceinline__ void roe_flux_fp64(const double* Ul, const double* ul, double irl,
+                                              const double* Ur, const double* ur, double irr,
+                                              const double* n, double g, double* f, double* d)
+{
+  const double gm1 = g - 1.0;
+  const double pl = gm1 * (Ul[4] - 0.5 * (Ul[1] * ul[0] + Ul[2] * ul[1] + Ul[3] * ul[2]));
+  const double pr = gm1 * (Ur[4] - 0.5 * (Ur[1] * ur[0] + Ur[2] * ur[1] + Ur[3] * ur[2]));
+  const double Hl = (Ul[4] + pl) * irl, Hr = (Ur[4] + pr) * irr;
+  const double x = Ur[0] * irl, s = x * rsq(x);
+  const double wr = s * rcp(1.0 + s);
+  const double u[3] = {ul[0] + wr * (ur[0] - ul[0]), ul[1] + wr * (ur[1] - ul[1]),
+                       ul[2] + wr * (ur[2] - ul[2])};
+  const double H = Hl + wr * (Hr - Hl);
+#pragma unroll
+  for (int r = 0; r < 5; ++r)
+    d[r] = Ur[r] - Ul[r];
+  const double qsq = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+  const double c2  = gm1 * (H - 0.5 * qsq);
+  const double ic = rsq(c2), c = c2 * ic;
+  const double un = u[0] * n[0] + u[1] * n[1] + u[2] * n[2];
+  const double l1 = un + c, l2 = un - c;
+  const double eps = 0.05 * c, ee = eps * eps, i2e = 10.0 * ic;
+  double al1 = fabs(l1), al2 = fabs(l2), al3 = fabs(un);
+  al1 = (al1 < eps) ? (ee + l1 * l1) * i2e : al1;
+  al2 = (al2 < eps) ? (ee + l2 * l2) * i2e : al2;
+  al3 = (al3 < eps) ? (ee + un * un) * i2e : al3;
+  const double s2  = 0.5 * (al1 - al2);
+  const double s13 = 0.5 * (al1 + al2) - al3;
+  const double mnl = Ul[1] * n[0] + Ul[2] * n[1] + Ul[3] * n[2];
+  const double mnr = Ur[1] * n[0] + Ur[2] * n[1] + Ur[3] * n[2];
+  const double G1 = gm1 * ic * (0.5 * qsq * d[0] - (u[0] * d[1] + u[1] * d[2] + u[2] * d[3]) + d[4]);
+  const double G2 = (mnr - mnl) - un * d[0];
+  // halves of the mean flux's and the dissipation's factors
+  const double c1 = 0.5 * ic * (G1 * s13 + G2 * s2), c2h = 0.5 * (G1 * s2 + s13 * G2);
+  const double ml = 0.5 * mnl, mr = 0.5 * mnr, a3 = 0.5 * al3, pn = 0.5 * (pl + pr) - c2h;
+  f[0] = (ml + mr) - (a3 * d[0] + c1);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    f[1 + i] = (ml * ul[i] + mr * ur[i] + pn * n[i]) - (a3 * d[1 + i] + c1 * u[i]);
+  f[4] = (ml * Hl + mr * Hr) - (a3 * d[4] + c1 * H + c2h * un);
+}
+
+__device__ __forceinline__ void roe_flux_fp64(const double* Ul, const double* Ur, const double* n,
+                                              double g, double* f)
+{
+  const double irl = rcp(Ul[0]), irr = rcp(Ur[0]);
+  const double ul[3] = {Ul[1] * irl, Ul[2] * irl, Ul[3] * irl};
+  const double ur[3] = {Ur[1] * irr, Ur[2] * irr, Ur[3] * irr};
+  double d[5];
+  roe_flux_fp64(Ul, ul, irl, Ur, ur, irr, n, g, f, d);
 }
 
 // Reverse mode of roe_flux: gl = d(psi . f)/dUl and gr = d(psi . f)/dUr,

@@ -446,29 +446,13 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_stage_kernel(MeshArgs me
         for (int r = 0; r < 5; ++r)
           Ub[r] = B[r * NF];
       }
-      face_point_physics(en >= 0, UL, Ub, vgL, vgR, nv, lamL, lamR, ph, fpo);
-
-      // contravariant dual-consistency flux h_c = Ji[c] . dcQ (rows 1-4)
-      const double irL = rcp(UL[0]);
-      const double uL[3] = {UL[1] * irL, UL[2] * irL, UL[3] * irL};
       const double sc = fJ * t.w[a] * t.w[b];
-      const double* S = fpo.S;
-      const double Sm[3][3] = {{S[0], S[3], S[4]}, {S[3], S[1], S[5]}, {S[4], S[5], S[2]}};
       double hc[3][4];
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-      {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          hc[c][i] = sc * (JiL[c][0] * Sm[0][i] + JiL[c][1] * Sm[1][i] + JiL[c][2] * Sm[2][i]);
-        hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
-      }
+      face_point<sizeof(TT) == sizeof(double)>(en >= 0, UL, Ub, vgL, vgR, nv, JiL, lamL, lamR, sc,
+                                               ph, fpo.G, hc);
 #pragma unroll
       for (int r = 0; r < 5; ++r)
-      {
-        fpo.G[r] *= sc;
         sR[tid * FS + r] = fpo.G[r];
-      }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
       {

@@ -169,6 +169,118 @@ __device__ __forceinline__ void face_point_physics(bool interior, const T* UL, c
 }
 
 
+// One face point of the FP64 kernels: face_point_physics and what follows it,
+// with fewer operations (FP64 issue bounds the state-reading kernel: 64^3 p = 3
+// cube 1312 -> 1290 us per stage with a mean of 1.03x over the q = 1 cases; 1-2 %
+// on the record-reading kernels).  From both traces with their velocities u and
+// reciprocal densities ir, the gradient tractions, the own inverse Jacobian
+// Ji with its normal products mc[c] = Ji[c] . n, and the quadrature factor sc:
+//   G[r]     sc (F - QH.n)
+//   hc[c][r] sc Ji[c] . dcQ, the contravariant dual-consistency flux, whose
+//            stress tau(a (x) n) gives  mu ((Ji[c].a) n + mc a - 2/3 (a.n) Ji[c])
+//            with a = s dmL, without forming the stress.
+__device__ __forceinline__ void face_point_fp64(bool interior, const double* UL, const double* uL,
+                                                double irL, const double* Ub, const double* uB,
+                                                double irB, const double* vgL, const double* vgR,
+                                                const double* n, const double Ji[3][3],
+                                                const double* mc, double lamL, double lamR,
+                                                double sc, const Phys& ph, double* G,
+                                                double hc[3][4])
+{
+  const double mu = ph.mu;
+  double d[5];  // Ub - UL
+  if (interior)
+    roe_flux_fp64(UL, uL, irL, Ub, uB, irB, n, ph.gamma, G, d);
+  else
+  {
+    euler_flux_n(Ub, ph.gamma, n, G);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      d[r] = Ub[r] - UL[r];
+  }
+  // velocity jumps at the two states, UL - Ub: dm = -(d_m - d_rho u) / rho
+  double dmL[3], dmB[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+  {
+    dmL[i] = (d[0] * uL[i] - d[1 + i]) * irL;
+    dmB[i] = (d[0] * uB[i] - d[1 + i]) * irB;
+  }
+  const double dnL = dmL[0] * n[0] + dmL[1] * n[1] + dmL[2] * n[2];
+  const double dnB = dmB[0] * n[0] + dmB[1] * n[1] + dmB[2] * n[2];
+  // h tau(grad u).n - c tau(dm (x) n).n of both sides (see face_point_physics)
+  const double em = ph.eta * mu;
+  const double hL = interior ? 0.5 : 1.0, cL = interior ? 0.25 * em * lamL : 0.0;
+  const double hB = interior ? 0.5 : 0.0, cB = interior ? 0.25 * em * lamR : em * lamL;
+  const double tL = cL * (1.0 / 3.0) * dnL, tB = cB * (1.0 / 3.0) * dnB;
+  double qE = 0.0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+  {
+    const double wL = hL * vgL[i] - cL * dmL[i] - tL * n[i];
+    const double wB = hB * vgR[i] - cB * dmB[i] - tB * n[i];
+    G[1 + i] = sc * (G[1 + i] - (wL + wB));
+    qE += uL[i] * wL + uB[i] * wB;
+  }
+  G[0] *= sc;
+  G[4] = sc * (G[4] - qE);
+  // dual-consistency flux
+  const double al = (interior ? 0.5 : 1.0) * mu * sc;
+  const double a[3] = {al * dmL[0], al * dmL[1], al * dmL[2]};
+  const double t = (2.0 / 3.0) * al * dnL;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+  {
+    const double k = Ji[c][0] * a[0] + Ji[c][1] * a[1] + Ji[c][2] * a[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      hc[c][i] = k * n[i] + mc[c] * a[i] - t * Ji[c][i];
+    hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
+  }
+}
+
+// One face point of the record-reading kernels: G scaled by sc and the
+// contravariant dual-consistency flux hc, by face_point_fp64 (FAST) or, in the
+// mixed forms, by face_point_physics.
+template <bool FAST>
+__device__ __forceinline__ void face_point(bool interior, const double* UL, const double* Ub,
+                                           const double* vgL, const double* vgR, const double* n,
+                                           const double Ji[3][3], double lamL, double lamR,
+                                           double sc, const Phys& ph, double* G, double hc[3][4])
+{
+  const double irL  = rcp(UL[0]);
+  const double uL[3] = {UL[1] * irL, UL[2] * irL, UL[3] * irL};
+  if constexpr (FAST)
+  {
+    const double irB   = rcp(Ub[0]);
+    const double uB[3] = {Ub[1] * irB, Ub[2] * irB, Ub[3] * irB};
+    const double mc[3] = {Ji[0][0] * n[0] + Ji[0][1] * n[1] + Ji[0][2] * n[2],
+                          Ji[1][0] * n[0] + Ji[1][1] * n[1] + Ji[1][2] * n[2],
+                          Ji[2][0] * n[0] + Ji[2][1] * n[1] + Ji[2][2] * n[2]};
+    face_point_fp64(interior, UL, uL, irL, Ub, uB, irB, vgL, vgR, n, Ji, mc, lamL, lamR, sc, ph, G,
+                    hc);
+  }
+  else
+  {
+    FacePoint fpo;
+    face_point_physics(interior, UL, Ub, vgL, vgR, n, lamL, lamR, ph, fpo);
+    // contravariant dual-consistency flux h_c = Ji[c] . dcQ (rows 1-4)
+    const double* S       = fpo.S;
+    const double Sm[3][3] = {{S[0], S[3], S[4]}, {S[3], S[1], S[5]}, {S[4], S[5], S[2]}};
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        hc[c][i] = sc * (Ji[c][0] * Sm[0][i] + Ji[c][1] * Sm[1][i] + Ji[c][2] * Sm[2][i]);
+      hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
+    }
+#pragma unroll
+    for (int r = 0; r < 5; ++r)
+      G[r] = fpo.G[r] * sc;
+  }
+}
+
 // Volume flux H = Q - F (flux.cpp:24-48 Euler, flux.cpp:156-202 Newtonian
 // viscous, no heat flux) at a Gauss node, in velocity-gradient form, from the
 // node state Vq and the reference-space derivatives gr[c][0..3] of (rho, m).

@@ -584,6 +584,9 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
   using SL = StageLds<P, Q>;
   constexpr int N = FD::N, NB = FD::NB, NF = FD::NF, EPW = FD::EPW, FS = FD::FS;
   constexpr int NG = (Q + 1) * (Q + 1) * (Q + 1);
+  // the short form of the face physics; at q > 1, where the kernel spills, it
+  // measured 1-5 % slower
+  constexpr bool FAST = Q == 1 && sizeof(TT) == sizeof(double);
 
   auto sV  = reinterpret_cast<double(*)[5][NB]>(lds + SL::oV);
   auto sX  = reinterpret_cast<double(*)[NG * 3]>(lds + SL::oX);      // own geometry nodes
@@ -735,7 +738,9 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       const int gi2 = (nd == 2) ? 0 : b;
       double JiL[3][3], nv[3];
       const double fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
-      if (en >= 0)
+      if (en >= 0 && FAST)
+        roe_flux_fp64(UL, Ub, nv, ph.gamma, fpo.G);
+      else if (en >= 0)
         roe_flux(UL, Ub, nv, ph.gamma, fpo.G);
       else
         euler_flux_n(Ub, ph.gamma, nv, fpo.G);
@@ -795,23 +800,9 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
         for (int r = 0; r < 5; ++r)
           Ub[r] = B[r * NF];
       }
-      face_point_physics(en >= 0, UL, Ub, vgL, vgR, nv, lamL, lamR, ph, fpo);
-
-      // contravariant dual-consistency flux h_c = Ji[c] . dcQ (rows 1-4)
-      const double irL = rcp(UL[0]);
-      const double uL[3] = {UL[1] * irL, UL[2] * irL, UL[3] * irL};
       const double sc = fJ * pt.w[a] * pt.w[b];
-      const double* S = fpo.S;
-      const double Sm[3][3] = {{S[0], S[3], S[4]}, {S[3], S[1], S[5]}, {S[4], S[5], S[2]}};
       double hc[3][4];
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-      {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          hc[c][i] = sc * (JiL[c][0] * Sm[0][i] + JiL[c][1] * Sm[1][i] + JiL[c][2] * Sm[2][i]);
-        hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
-      }
+      face_point<FAST>(en >= 0, UL, Ub, vgL, vgR, nv, JiL, lamL, lamR, sc, ph, fpo.G, hc);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
       {
@@ -821,10 +812,7 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       }
 #pragma unroll
       for (int r = 0; r < 5; ++r)
-      {
-        fpo.G[r] *= sc;
         sR[tid * FS + r] = fpo.G[r];
-      }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
       {

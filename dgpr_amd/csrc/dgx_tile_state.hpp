@@ -150,21 +150,21 @@ __device__ __forceinline__ void line_traces(const double (&x)[5][N], const doubl
 }
 
 // Gradient traction tau(grad u).n of one side of face point (a, b): its trace
-// U, normal derivative dn and inverse Jacobian Ji, with the traces of the
-// face's other points in s ([4][64], this face's points from fbase), or at
-// p = 3 (lane = a + 4 face + 16 b) on the matrix cores.  The sums
-// of grad_traction, one reference direction after the other, so that four
-// derivatives are live at a time instead of twelve.
+// U with velocity u and reciprocal density ir, normal derivative dn, inverse
+// Jacobian Ji with mc[c] = Ji[c] . n, and the traces of the face's other points
+// in s ([4][64], this face's points from fbase), or at p = 3 (lane = a + 4
+// face + 16 b) on the matrix cores.  The sums of grad_traction, scaled by mu/rho
+// once, one reference direction after the other, so that four derivatives
+// are live at a time instead of twelve.
 template <int P, int D>
 __device__ __forceinline__ void face_traction(const PTab& pt, const MfTabs& mf, const double* s,
                                               int fbase, int a, int b, const double* U,
-                                              const double* dn, const double Ji[3][3],
-                                              const double* n, double mu, double* vg)
+                                              const double* u, double ir, const double* dn,
+                                              const double Ji[3][3], const double* n,
+                                              const double* mc, double mu, double* vg)
 {
   constexpr int N = P + 1;
-  const double ir = rcp(U[0]);
-  const double u[3] = {U[1] * ir, U[2] * ir, U[3] * ir};
-  double Ln[3] = {0.0, 0.0, 0.0}, LTn[3] = {0.0, 0.0, 0.0}, tr = 0.0;
+  double A[3] = {0.0, 0.0, 0.0}, tr = 0.0;
 #pragma unroll
   for (int c = 0; c < 3; ++c)
   {
@@ -189,21 +189,21 @@ __device__ __forceinline__ void face_traction(const PTab& pt, const MfTabs& mf, 
                                 : pt.Dg[b][m] * s[r * 64 + fbase + a + N * m];
       g[r] = d;
     }
-    const double dv0 = (g[1] - g[0] * u[0]) * ir;
-    const double dv1 = (g[2] - g[0] * u[1]) * ir;
-    const double dv2 = (g[3] - g[0] * u[2]) * ir;
-    const double mc = Ji[c][0] * n[0] + Ji[c][1] * n[1] + Ji[c][2] * n[2];
-    const double kc = dv0 * n[0] + dv1 * n[1] + dv2 * n[2];
-    Ln[0] += dv0 * mc;
-    Ln[1] += dv1 * mc;
-    Ln[2] += dv2 * mc;
-    LTn[0] += Ji[c][0] * kc;
-    LTn[1] += Ji[c][1] * kc;
-    LTn[2] += Ji[c][2] * kc;
-    tr += dv0 * Ji[c][0] + dv1 * Ji[c][1] + dv2 * Ji[c][2];
-    order_after(Ln, fbase);
+    // rho d u / d xi_c
+    const double dv[3] = {g[1] - g[0] * u[0], g[2] - g[0] * u[1], g[3] - g[0] * u[2]};
+    const double kc = dv[0] * n[0] + dv[1] * n[1] + dv[2] * n[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+      A[i] += dv[i] * mc[c] + Ji[c][i] * kc;
+      tr += dv[i] * Ji[c][i];
+    }
+    order_after(A, fbase);
   }
-  tau_n(mu, Ln, LTn, tr, n, vg);
+  const double k = mu * ir, t = (2.0 / 3.0) * tr;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    vg[i] = k * (A[i] - t * n[i]);
 }
 
 // Geometry a tile keeps per element face about the element across it: on
@@ -342,7 +342,16 @@ __device__ __forceinline__ void state_face_subpass(
       geometry_at<Q, false>(qt, sX[l], sG[l], D, hi, gi[0], gi[1], gi[2], J, JiL, det);
       fJ = face_normal(J, D, hi, nv);
     }
-    face_traction<P, D>(pt, mf, sR, fbase, a, b, UL, dL, JiL, nv, ph.mu, vgL);
+    double uL[3], uR[3], mcL[3];
+    const double irL = rcp(UL[0]), irR = rcp(Ub[0]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+      uL[i]  = UL[1 + i] * irL;
+      uR[i]  = Ub[1 + i] * irR;
+      mcL[i] = JiL[i][0] * nv[0] + JiL[i][1] * nv[1] + JiL[i][2] * nv[2];
+    }
+    face_traction<P, D>(pt, mf, sR, fbase, a, b, UL, uL, irL, dL, JiL, nv, mcL, ph.mu, vgL);
     int fbR = fbase;
     order_after(vgL, fbR);
     {
@@ -371,10 +380,16 @@ __device__ __forceinline__ void state_face_subpass(
         }
         inv3(J, det3(J), JiR);
       }
-      face_traction<P, D>(pt, mf, sR + 4 * 64, fbR, a, b, Ub, dR, JiR, nv, ph.mu, vgR);
+      double mcR[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        mcR[i] = JiR[i][0] * nv[0] + JiR[i][1] * nv[1] + JiR[i][2] * nv[2];
+      face_traction<P, D>(pt, mf, sR + 4 * 64, fbR, a, b, Ub, uR, irR, dR, JiR, nv, mcR, ph.mu,
+                          vgR);
     }
     order_after(vgR, UL[0], Ub[0]);
     next();
+    double irB = irR;
     if (en < 0)
     {
       // boundary state written with Vin
@@ -382,30 +397,17 @@ __device__ __forceinline__ void state_face_subpass(
 #pragma unroll
       for (int r = 0; r < 5; ++r)
         Ub[r] = B[r * NF];
+      irB = rcp(Ub[0]);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
+      {
+        uR[i]  = Ub[1 + i] * irB;
         vgR[i] = 0.0;
+      }
     }
-    FacePoint fpo;
-    face_point_physics(en >= 0, UL, Ub, vgL, vgR, nv, lamL, lamR, ph, fpo);
-
-    // contravariant dual-consistency flux h_c = Ji[c] . dcQ (rows 1-4)
-    const double irL  = rcp(UL[0]);
-    const double uL[3] = {UL[1] * irL, UL[2] * irL, UL[3] * irL};
-    const double sc   = fJ * pt.w[a] * pt.w[b];
-    const double* st  = fpo.S;
-    const double Sm[3][3] = {{st[0], st[3], st[4]}, {st[3], st[1], st[5]}, {st[4], st[5], st[2]}};
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-    {
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        hc[c][i] = sc * (JiL[c][0] * Sm[0][i] + JiL[c][1] * Sm[1][i] + JiL[c][2] * Sm[2][i]);
-      hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
-    }
-#pragma unroll
-    for (int r = 0; r < 5; ++r)
-      G[r] = fpo.G[r] * sc;
+    const double sc = fJ * pt.w[a] * pt.w[b];
+    face_point_fp64(en >= 0, UL, uL, irL, Ub, uR, irB, vgL, vgR, nv, JiL, mcL, lamL, lamR, sc, ph,
+                    G, hc);
   }
   // T = G - Dg^T(t1) h_t1 - Dg^T(t2) h_t2 (the mass row has no viscous part)
 #pragma unroll
