@@ -52,14 +52,7 @@ void dgx_adj_main_kernel(MeshArgs mesh, Phys ph, const double* __restrict__ V,
   const bool vact = (le < EPW) && (e < mesh.nelem);
   if constexpr (PART == 1)
     face_table<EPW>(mesh, e0, sNb, sBt);
-  for (int x = tid; x < EPW * NG * 3; x += 64)
-  {
-    int ee = e0 + x / (NG * 3);
-    sX[x / (NG * 3)][x % (NG * 3)] =
-        (ee < mesh.nelem) ? mesh.nodes[(size_t)ee * NG * 3 + x % (NG * 3)] : 0.0;
-  }
-  if (AFF && tid < EPW)
-    affine_record(mesh.nodes, e0 + tid, mesh.nelem, sG[tid]);
+  load_geometry<Q, EPW, AFF>(mesh, e0, sX, sG);
   const int idx[3] = {nd0 % N, (nd0 / N) % N, nd0 / (N * N)};
   double Ji[3][3], wJ = 1.0;
   if (PART == 0 && vact)
@@ -519,14 +512,7 @@ __global__ __launch_bounds__(64) void dgx_adj_trace_kernel(MeshArgs mesh, Phys p
   const int tid = threadIdx.x, le = tid / NB, nd0 = tid % NB;
   const int e0 = blockIdx.x * EPW, e = e0 + le;
   const bool vact = (le < EPW) && (e < mesh.nelem);
-  for (int x = tid; x < EPW * NG * 3; x += 64)
-  {
-    int ee = e0 + x / (NG * 3);
-    sX[x / (NG * 3)][x % (NG * 3)] =
-        (ee < mesh.nelem) ? mesh.nodes[(size_t)ee * NG * 3 + x % (NG * 3)] : 0.0;
-  }
-  if (AFF && tid < EPW)
-    affine_record(mesh.nodes, e0 + tid, mesh.nelem, sG[tid]);
+  load_geometry<Q, EPW, AFF>(mesh, e0, sX, sG);
   double pv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (vact)
   {

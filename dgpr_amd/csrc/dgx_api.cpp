@@ -104,6 +104,8 @@ MeshArgs dgx::mesh_args(const dgx_ctx* c)
   m.affine = c->affine;
   m.lamf   = c->lamf;
   m.arec   = c->arec;
+  m.geov   = c->geo;
+  m.geof   = c->geo ? c->geo + (size_t)c->nelem * GEOV * c->nbf : nullptr;
   return m;
 }
 
@@ -326,6 +328,32 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
     if ((e = affine_record_dispatch(c->nodes, c->nelem, c->arec, c->stream)) != hipSuccess)
       return bail("affine records", e);
   }
+  // curved geometry of the q > 1 and general orders is stored once (80 bytes
+  // per Gauss node and 104 per face point) where it takes at most a quarter of
+  // the free memory, so that no mesh that fitted without it is refused;
+  // otherwise every stage evaluates it from the nodes
+  if (!c->affine && (c->q > 1 || general_order(c->p, c->q)))
+  {
+    const size_t nf = (size_t)(c->p + 1) * (c->p + 1);
+    const size_t gb = (size_t)c->nelem * (GEOV * c->nbf + 6 * GEOF * nf) * sizeof(double);
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && gb <= fr / 4)
+    {
+      if (hipMalloc(&c->geo, gb) != hipSuccess)
+      {
+        (void)hipGetLastError();
+        c->geo = nullptr;
+      }
+      else
+      {
+        const MeshArgs ma = mesh_args(c);
+        if ((e = geometry_dispatch(c->p, c->q, ma, c->geo, const_cast<double*>(ma.geof),
+                                   c->stream)) != hipSuccess)
+          return bail("stored geometry", e);
+        c->bytes += gb;
+      }
+    }
+  }
   if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);
   if ((e = hipStreamSynchronize(c->stream)) != hipSuccess)
@@ -340,8 +368,8 @@ dgx_status dgx_destroy(dgx_ctx* c)
     return DGX_OK;
   if (c->stream)
     (void)hipStreamSynchronize(c->stream);
-  double* bufs[15] = {c->U,   c->Ua,  c->Ub,   c->acc, c->fs,  c->nodes, c->partial, c->sum,
-                      c->lam, c->lamf, c->arec, c->TU, c->TUa, c->TUb,   c->mean};
+  double* bufs[16] = {c->U,   c->Ua,   c->Ub,   c->acc, c->fs, c->nodes, c->partial, c->sum,
+                      c->lam, c->lamf, c->arec, c->geo, c->TU, c->TUa,   c->TUb,     c->mean};
   for (double* b : bufs)
     if (b)
       (void)hipFree(b);

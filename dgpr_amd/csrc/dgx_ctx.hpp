@@ -30,6 +30,7 @@ struct dgx_ctx
   double* lam;      // BR2 lifting coefficients [e][6][(p+1)^2]
   double* lamf;     // affine meshes: one coefficient per element face [e][6]
   double* arec;     // affine meshes: each element's constant geometry
+  double* geo;      // stored geometry (geov, then geof), or null
   double* TU;       // face trace records of U, Ua, Ub [e][6][8][(p+1)^2]
   double* TUa;
   double* TUb;

@@ -27,7 +27,7 @@ constexpr size_t ens_body_bytes()
   if constexpr (TILE == 1)
     return StateLds<P, 1, tile_rows(P), AFF>::bytes;
   else
-    return StageLds<P, 1>::bytes;
+    return StageLds<P, 1, AFF>::bytes;
 }
 
 template <int TILE, bool AFF>

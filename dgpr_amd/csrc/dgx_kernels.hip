@@ -12,12 +12,12 @@ namespace dgx
 // W is the occupancy target (waves per SIMD) handed to the register
 // allocator; the launch picks one of the compiled targets per (P, Q).  TT is
 // the type of the trace records read and written (float: mixed precision).
-template <int P, int Q, int W, typename TT, bool AFF>
+template <int P, int Q, int W, typename TT, bool AFF, bool STO>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
 void dgx_rhs_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
                           int* status)
 {
-  stage_body<P, Q, TT, AFF>(mesh, ph, sa, lam, status, blockIdx.x);
+  stage_body<P, Q, TT, AFF, STO>(mesh, ph, sa, lam, status, blockIdx.x);
 }
 
 // The inviscid right-hand side of the one-row body (INV): f(V; mu = 0) from
@@ -27,7 +27,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 void dgx_inviscid_rhs_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
                              int* status)
 {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[StageLds<P, Q>::bytes];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[StageLds<P, Q, AFF>::bytes];
   stage_body_lds<P, Q, double, AFF, true>(mesh, ph, sa, lam, status, blockIdx.x, lds);
 }
 
@@ -96,6 +96,52 @@ __global__ __launch_bounds__(64) void dgx_lift_coef_kernel(MeshArgs mesh, double
     s += pt.L[hi][m] * pt.L[hi][m] / (pt.w[m] * det3(Jm));
   }
   lam[t] = fJ * s;
+}
+
+// Stored geometry of a q > 1 mesh (geov, geof of MeshArgs): one thread per
+// Gauss node, then one per face point; the values that geometry_at and
+// face_geometry give in the kernels.
+template <int P, int Q>
+__global__ __launch_bounds__(64) void dgx_geometry_kernel(MeshArgs mesh, double* __restrict__ geov,
+                                                          double* __restrict__ geof)
+{
+  constexpr int N = P + 1, NB = N * N * N, NF = N * N, NG = (Q + 1) * (Q + 1) * (Q + 1);
+  const PTab& pt = c_ptab[P - 1];
+  const QTab& qt = c_qtab[P - 1][Q - 1];
+  const size_t t = (size_t)blockIdx.x * 64 + threadIdx.x, nv = (size_t)mesh.nelem * NB;
+  double Ji[3][3];
+  if (t < nv)
+  {
+    const size_t e = t / NB;
+    const int nd = (int)(t % NB), i = nd % N, j = (nd / N) % N, k = nd / (N * N);
+    double J[3][3], det;
+    geometry_at<Q, false>(qt, mesh.nodes + e * NG * 3, nullptr, -1, 0, i, j, k, J, Ji, det);
+    double* g = geov + e * GEOV * NB + nd;
+#pragma unroll
+    for (int x = 0; x < 9; ++x)
+      g[x * NB] = Ji[x / 3][x % 3];
+    g[9 * NB] = pt.w[i] * pt.w[j] * pt.w[k] * det;
+  }
+  else if (t < nv + (size_t)mesh.nelem * 6 * NF)
+  {
+    const size_t u = t - nv, e = u / (6 * NF);
+    const int fpt = (int)(u % NF), f = (int)((u / NF) % 6), nd = f >> 1, hi = f & 1;
+    const int a = fpt % N, b = fpt / N;
+    const int gi0 = (nd == 0) ? 0 : a;
+    const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
+    const int gi2 = (nd == 2) ? 0 : b;
+    double n[3];
+    const double fJ = face_geometry<Q, false>(qt, mesh.nodes + e * NG * 3, nullptr, nd, hi, gi0,
+                                              gi1, gi2, Ji, n);
+    double* g = geof + (e * 6 + f) * GEOF * NF + fpt;
+#pragma unroll
+    for (int x = 0; x < 9; ++x)
+      g[x * NF] = Ji[x / 3][x % 3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+      g[(9 + x) * NF] = n[x];
+    g[12 * NF] = fJ;
+  }
 }
 
 // ---- basis conversions and residual output ------------------------------
@@ -507,35 +553,39 @@ __global__ __launch_bounds__(256) void dgx_mean_kernel(const double* __restrict_
 
 // ---- launch helpers (host) -----------------------------------------------
 
-template <int P, int Q, typename TT, bool AFF>
+template <int P, int Q, typename TT, bool AFF, bool STO>
 hipError_t launch_rhs_t(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
                         int* status, int waves, hipStream_t st)
 {
   constexpr int EPW = Dims<P, Q>::EPW;
   int nblk = (m.nelem + EPW - 1) / EPW;
   if (waves == 1)
-    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 1, TT, AFF>), dim3(nblk), dim3(64), 0, st, m,
+    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 1, TT, AFF, STO>), dim3(nblk), dim3(64), 0, st, m,
                        ph, sa, lam, status);
   else if (waves == 2)
-    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 2, TT, AFF>), dim3(nblk), dim3(64), 0, st, m,
+    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 2, TT, AFF, STO>), dim3(nblk), dim3(64), 0, st, m,
                        ph, sa, lam, status);
   else if (waves == 3)
-    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 3, TT, AFF>), dim3(nblk), dim3(64), 0, st, m,
+    hipLaunchKernelGGL((dgx_rhs_stage_kernel<P, Q, 3, TT, AFF, STO>), dim3(nblk), dim3(64), 0, st, m,
                        ph, sa, lam, status);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-// affine q = 1 meshes take the constant-Jacobian instantiation
+// affine q = 1 meshes take the constant-Jacobian instantiation, q > 1 meshes
+// the one that reads the stored geometry where the context holds it
 template <int P, int Q, typename TT>
 hipError_t launch_rhs_a(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
                         int* status, int waves, hipStream_t st)
 {
   if constexpr (Q == 1)
     if (m.affine)
-      return launch_rhs_t<P, Q, TT, true>(m, ph, sa, lam, status, waves, st);
-  return launch_rhs_t<P, Q, TT, false>(m, ph, sa, lam, status, waves, st);
+      return launch_rhs_t<P, Q, TT, true, false>(m, ph, sa, lam, status, waves, st);
+  if constexpr (Q > 1)
+    if (m.geov)
+      return launch_rhs_t<P, Q, TT, false, true>(m, ph, sa, lam, status, waves, st);
+  return launch_rhs_t<P, Q, TT, false, false>(m, ph, sa, lam, status, waves, st);
 }
 
 template <int P, int Q>
@@ -773,6 +823,30 @@ __global__ __launch_bounds__(64) void dgx_affine_record_kernel(const double* __r
   const int e = blockIdx.x * 64 + threadIdx.x;
   if (e < nelem)
     affine_record(nodes, e, nelem, arec + (size_t)e * GREC);
+}
+
+template <int P, int Q>
+static hipError_t launch_geometry(const MeshArgs& m, double* geov, double* geof, hipStream_t st)
+{
+  if constexpr (Q > 1)
+  {
+    constexpr int N = P + 1;
+    const size_t n = (size_t)m.nelem * (N * N * N + 6 * N * N);
+    hipLaunchKernelGGL((dgx_geometry_kernel<P, Q>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st,
+                       m, geov, geof);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t geometry_dispatch(int p, int q, const MeshArgs& m, double* geov, double* geof,
+                             hipStream_t st)
+{
+  if (general_order(p, q))
+    return gen_geometry_dispatch(p, q, m, geov, geof, st);
+#define CALL_GEO(P, Q) launch_geometry<P, Q>(m, geov, geof, st)
+  DGX_DISPATCH_PQ(p, q, CALL_GEO)
+#undef CALL_GEO
 }
 
 size_t affine_record_doubles(int nelem)

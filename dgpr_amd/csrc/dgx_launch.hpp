@@ -74,7 +74,14 @@ struct MeshArgs
   // affine meshes: each element's constant geometry [e][GREC] (affine_record
   // in dgx_stage.hpp); null otherwise
   const double* arec;
+  // stored geometry (null where it is evaluated in the kernels): J^-1 and
+  // w detJ at every Gauss node [e][GEOV][(p+1)^3], and J^-1, the outward unit
+  // normal and the surface element at every face point
+  // [e][6][GEOF][(p+1)^2]
+  const double* geov;
+  const double* geof;
 };
+constexpr int GEOV = 10, GEOF = 13;
 
 // Epilogue of one right-hand-side evaluation:
 //   Vout = ca*Vbase + cb*Vin + cf*fterm
@@ -143,6 +150,11 @@ hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const dou
 hipError_t upload_tables_tile(const PTab* pt, const QTab* qt);
 // affine meshes: arec (affine_record_doubles(nelem)) of every element
 size_t affine_record_doubles(int nelem);
+// geov and geof of the mesh (q > 1, or an order of the general kernels)
+hipError_t geometry_dispatch(int p, int q, const MeshArgs& m, double* geov, double* geof,
+                             hipStream_t st);
+hipError_t gen_geometry_dispatch(int p, int q, const MeshArgs& m, double* geov, double* geof,
+                                 hipStream_t st);
 hipError_t affine_record_dispatch(const double* nodes, int nelem, double* arec, hipStream_t st);
 // one stage of several meshes of the same (p, q): items_dev (device memory,
 // sorted by block0) covers nblocks blocks in total; affine: every member is

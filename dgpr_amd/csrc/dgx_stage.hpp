@@ -197,8 +197,7 @@ __device__ __forceinline__ double face_normal(const double J[3][3], int nd, int 
 // reference direction d the outward unit normal of the element's high face
 // normal to d and its surface element, g[19 + 4d .. 22 + 4d]; the low face
 // has the opposite normal) instead of evaluating the geometry basis at every
-// node and face point.  Lanes 0..EPW-1 fill one record each; a barrier must
-// follow before use.
+// node and face point.
 constexpr int GREC = 31;
 __device__ __forceinline__ void affine_record(const double* __restrict__ nodes, int e, int nelem,
                                               double* g)
@@ -282,6 +281,56 @@ __device__ __forceinline__ double face_geometry(const QTab& qt, const double* X,
   double J[3][3], det;
   geometry_at<Q, false>(qt, X, g, nd, hi, i, j, k, J, Ji, det);
   return face_normal(J, nd, hi, nv);
+}
+
+// Geometry of the EPW elements from e0 in LDS: on affine meshes each element's
+// record (sG, written once per context by affine_record), else its nodes (sX).
+// A barrier must follow before use.
+template <int Q, int EPW, bool AFF>
+__device__ __forceinline__ void load_geometry(const MeshArgs& mesh, int e0,
+                                              double (*sX)[(Q + 1) * (Q + 1) * (Q + 1) * 3],
+                                              double (*sG)[GREC])
+{
+  constexpr int NX  = AFF ? GREC : (Q + 1) * (Q + 1) * (Q + 1) * 3;
+  const double* src = (AFF ? mesh.arec : mesh.nodes) + (size_t)e0 * NX;
+  double* dst       = AFF ? &sG[0][0] : &sX[0][0];
+  const int left    = min(mesh.nelem - e0, EPW) * NX;
+  for (int x = threadIdx.x; x < EPW * NX; x += 64)
+    dst[x] = (x < left) ? src[x] : 0.0;
+}
+
+// Stored geometry of q > 1 meshes (MeshArgs::geov, geof, written once per
+// context by dgx_geometry_kernel): J^-1 and w detJ at Gauss node nd of element
+// e, and J^-1, the outward unit normal and the surface element at point fpt of
+// its face f.  Evaluating the geometry basis in the stage takes 400 (q = 2) to
+// 1000 (q = 3) FP64 operations a point, at five points a lane, and 80-400
+// spilled registers; the stored values are 80 bytes a node and 104 a face
+// point and leave 164 registers.  Per TVD-RK3 stage: 30x14x11 p = 2 q = 2 bump
+// channel 74 -> 26 us, 24x16x16 p = 3 q = 2 channel 140 -> 51 us.  q = 1 keeps its
+// 8-node basis: 110 operations a point.
+template <int NB>
+__device__ __forceinline__ double stored_volume_geometry(const MeshArgs& mesh, size_t e, int nd,
+                                                         double Ji[3][3])
+{
+  const double* g = mesh.geov + e * GEOV * NB + nd;
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+    Ji[k / 3][k % 3] = g[k * NB];
+  return g[9 * NB];
+}
+
+template <int NF>
+__device__ __forceinline__ double stored_face_geometry(const MeshArgs& mesh, size_t e, int f,
+                                                       int fpt, double Ji[3][3], double* nv)
+{
+  const double* g = mesh.geof + (e * 6 + f) * GEOF * NF + fpt;
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+    Ji[k / 3][k % 3] = g[k * NF];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    nv[k] = g[(9 + k) * NF];
+  return g[12 * NF];
 }
 
 // Copies the 1D tables of (P, Q) into LDS: the lane-dependent table reads of
@@ -399,7 +448,7 @@ struct FaceDims
 // type: double, or float for the mixed-precision form (the records are
 // computed in double and rounded once on the store).  Called by every
 // thread of the block; sR needs 4*64 doubles.
-template <int P, int Q, typename TT, bool AFF = false>
+template <int P, int Q, typename TT, bool AFF = false, bool STO = false>
 __device__ __forceinline__ void produce_traces(const MeshArgs& mesh, const Phys& ph,
                                                const PTab& pt, const QTab& qt,
                                                const double (*sV)[5][FaceDims<P>::NB],
@@ -456,7 +505,10 @@ __device__ __forceinline__ void produce_traces(const MeshArgs& mesh, const Phys&
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
       double Ji[3][3], nv[3];
-      face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
+      if constexpr (STO)
+        stored_face_geometry<NF>(mesh, ee, f, fpt, Ji, nv);
+      else
+        face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
       double gr[3][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -528,33 +580,26 @@ __global__ __launch_bounds__(64) void dgx_trace_kernel(MeshArgs mesh, Phys ph,
     for (int r = 0; r < 5; ++r)
       sV[le][r][nd0] = V[((size_t)(e0 + le) * 5 + r) * NB + nd0];
   }
-  for (int x = tid; x < EPW * NG * 3; x += 64)
-  {
-    int ee = e0 + x / (NG * 3);
-    sX[x / (NG * 3)][x % (NG * 3)] =
-        (ee < mesh.nelem) ? mesh.nodes[(size_t)ee * NG * 3 + x % (NG * 3)] : 0.0;
-  }
-  if (AFF && tid < EPW)
-    affine_record(mesh.nodes, e0 + tid, mesh.nelem, sG[tid]);
+  load_geometry<Q, EPW, AFF>(mesh, e0, sX, sG);
   __syncthreads();
   produce_traces<P, Q, TT, AFF>(mesh, ph, sPT, sQT, sV, sX, sG, sNb, sBt, sR, e0, Tout, status);
 }
 
 // LDS of one stage-body block, carved from a byte buffer so that kernels
 // holding the bodies of several orders (the ensemble stage kernel) give
-// them one shared region: state [EPW][5][NB], own geometry nodes
-// [EPW][NG*3], affine-element records [EPW][GREC], the exchange region
+// them one shared region: state [EPW][5][NB], own geometry nodes [EPW][NG*3]
+// or affine-element records [EPW][GREC] (neither with stored geometry, STO),
+// the exchange region
 // (volume flux of one direction, then one face pass), the 1D tables and the
 // face table.
-template <int P, int Q>
+template <int P, int Q, bool AFF, bool STO = false>
 struct StageLds
 {
   using FD = FaceDims<P>;
   static constexpr int EPW = FD::EPW, NB = FD::NB, NG = (Q + 1) * (Q + 1) * (Q + 1);
   static constexpr size_t oV  = 0;
   static constexpr size_t oX  = oV + sizeof(double) * EPW * 5 * NB;
-  static constexpr size_t oG  = oX + sizeof(double) * EPW * NG * 3;
-  static constexpr size_t oR  = oG + sizeof(double) * EPW * GREC;
+  static constexpr size_t oR  = oX + sizeof(double) * EPW * (STO ? 0 : (AFF ? GREC : NG * 3));
   static constexpr size_t oPT = oR + sizeof(double) * FD::RG;
   static constexpr size_t oQT = oPT + sizeof(PTab);
   static constexpr size_t oNb = oQT + sizeof(QTab);
@@ -574,23 +619,23 @@ struct StageLds
 // gradients, tractions, BR2 or dual-consistency terms), which equals the
 // full one at mu = 0 (whose viscous terms are exact zeros) without reading
 // the tractions of the records: the adjoint's d f / d mu.
-template <int P, int Q, typename TT, bool AFF = false, bool INV = false>
+template <int P, int Q, typename TT, bool AFF = false, bool INV = false, bool STO = false>
 __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys& ph,
                                                const StageArgs& sa,
                                                const double* __restrict__ lam, int* status,
                                                int block, unsigned char* lds)
 {
   using FD = FaceDims<P>;
-  using SL = StageLds<P, Q>;
+  using SL = StageLds<P, Q, AFF, STO>;
   constexpr int N = FD::N, NB = FD::NB, NF = FD::NF, EPW = FD::EPW, FS = FD::FS;
   constexpr int NG = (Q + 1) * (Q + 1) * (Q + 1);
-  // the short form of the face physics; at q > 1, where the kernel spills, it
-  // measured 1-5 % slower
-  constexpr bool FAST = Q == 1 && sizeof(TT) == sizeof(double);
+  // the short form of the face physics; where the q > 1 kernel evaluates the
+  // geometry basis and spills, it measured 1-5 % slower
+  constexpr bool FAST = (Q == 1 || STO) && sizeof(TT) == sizeof(double);
 
   auto sV  = reinterpret_cast<double(*)[5][NB]>(lds + SL::oV);
   auto sX  = reinterpret_cast<double(*)[NG * 3]>(lds + SL::oX);      // own geometry nodes
-  auto sG  = reinterpret_cast<double(*)[GREC]>(lds + SL::oG);        // affine records
+  auto sG  = reinterpret_cast<double(*)[GREC]>(lds + SL::oX);        // or affine records
   double* sR = reinterpret_cast<double*>(lds + SL::oR);  // volume flux, then one face pass
   PTab& sPT = *reinterpret_cast<PTab*>(lds + SL::oPT);
   QTab& sQT = *reinterpret_cast<QTab*>(lds + SL::oQT);
@@ -616,14 +661,8 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
     for (int r = 0; r < 5; ++r)
       sV[le][r][nd0] = sa.Vin[((size_t)e * 5 + r) * NB + nd0];
   }
-  for (int x = tid; x < EPW * NG * 3; x += 64)
-  {
-    int l  = x / (NG * 3);
-    int ee = e0 + l;
-    sX[l][x % (NG * 3)] = (ee < mesh.nelem) ? mesh.nodes[(size_t)ee * NG * 3 + x % (NG * 3)] : 0.0;
-  }
-  if (AFF && tid < EPW)
-    affine_record(mesh.nodes, e0 + tid, mesh.nelem, sG[tid]);
+  if constexpr (!STO)
+    load_geometry<Q, EPW, AFF>(mesh, e0, sX, sG);
   __syncthreads();
 
   const int idx[3] = {nd0 % N, (nd0 / N) % N, nd0 / (N * N)};
@@ -635,9 +674,14 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
   // ---- volume: velocity gradient, fluxes ----
   if (vact)
   {
-    double J[3][3], det;
-    geometry_at<Q, AFF>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
-    wJ = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]] * det;
+    if constexpr (STO)
+      wJ = stored_volume_geometry<NB>(mesh, e, nd0, Ji);
+    else
+    {
+      double J[3][3], det;
+      geometry_at<Q, AFF>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
+      wJ = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]] * det;
+    }
     double Vq[5];
 #pragma unroll
     for (int r = 0; r < 5; ++r)
@@ -736,8 +780,11 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       const int gi0 = (nd == 0) ? 0 : a;
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
-      double JiL[3][3], nv[3];
-      const double fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
+      double JiL[3][3], nv[3], fJ;
+      if constexpr (STO)
+        fJ = stored_face_geometry<NF>(mesh, ee, f, fpt, JiL, nv);
+      else
+        fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
       if (en >= 0 && FAST)
         roe_flux_fp64(UL, Ub, nv, ph.gamma, fpo.G);
       else if (en >= 0)
@@ -771,8 +818,11 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       const int gi0 = (nd == 0) ? 0 : a;
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
-      double JiL[3][3], nv[3];
-      const double fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
+      double JiL[3][3], nv[3], fJ;
+      if constexpr (STO)
+        fJ = stored_face_geometry<NF>(mesh, ee, f, fpt, JiL, nv);
+      else
+        fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
       // affine meshes: the face's constant coefficient
       const double lamL =
           AFF ? mesh.lamf[(size_t)ee * 6 + f] : lam[((size_t)ee * 6 + f) * NF + fpt];
@@ -902,18 +952,18 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
   if (sa.Tout)
   {
     __syncthreads();
-    produce_traces<P, Q, TT, AFF>(mesh, ph, pt, qt, sV, sX, sG, sNb, sBt, sR, e0,
-                                  reinterpret_cast<TT*>(sa.Tout), status);
+    produce_traces<P, Q, TT, AFF, STO>(mesh, ph, pt, qt, sV, sX, sG, sNb, sBt, sR, e0,
+                                       reinterpret_cast<TT*>(sa.Tout), status);
   }
 }
 
-template <int P, int Q, typename TT, bool AFF = false>
+template <int P, int Q, typename TT, bool AFF = false, bool STO = false>
 __device__ __forceinline__ void stage_body(const MeshArgs& mesh, const Phys& ph,
                                            const StageArgs& sa, const double* __restrict__ lam,
                                            int* status, int block)
 {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[StageLds<P, Q>::bytes];
-  stage_body_lds<P, Q, TT, AFF>(mesh, ph, sa, lam, status, block, lds);
+  __shared__ __attribute__((aligned(16))) unsigned char lds[StageLds<P, Q, AFF, STO>::bytes];
+  stage_body_lds<P, Q, TT, AFF, false, STO>(mesh, ph, sa, lam, status, block, lds);
 }
 
 #include "dgx_tile.hpp"
