@@ -455,6 +455,39 @@ __device__ __forceinline__ void visc_apply_n(const ViscState& vs, const double G
     Qn[r] = Q[0][r] * n[0] + Q[1][r] * n[1] + Q[2][r] * n[2];
 }
 
+// Boundary states that take a few operations from the interior trace UL and
+// the outward normal n: free stream (-3), inviscid wall (-4), no-slip wall (-7).
+template <typename T>
+__device__ __forceinline__ void wall_state(int bt, const T* UL, const double* n, const Phys& ph,
+                                           T* Ub)
+{
+  if (bt == -3)  // freestream
+  {
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      Ub[i] = ph.Ufr[i];
+  }
+  else if (bt == -4)  // inviscid wall: remove the normal velocity
+  {
+    T ir = rcp(UL[0]);
+    T up = UL[1] * ir, vp = UL[2] * ir, wp = UL[3] * ir;
+    T vdn = up * n[0] + vp * n[1] + wp * n[2];
+    Ub[0] = UL[0];
+    Ub[1] = UL[0] * (up - vdn * n[0]);
+    Ub[2] = UL[0] * (vp - vdn * n[1]);
+    Ub[3] = UL[0] * (wp - vdn * n[2]);
+    Ub[4] = UL[4];
+  }
+  else  // no-slip wall, energy taken from the interior
+  {
+    Ub[0] = UL[0]; Ub[1] = 0.0; Ub[2] = 0.0; Ub[3] = 0.0; Ub[4] = UL[4];
+  }
+}
+
+// The characteristic boundaries, inflow (-5) and outflow (-6): pow, square
+// roots and divisions, kept out of the face loops.
+__host__ __device__ __forceinline__ bool characteristic_bc(int bt) { return bt == -5 || bt == -6; }
+
 // Boundary state Ub from interior trace UL and outward normal n.
 // Returns false when the subsonic-inflow Mach quadratic has no
 // non-negative root (the reference aborts there on the host).  T is double
@@ -467,26 +500,9 @@ __device__ __forceinline__ bool boundary_state(int bt, const T* UL, const double
   double gamma = ph.gamma, gm1 = gamma - 1.0;
   switch (bt)
   {
-    case -3:  // freestream
-#pragma unroll
-      for (int i = 0; i < 5; ++i)
-        Ub[i] = ph.Ufr[i];
-      return true;
-    case -4:  // inviscid wall: remove the normal velocity
-    {
-      T ir = rcp(UL[0]);
-      T up = UL[1] * ir, vp = UL[2] * ir, wp = UL[3] * ir;
-      T vdn = up * n[0] + vp * n[1] + wp * n[2];
-      Ub[0] = UL[0];
-      Ub[1] = UL[0] * (up - vdn * n[0]);
-      Ub[2] = UL[0] * (vp - vdn * n[1]);
-      Ub[3] = UL[0] * (wp - vdn * n[2]);
-      Ub[4] = UL[4];
-      return true;
-    }
-    case -7:  // no-slip wall, energy taken from the interior
-      Ub[0] = UL[0]; Ub[1] = 0.0; Ub[2] = 0.0; Ub[3] = 0.0; Ub[4] = UL[4];
-      return true;
+    case -3:
+    case -4:
+    case -7: wall_state(bt, UL, n, ph, Ub); return true;
     case -5:  // subsonic inflow: total T, total P, outgoing Riemann invariant
     {
       double R = ph.Rgas, Tt = ph.Tt, Pt = ph.Pt;

@@ -111,8 +111,8 @@ struct StageArgs
   // sum of R^2, R = -B3^T W f (the residual norm of this stage's f), for
   // tile_blocks(p, nelem) blocks
   double* normp = nullptr;
-  // FP64 tiled kernel only: 0 writes just the boundary states of Vout's
-  // domain-boundary faces to Tout (all that its next stage reads); the other
+  // FP64 tiled kernel only: 0 writes just the boundary states of Vout's inflow
+  // and outflow faces to Tout (all that its next stage reads); the other
   // kernels, and the adjoint, read the trace records of every face
   int records = 1;
 };
@@ -144,7 +144,7 @@ bool tile_valid(int p, int q, int tile, int waves);
 hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
                              const double* lam, int* status, int waves, hipStream_t st);
 // boundary states of V (q = 1) into the boundary section of the record set
-// Tout; nothing to do on periodic meshes
+// Tout; nothing to do on meshes without inflow or outflow
 hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
                              double* Tout, int* status, hipStream_t st);
 hipError_t upload_tables_tile(const PTab* pt, const QTab* qt);

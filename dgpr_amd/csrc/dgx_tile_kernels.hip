@@ -78,10 +78,10 @@ static hipError_t launch_boundary(const MeshArgs& m, const Phys& ph, const doubl
 hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
                              double* Tout, int* status, hipStream_t st)
 {
-  bool walls = false;
+  bool any = false;
   for (int i = 0; i < 6; ++i)
-    walls = walls || m.bounds[i] != -2;
-  if (!walls)
+    any = any || characteristic_bc(m.bounds[i]);
+  if (!any)
     return hipSuccess;
   switch (p)
   {

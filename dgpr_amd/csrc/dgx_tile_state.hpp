@@ -8,7 +8,7 @@
 // the neighbour's 4 nodes behind each face point instead (L2 and Infinity
 // Cache hits mostly: every element is read once as own and six times as a
 // neighbour) leaves the state arrays; the traces of the new state need not be
-// produced, only the boundary states of domain-boundary faces.  What bounds
+// produced, only the states of inflow and outflow boundary faces.  What bounds
 // this kernel is FP64 issue (about 2300 FP64 and 160 matrix instructions per
 // wavefront of 128 nodes).  Per RK4 stage, 64^3 p = 3 cube: 1313 us against
 // 1698 us (traffic 5.1 against 7.5 GB); 64^3 p = 1 cube: 299 us against
@@ -23,8 +23,9 @@ struct Const
   static constexpr int value = I;
 };
 
-// Whether a face of the tile's E elements lies on a domain boundary (uniform);
-// fills the face table as tile_face_table does.
+// Fills the face table as tile_face_table does; whether a face of the tile's E
+// elements lies on a characteristic boundary (uniform), whose state the next
+// stage reads instead of forming it (wall_state) at the face point.
 template <int E>
 __device__ __forceinline__ bool state_face_table(const MeshArgs& mesh, int e0, int (*sNb)[6],
                                                  int (*sBt)[6])
@@ -32,7 +33,7 @@ __device__ __forceinline__ bool state_face_table(const MeshArgs& mesh, int e0, i
   static_assert(E * 6 <= 64, "one face per lane");
   tile_face_table<E>(mesh, e0, sNb, sBt);
   const int x = threadIdx.x;  // each lane reads back the face it wrote
-  return __any(x < E * 6 && sNb[x / 6][x % 6] < 0);
+  return __any(x < E * 6 && characteristic_bc(sBt[x / 6][x % 6]));
 }
 
 // The lane index, opaque to common subexpressions: each face subpass derives
@@ -294,8 +295,8 @@ __device__ __forceinline__ void state_face_subpass(
     const MeshArgs& mesh, const Phys& ph, const PTab& pt, const QTab& qt,
     const double* __restrict__ Tin, const double (*sV)[5][TileDims<P, R>::NB],
     const double (*sX)[(Q + 1) * (Q + 1) * (Q + 1) * 3], const double (*sG)[GREC],
-    const double (*sH)[NbrGeo<AFF>::n], const int (*sNb)[6], double* sR, const MfTabs& mf, int e0,
-    double (&acc)[R][5], FaceData<P>& fd, Next next)
+    const double (*sH)[NbrGeo<AFF>::n], const int (*sNb)[6], const int (*sBt)[6], double* sR,
+    const MfTabs& mf, int e0, double (&acc)[R][5], FaceData<P>& fd, Next next)
 {
   using TD = TileDims<P, R>;
   using FL = FaceLane<P, R, S>;
@@ -392,11 +393,18 @@ __device__ __forceinline__ void state_face_subpass(
     double irB = irR;
     if (en < 0)
     {
-      // boundary state written with Vin
-      const double* B = Tin + (size_t)mesh.nelem * 6 * 8 * NF + (size_t)(-1 - en) * 5 * NF + a + N * b;
+      const int bt = sBt[l][f];
+      if (characteristic_bc(bt))
+      {
+        // written with Vin
+        const double* B =
+            Tin + (size_t)mesh.nelem * 6 * 8 * NF + (size_t)(-1 - en) * 5 * NF + a + N * b;
 #pragma unroll
-      for (int r = 0; r < 5; ++r)
-        Ub[r] = B[r * NF];
+        for (int r = 0; r < 5; ++r)
+          Ub[r] = B[r * NF];
+      }
+      else
+        wall_state(bt, UL, nv, ph, Ub);
       irB = rcp(Ub[0]);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
@@ -479,8 +487,8 @@ __device__ __forceinline__ void state_face_subpass(
   phase_fence();
 }
 
-// Of the tile's new states in sV: the boundary states of its domain-boundary
-// faces (what the next tiled stage reads), or with records != 0 the trace
+// Of the tile's new states in sV: the boundary states of its characteristic
+// boundary faces (what the next tiled stage reads), or with records != 0 the trace
 // records of every face too (see produce_traces, whose layout they have).  One
 // loop over passes of whole faces, the face direction a per-lane value: run
 // by tiles at the domain boundary and by the adjoint's forward sweep only, so
@@ -504,7 +512,7 @@ __device__ __forceinline__ void state_traces(const MeshArgs& mesh, const Phys& p
   {
     const int g = g0 + slot, l = g / 6, f = g % 6, ee = e0 + l;
     const bool fact = (slot < FPS) && (g < NFACE) && (ee < mesh.nelem);
-    const int nb = fact ? sNb[l][f] : 0;
+    const int nb = fact && (records || characteristic_bc(sBt[l][f])) ? sNb[l][f] : 0;
     if (!records && !__any(nb < 0))
       continue;
     const int nd = f >> 1, hi = f & 1;
@@ -778,7 +786,7 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
   auto subpass = [&](auto sc) __attribute__((always_inline)) {
     constexpr int S = decltype(sc)::value;
     state_face_subpass<P, Q, R, S, AFF>(
-        mesh, ph, pt, qt, Tin, sV, sX, sG, sH, sNb, sR, mf, e0, acc, fd,
+        mesh, ph, pt, qt, Tin, sV, sX, sG, sH, sNb, sBt, sR, mf, e0, acc, fd,
         [&]() __attribute__((always_inline)) {
           if constexpr (S + 1 < 3 * TD::NSUB)
             face_load<P, R, S + 1, AFF>(mesh, sa.Vin, lam, sNb, e0, fd);
@@ -884,8 +892,8 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
       sa.normp[block] = sq;
   }
 
-  // ---- of the new state: the boundary states of domain-boundary faces for
-  // the next stage, or (sa.records) the trace records of every face ----
+  // ---- of the new state: the states of characteristic boundary faces for the
+  // next stage, or (sa.records) the trace records of every face ----
   if (sa.Tout && (sa.records || wall))
   {
     __syncthreads();
