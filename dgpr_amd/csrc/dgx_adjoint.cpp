@@ -71,27 +71,46 @@ dgx_status afail(dgx_ctx* c, dgx_status st, const char* fmt, ...)
       return afail((c), DGX_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));       \
   } while (0)
 
-// Workspace of the residual adjoint
-struct AdjScratch
-{
-  DevBuf pvol, aown, anbr;
-};
-
 hipError_t alloc(DevBuf& b, size_t ndouble)
 {
   return hipMalloc(&b.p, ndouble * sizeof(double));
 }
 
-hipError_t alloc_scratch(const dgx_ctx* c, AdjScratch& s)
+// The temporaries of one adjoint call, cut from the context's workspace.  It
+// stays with the context (grown when a call needs more) until
+// dgx_adjoint_release or dgx_destroy: allocating and freeing a dozen buffers
+// took 1-3 ms a call, more than the kernels of a small residual adjoint.
+struct Workspace
 {
-  size_t tr = trace_doubles(c->p, c->nx, c->ny, c->nz);
-  hipError_t e = alloc(s.pvol, c->nstate);
-  if (e == hipSuccess)
-    e = alloc(s.aown, tr);
-  if (e == hipSuccess)
-    e = alloc(s.anbr, tr);
-  return e;
-}
+  double* next = nullptr;
+  hipError_t open(dgx_ctx* c, size_t ndouble)
+  {
+    const size_t need = ndouble * sizeof(double);
+    if (c->adj_ws_bytes < need)
+    {
+      hipError_t e = hipStreamSynchronize(c->stream);
+      if (e == hipSuccess && c->adj_ws)
+        e = hipFree(c->adj_ws);
+      c->adj_ws       = nullptr;
+      c->adj_ws_bytes = 0;
+      if (e == hipSuccess)
+        e = hipMalloc(&c->adj_ws, need);
+      if (e != hipSuccess)
+        return e;
+      c->adj_ws_bytes = need;
+    }
+    next = c->adj_ws;
+    return hipSuccess;
+  }
+  // n doubles, at a multiple of 256 bytes (open() asks for `padded` sizes)
+  double* take(size_t n)
+  {
+    double* p = next;
+    next += padded(n);
+    return p;
+  }
+  static size_t padded(size_t n) { return (n + 31) & ~(size_t)31; }
+};
 
 // one stage kernel launch with explicit physics: Vout = Vbase + cf f(Vin)
 // (Vout may be null), fout = f(Vin) (may be null)
@@ -184,11 +203,44 @@ dgx_status dgx_kinetic_energy(dgx_ctx* c, double* J)
     return DGX_ERR_INVALID;
   if (general_order(c->p, c->q))
     return afail(c, DGX_ERR_UNSUPPORTED, "the adjoint covers 1 <= p, q <= 3");
-  DevBuf g;
-  AHIP(c, alloc(g, c->nstate));
-  AHIP(c, kinetic_energy_dispatch(c->p, c->q, mesh_args(c), c->U, g.p, c->partial, c->stream));
+  AHIP(c, kinetic_energy_dispatch(c->p, c->q, mesh_args(c), c->U, nullptr, c->partial,
+                                  c->stream));
   AHIP(c, sum_dispatch(c->partial, c->npartial, c->sum, c->stream));
   AHIP(c, hipMemcpyAsync(J, c->sum, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  AHIP(c, hipStreamSynchronize(c->stream));
+  return DGX_OK;
+}
+
+static dgx_status vjp_check(dgx_ctx* c)
+{
+  if (general_order(c->p, c->q))
+    return afail(c, DGX_ERR_UNSUPPORTED, "the adjoint covers 1 <= p, q <= 3");
+  if (c->prec != DGX_PREC_FP64)
+    return afail(c, DGX_ERR_UNSUPPORTED, "the residual adjoint needs DGX_PREC_FP64");
+  return DGX_OK;
+}
+
+// w and g on the host (host) or the device
+static dgx_status residual_vjp(dgx_ctx* c, const double* w, double* g, bool host)
+{
+  dgx_status st = vjp_check(c);
+  if (st != DGX_OK)
+    return st;
+  const size_t n = c->nstate, tr = trace_doubles(c->p, c->nx, c->ny, c->nz);
+  Workspace ws;
+  AHIP(c, ws.open(c, 3 * Workspace::padded(n) + 2 * Workspace::padded(tr)));
+  double *pvol = ws.take(n), *a = ws.take(n), *b = ws.take(n);
+  double *aown = ws.take(tr), *anbr = ws.take(tr);
+  AHIP(c, ensure_traces(c));
+  // f = B3^-1 f_g(B3 U): (df/dU)^T w = B3^T (df_g/dV)^T B3^-T w
+  if (host)
+    AHIP(c, hipMemcpyAsync(a, w, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  AHIP(c, basis_dispatch(c->p, host ? a : w, b, c->nelem, 3, c->stream));
+  AHIP(c, adjoint_dispatch(c->p, c->q, mesh_args(c), c->phys, c->U, c->TU, c->lam, b, pvol, aown,
+                           anbr, a, c->stream));
+  AHIP(c, basis_dispatch(c->p, a, host ? b : g, c->nelem, 2, c->stream));
+  if (host)
+    AHIP(c, hipMemcpyAsync(g, b, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   AHIP(c, hipStreamSynchronize(c->stream));
   return DGX_OK;
 }
@@ -197,37 +249,23 @@ dgx_status dgx_residual_vjp(dgx_ctx* c, const double* w_host, double* g_host)
 {
   if (!c || !w_host || !g_host)
     return DGX_ERR_INVALID;
-  if (general_order(c->p, c->q))
-    return afail(c, DGX_ERR_UNSUPPORTED, "the adjoint covers 1 <= p, q <= 3");
-  if (c->prec != DGX_PREC_FP64)
-    return afail(c, DGX_ERR_UNSUPPORTED, "the residual adjoint needs DGX_PREC_FP64");
-  AdjScratch s;
-  DevBuf a, b;
-  AHIP(c, alloc_scratch(c, s));
-  AHIP(c, alloc(a, c->nstate));
-  AHIP(c, alloc(b, c->nstate));
-  AHIP(c, ensure_traces(c));
-  // f = B3^-1 f_g(B3 U): (df/dU)^T w = B3^T (df_g/dV)^T B3^-T w
-  AHIP(c, hipMemcpyAsync(a.p, w_host, c->nstate * sizeof(double), hipMemcpyHostToDevice,
-                         c->stream));
-  AHIP(c, basis_dispatch(c->p, a.p, b.p, c->nelem, 3, c->stream));
-  AHIP(c, adjoint_dispatch(c->p, c->q, mesh_args(c), c->phys, c->U, c->TU, c->lam, b.p,
-                           s.pvol.p, s.aown.p, s.anbr.p, a.p, c->stream));
-  AHIP(c, basis_dispatch(c->p, a.p, b.p, c->nelem, 2, c->stream));
-  AHIP(c, hipMemcpyAsync(g_host, b.p, c->nstate * sizeof(double), hipMemcpyDeviceToHost,
-                         c->stream));
-  AHIP(c, hipStreamSynchronize(c->stream));
-  return DGX_OK;
+  return residual_vjp(c, w_host, g_host, true);
+}
+
+dgx_status dgx_residual_vjp_device(dgx_ctx* c, const double* w_dev, double* g_dev)
+{
+  if (!c || !w_dev || !g_dev)
+    return DGX_ERR_INVALID;
+  return residual_vjp(c, w_dev, g_dev, false);
 }
 
 dgx_status dgx_residual_vjp_device_noalloc(dgx_ctx* c, const double* w_dev, double* g_dev)
 {
   if (!c || !w_dev || !g_dev)
     return DGX_ERR_INVALID;
-  if (general_order(c->p, c->q))
-    return afail(c, DGX_ERR_UNSUPPORTED, "the adjoint covers 1 <= p, q <= 3");
-  if (c->prec != DGX_PREC_FP64)
-    return afail(c, DGX_ERR_UNSUPPORTED, "the residual adjoint needs DGX_PREC_FP64");
+  dgx_status st = vjp_check(c);
+  if (st != DGX_OK)
+    return st;
   const size_t n = c->nstate;
   const size_t tr = trace_doubles(c->p, c->nx, c->ny, c->nz);
   const size_t need = 3 * n + 2 * tr;
@@ -266,8 +304,10 @@ dgx_status dgx_residual_vjp_device_noalloc(dgx_ctx* c, const double* w_dev, doub
   return DGX_OK;
 }
 
-dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t interval, double* J,
-                           double* dJdU0_host, double* dJdmu)
+// the gradient with respect to the initial state goes to dJdU0_host or
+// dJdU0_dev (either may be null)
+static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t interval,
+                              double* J, double* dJdU0_host, double* dJdU0_dev, double* dJdmu)
 {
   if (!c || nsteps == 0 || !(dt > 0.0))
     return DGX_ERR_INVALID;
@@ -280,20 +320,14 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   const size_t n = c->nstate;
   const size_t ntr = trace_doubles(c->p, c->nx, c->ny, c->nz);
 
-  DevBuf lam, lk, acur, asum, f0, dpart, dsum, final_state;
-  AHIP(c, alloc(lam, n));
-  AHIP(c, alloc(lk, n));
-  AHIP(c, alloc(acur, n));
-  AHIP(c, alloc(asum, n));
-  AHIP(c, alloc(final_state, n));
-  if (dJdmu)
-    AHIP(c, alloc(f0, n));
   const int ndot = 1024;
-  AHIP(c, alloc(dpart, ndot));
-  // one dot product per reverse stage for dJ/dmu, read back once at the end
-  AHIP(c, alloc(dsum, dJdmu ? 4 * nsteps : 1));
-  AdjScratch scr;
-  AHIP(c, alloc_scratch(c, scr));
+  const size_t nsum = dJdmu ? 4 * nsteps : 1;  // one dot product per reverse stage, read back once
+  Workspace ws;
+  AHIP(c, ws.open(c, (dJdmu ? 7 : 6) * Workspace::padded(n) + 2 * Workspace::padded(ntr) +
+                         Workspace::padded(ndot) + Workspace::padded(nsum)));
+  double *lam = ws.take(n), *lk = ws.take(n), *acur = ws.take(n), *asum = ws.take(n);
+  double *final_state = ws.take(n), *pvol = ws.take(n), *f0 = dJdmu ? ws.take(n) : nullptr;
+  double *aown = ws.take(ntr), *anbr = ws.take(ntr), *dpart = ws.take(ndot), *dsum = ws.take(nsum);
 
   // Schedule.  interval == 0: keep every stage state with its trace records
   // (and f for dJ/dmu) from the forward sweep when that fits in three
@@ -363,7 +397,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   auto wa_of = [&](int k) { return (k == 2) ? dt : 0.5 * dt; };
   auto reverse_step = [&](double* const* Si, double* const* Ti, double* const* Ki) -> dgx_status {
     // lk of stage 3 = w_l l
-    AHIP(c, adj_tail_dispatch(lam.p, nullptr, nullptr, nullptr, lk.p, wl_of(3), 0.0, n,
+    AHIP(c, adj_tail_dispatch(lam, nullptr, nullptr, nullptr, lk, wl_of(3), 0.0, n,
                               c->stream));
     for (int i = 3; i >= 0; --i)
     {
@@ -371,20 +405,20 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
       {
         // df/dmu at S_i: (k_(i+1) - f(S_i; 0)) / mu, f(S_i; 0) the inviscid
         // right-hand side from S_i and its records
-        AHIP(c, inviscid_rhs_dispatch(c->p, c->q, mesh_args(c), c->phys, Si[i], Ti[i], f0.p,
+        AHIP(c, inviscid_rhs_dispatch(c->p, c->q, mesh_args(c), c->phys, Si[i], Ti[i], f0,
                                       c->lam, c->status, c->stream));
-        AHIP(c, dot_dispatch(lk.p, Ki[i], f0.p, 1.0 / c->phys.mu, n, dpart.p, ndot,
-                             dsum.p + ndmu, c->stream));
+        AHIP(c, dot_dispatch(lk, Ki[i], f0, 1.0 / c->phys.mu, n, dpart, ndot,
+                             dsum + ndmu, c->stream));
         ++ndmu;
       }
-      AHIP(c, adjoint_dispatch(c->p, c->q, mesh_args(c), c->phys, Si[i], Ti[i], c->lam, lk.p,
-                               scr.pvol.p, scr.aown.p, scr.anbr.p, acur.p, c->stream));
+      AHIP(c, adjoint_dispatch(c->p, c->q, mesh_args(c), c->phys, Si[i], Ti[i], c->lam, lk,
+                               pvol, aown, anbr, acur, c->stream));
       // asum = l + a_3 + ... + a_i; lk of stage i-1 = w_l l + w_a a_i
-      AHIP(c, adj_tail_dispatch(lam.p, acur.p, (i == 3) ? lam.p : asum.p, asum.p,
-                                (i > 0) ? lk.p : nullptr, (i > 0) ? wl_of(i - 1) : 0.0,
+      AHIP(c, adj_tail_dispatch(lam, acur, (i == 3) ? lam : asum, asum,
+                                (i > 0) ? lk : nullptr, (i > 0) ? wl_of(i - 1) : 0.0,
                                 (i > 0) ? wa_of(i - 1) : 0.0, n, c->stream));
     }
-    std::swap(lam.p, asum.p);  // the adjoint of the step's start state becomes l
+    std::swap(lam, asum);  // the adjoint of the step's start state becomes l
     return DGX_OK;
   };
 
@@ -457,10 +491,10 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   // forward sweep
   if (store_all)
   {
-    dgx_status st = forward_store(c->U, nsteps, final_state.p);
+    dgx_status st = forward_store(c->U, nsteps, final_state);
     if (st != DGX_OK)
       return st;
-    AHIP(c, copy_state(c, c->U, final_state.p));
+    AHIP(c, copy_state(c, c->U, final_state));
     drop_traces(c);
   }
   else
@@ -474,21 +508,21 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
         AHIP(c, copy_state(c, chk[s / K].p, c->U));
       if (seg_store && s == s_last)
       {
-        dgx_status st = forward_store(c->U, nsteps - s_last, final_state.p);
+        dgx_status st = forward_store(c->U, nsteps - s_last, final_state);
         if (st != DGX_OK)
           return st;
-        AHIP(c, copy_state(c, c->U, final_state.p));
+        AHIP(c, copy_state(c, c->U, final_state));
         drop_traces(c);
         break;
       }
       AHIP(c, step_ctx(c, dt));
     }
     if (!seg_store)
-      AHIP(c, copy_state(c, final_state.p, c->U));
+      AHIP(c, copy_state(c, final_state, c->U));
   }
 
   // objective and its gradient at the final state
-  AHIP(c, kinetic_energy_dispatch(c->p, c->q, mesh_args(c), final_state.p, lam.p, c->partial,
+  AHIP(c, kinetic_energy_dispatch(c->p, c->q, mesh_args(c), final_state, lam, c->partial,
                                   c->stream));
   AHIP(c, sum_dispatch(c->partial, c->npartial, c->sum, c->stream));
   double Jv = 0.0;
@@ -509,7 +543,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
     {
       const uint64_t s0 = sg * K, s1 = (s0 + K < nsteps) ? s0 + K : nsteps;
       // the segment's end state is not needed again: acur is free here
-      dgx_status st = (sg + 1 < nchk) ? forward_store(chk[sg].p, s1 - s0, acur.p) : DGX_OK;
+      dgx_status st = (sg + 1 < nchk) ? forward_store(chk[sg].p, s1 - s0, acur) : DGX_OK;
       if (st == DGX_OK)
         st = reverse_store(s1 - s0);
       if (st != DGX_OK)
@@ -564,7 +598,7 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   if (ndmu)
   {
     std::vector<double> parts(ndmu);
-    AHIP(c, hipMemcpyAsync(parts.data(), dsum.p, ndmu * sizeof(double), hipMemcpyDeviceToHost,
+    AHIP(c, hipMemcpyAsync(parts.data(), dsum, ndmu * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
     AHIP(c, hipStreamSynchronize(c->stream));
     for (size_t i = ndmu; i-- > 0;)
@@ -573,12 +607,14 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   // gradient with respect to the initial state in the reference layout
   if (dJdU0_host)
   {
-    AHIP(c, basis_dispatch(c->p, lam.p, asum.p, c->nelem, 2, c->stream));
-    AHIP(c, hipMemcpyAsync(dJdU0_host, asum.p, n * sizeof(double), hipMemcpyDeviceToHost,
+    AHIP(c, basis_dispatch(c->p, lam, asum, c->nelem, 2, c->stream));
+    AHIP(c, hipMemcpyAsync(dJdU0_host, asum, n * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
   }
+  if (dJdU0_dev)
+    AHIP(c, basis_dispatch(c->p, lam, dJdU0_dev, c->nelem, 2, c->stream));
   // the context ends at the final state, as after dgx_step
-  AHIP(c, copy_state(c, c->U, final_state.p));
+  AHIP(c, copy_state(c, c->U, final_state));
   drop_traces(c);
   AHIP(c, hipStreamSynchronize(c->stream));
   int h = 0;
@@ -595,13 +631,30 @@ dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t inte
   return DGX_OK;
 }
 
+dgx_status dgx_adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t interval, double* J,
+                           double* dJdU0_host, double* dJdmu)
+{
+  return adjoint_rk4(c, dt, nsteps, interval, J, dJdU0_host, nullptr, dJdmu);
+}
+
+dgx_status dgx_adjoint_rk4_device(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t interval,
+                                  double* J, double* dJdU0_dev, double* dJdmu)
+{
+  return adjoint_rk4(c, dt, nsteps, interval, J, nullptr, dJdU0_dev, dJdmu);
+}
+
 dgx_status dgx_adjoint_set_store_limit(dgx_ctx* c, uint64_t bytes)
 {
   if (!c)
     return DGX_ERR_INVALID;
   c->adj_store_limit = (size_t)bytes;
-  if (bytes && c->adj_store && c->adj_store_bytes > bytes)
-    return dgx_adjoint_release(c);
+  if (bytes && c->adj_store_bytes > bytes)
+  {
+    AHIP(c, hipStreamSynchronize(c->stream));
+    AHIP(c, hipFree(c->adj_store));
+    c->adj_store       = nullptr;
+    c->adj_store_bytes = 0;
+  }
   return DGX_OK;
 }
 
@@ -609,13 +662,16 @@ dgx_status dgx_adjoint_release(dgx_ctx* c)
 {
   if (!c)
     return DGX_ERR_INVALID;
-  if (c->adj_store)
-  {
+  if (c->adj_store || c->adj_ws)
     AHIP(c, hipStreamSynchronize(c->stream));
+  if (c->adj_store)
     AHIP(c, hipFree(c->adj_store));
-    c->adj_store = nullptr;
-    c->adj_store_bytes = 0;
-  }
+  c->adj_store       = nullptr;
+  c->adj_store_bytes = 0;
+  if (c->adj_ws)
+    AHIP(c, hipFree(c->adj_ws));
+  c->adj_ws       = nullptr;
+  c->adj_ws_bytes = 0;
   return DGX_OK;
 }
 

@@ -693,12 +693,15 @@ __global__ __launch_bounds__(64) void dgx_kinetic_energy_kernel(MeshArgs mesh,
     const double ir = 1.0 / s[0];
     const double u = s[1] * ir, v = s[2] * ir, w = s[3] * ir;
     k = wJ * 0.5 * (s[1] * u + s[2] * v + s[3] * w);
-    double* g = grad + (size_t)e * 5 * NB + nd0;
-    g[0]      = -0.5 * wJ * (u * u + v * v + w * w);
-    g[NB]     = wJ * u;
-    g[2 * NB] = wJ * v;
-    g[3 * NB] = wJ * w;
-    g[4 * NB] = 0.0;
+    if (grad)
+    {
+      double* g = grad + (size_t)e * 5 * NB + nd0;
+      g[0]      = -0.5 * wJ * (u * u + v * v + w * w);
+      g[NB]     = wJ * u;
+      g[2 * NB] = wJ * v;
+      g[3 * NB] = wJ * w;
+      g[4 * NB] = 0.0;
+    }
   }
   red[tid] = k;
   __syncthreads();

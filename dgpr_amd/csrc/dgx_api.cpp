@@ -375,6 +375,8 @@ dgx_status dgx_destroy(dgx_ctx* c)
       (void)hipFree(b);
   if (c->adj_store)
     (void)hipFree(c->adj_store);
+  if (c->adj_ws)
+    (void)hipFree(c->adj_ws);
   if (c->status)
     (void)hipFree(c->status);
   if (c->stream)

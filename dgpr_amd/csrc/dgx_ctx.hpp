@@ -45,6 +45,8 @@ struct dgx_ctx
   double* adj_store;       // stored stages of the last dgx_adjoint_rk4 (kept:
   size_t adj_store_bytes;  // freeing tens of GB can take seconds)
   size_t adj_store_limit;  // most bytes that store may take (0: no limit)
+  double* adj_ws;          // workspace of the adjoint calls, kept likewise
+  size_t adj_ws_bytes;
   int* status;      // kernel-side error flags
   int npartial;
   size_t bytes;

@@ -214,7 +214,7 @@ hipError_t adjoint_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, con
                             double* pvol, double* aown, double* anbr, double* psiV,
                             hipStream_t st);
 // kinetic energy (per-block partials in partial[resid_out_blocks]) and its
-// gradient with respect to the Gauss-nodal state
+// gradient with respect to the Gauss-nodal state (may be null)
 hipError_t kinetic_energy_dispatch(int p, int q, const MeshArgs& m, const double* V,
                                    double* grad, double* partial, hipStream_t st);
 // one pass of the reverse RK stage algebra: sum_out = sum_in + a and

@@ -118,7 +118,9 @@ def lib():
         L.dgx_mesh_is_affine.argtypes = [C.POINTER(_CMesh), C.POINTER(C.c_int)]
         L.dgx_kinetic_energy.argtypes = [P_ctx, PD]
         L.dgx_residual_vjp.argtypes = [P_ctx, PD, PD]
+        L.dgx_residual_vjp_device.argtypes = [P_ctx, C.c_void_p, C.c_void_p]
         L.dgx_adjoint_rk4.argtypes = [P_ctx, D, U64, U64, PD, PD, PD]
+        L.dgx_adjoint_rk4_device.argtypes = [P_ctx, D, U64, U64, PD, C.c_void_p, PD]
         L.dgx_adjoint_release.argtypes = [P_ctx]
         L.dgx_adjoint_set_store_limit.argtypes = [P_ctx, U64]
         L.dgx_residual_vjp_device_noalloc.argtypes = [P_ctx, C.c_void_p, C.c_void_p]
@@ -172,6 +174,7 @@ def lib():
                    "dgx_ensemble_step", "dgx_ensemble_sync", "dgx_ensemble_get_stream",
                    "dgx_ensemble_autotune", "dgx_ensemble_set_layout",
                    "dgx_ensemble_member_tuning", "dgx_kinetic_energy", "dgx_residual_vjp",
+                   "dgx_residual_vjp_device", "dgx_adjoint_rk4_device",
                    "dgx_adjoint_rk4", "dgx_adjoint_release", "dgx_adjoint_set_store_limit",
                    "dgx_residual_vjp_device_noalloc"):
             getattr(L, nm).restype = st
@@ -461,6 +464,12 @@ class Solver:
         _chk(lib().dgx_residual_vjp(self.ctx, _p(w), _p(g)), self.ctx)
         return g
 
+    def residual_vjp_device(self, w_ptr, g_ptr):
+        """residual_vjp on device buffers given as integer addresses; returns
+        after completion."""
+        _chk(lib().dgx_residual_vjp_device(self.ctx, C.c_void_p(int(w_ptr)),
+                                           C.c_void_p(int(g_ptr))), self.ctx)
+
     def residual_vjp_device_noalloc(self, w_ptr, g_ptr):
         """dgx_residual_vjp_device_noalloc on device buffers given as integer
         addresses: (df/dU)^T w into g with the library's fixed workspace."""
@@ -477,8 +486,18 @@ class Solver:
                                    C.byref(dmu) if want_mu else None), self.ctx)
         return J.value, g, (dmu.value if want_mu else None)
 
+    def adjoint_rk4_device(self, dt, nsteps, g_ptr, interval=0, want_mu=True):
+        """adjoint_rk4 with the state gradient written to a device buffer given
+        as an integer address; returns (J, dJ/dmu or None)."""
+        J, dmu = C.c_double(), C.c_double()
+        _chk(lib().dgx_adjoint_rk4_device(self.ctx, dt, int(nsteps), int(interval), C.byref(J),
+                                          C.c_void_p(int(g_ptr)),
+                                          C.byref(dmu) if want_mu else None), self.ctx)
+        return J.value, (dmu.value if want_mu else None)
+
     def adjoint_release(self):
-        """Free the stored-stage buffer adjoint_rk4 keeps between calls."""
+        """Free the stored-stage buffer and the workspace that the adjoint
+        calls keep between calls."""
         _chk(lib().dgx_adjoint_release(self.ctx), self.ctx)
 
     def adjoint_store_limit(self, nbytes):

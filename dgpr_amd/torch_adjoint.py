@@ -8,13 +8,13 @@
     dJ/dU0 and dJ/dmu through ``dgx_adjoint_rk4`` (discrete adjoint of the
     stages: every stage state kept from the forward sweep when it fits in
     device memory, else checkpoints every ceil(sqrt(n)) steps, or every
-    ``interval`` steps when given).  The stored stages stay with the solver
-    for later backward passes until ``solver.adjoint_release()`` or
-    ``solver.close()``.
+    ``interval`` steps when given).  The stored stages and the workspace
+    stay with the solver for later backward passes until
+    ``solver.adjoint_release()`` or ``solver.close()``.
 
 Both act on meshes with any boundary types.  States are float64 tensors in the simstate layout U[e][r][bf]:
-device tensors are handed to the library by address after the caller's
-stream is drained, host tensors are copied.  The library runs on its own
+device tensors (states and gradients) are handed to the library by address
+after the caller's stream is drained, host tensors are copied.  The library runs on its own
 stream and every call returns after completion, so results are ready when
 these functions return.  There is no CPU fallback: without libdgx or a HIP
 device the calls raise.
@@ -64,8 +64,14 @@ class ResidualFunction(torch.autograd.Function):
         (U,) = ctx.saved_tensors
         solver = ctx.solver
         _load_state(solver, U)
+        if U.is_cuda:
+            w = g.detach().to(U.device, torch.float64).contiguous()
+            gU = torch.empty(U.shape, dtype=torch.float64, device=U.device)
+            torch.cuda.current_stream(U.device).synchronize()
+            solver.residual_vjp_device(w.data_ptr(), gU.data_ptr())
+            return gU, None
         gU = solver.residual_vjp(g.detach().reshape(-1).cpu().numpy())
-        return torch.from_numpy(gU).to(U.device).view_as(U), None
+        return torch.from_numpy(gU).view_as(U), None
 
 
 class KineticEnergyRK4(torch.autograd.Function):
@@ -97,9 +103,16 @@ class KineticEnergyRK4(torch.autograd.Function):
         solver.set_params(prm)
         _load_state(solver, U0)
         want_mu = bool(ctx.needs_input_grad[1])
-        _, g, dmu = solver.adjoint_rk4(ctx.dt, ctx.nsteps, ctx.interval, want_mu=want_mu)
         s = gJ.detach().to(torch.float64)
-        gU = torch.from_numpy(g).to(U0.device).view_as(U0) * s.to(U0.device)
+        if U0.is_cuda:
+            gU = torch.empty(U0.shape, dtype=torch.float64, device=U0.device)
+            torch.cuda.current_stream(U0.device).synchronize()
+            _, dmu = solver.adjoint_rk4_device(ctx.dt, ctx.nsteps, gU.data_ptr(), ctx.interval,
+                                               want_mu=want_mu)
+            gU *= s.to(U0.device)
+        else:
+            _, g, dmu = solver.adjoint_rk4(ctx.dt, ctx.nsteps, ctx.interval, want_mu=want_mu)
+            gU = torch.from_numpy(g).view_as(U0) * s.to(U0.device)
         gmu = (torch.tensor(dmu, dtype=torch.float64, device=mu.device) * s.to(mu.device)
                if want_mu else None)
         return gU, gmu, None, None, None, None

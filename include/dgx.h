@@ -283,6 +283,11 @@ dgx_status dgx_kinetic_energy(dgx_ctx* ctx, double* J);
  * residual()'s f = -Minv R (solve.cpp:150-807); w and g in simstate layout. */
 dgx_status dgx_residual_vjp(dgx_ctx* ctx, const double* w_host, double* g_host);
 
+/* Device-pointer form of dgx_residual_vjp: w_dev and g_dev are device buffers
+ * in simstate layout.  Returns after completion.  Like the other adjoint calls
+ * it keeps its workspace on the context (see dgx_adjoint_release). */
+dgx_status dgx_residual_vjp_device(dgx_ctx* ctx, const double* w_dev, double* g_dev);
+
 /* Allocation-free form of dgx_residual_vjp on device buffers (no
  * counterpart in the reference, which has no adjoint): for callers that
  * cannot allocate device memory (code under HIP graph capture, tight
@@ -318,9 +323,15 @@ dgx_status dgx_residual_vjp_device_noalloc(dgx_ctx* ctx, const double* w_dev, do
 dgx_status dgx_adjoint_rk4(dgx_ctx* ctx, double dt, uint64_t nsteps, uint64_t interval,
                            double* J, double* dJdU0_host, double* dJdmu);
 
-/* Frees the stored-stage buffer that dgx_adjoint_rk4 keeps on the context
- * (no counterpart in the reference, which has no adjoint).  No-op when none
- * is held. */
+/* dgx_adjoint_rk4 with the gradient in a device buffer (simstate layout, may
+ * be NULL). */
+dgx_status dgx_adjoint_rk4_device(dgx_ctx* ctx, double dt, uint64_t nsteps, uint64_t interval,
+                                  double* J, double* dJdU0_dev, double* dJdmu);
+
+/* Frees what the adjoint calls keep on the context: the stored-stage buffer
+ * of dgx_adjoint_rk4 and the workspace (3 to 7 states and 2 trace-record sets)
+ * of dgx_adjoint_rk4 and dgx_residual_vjp (no counterpart in the reference,
+ * which has no adjoint).  No-op when none is held. */
 dgx_status dgx_adjoint_release(dgx_ctx* ctx);
 /* Caps the stored-stage buffer of dgx_adjoint_rk4 at `bytes` (0: no cap
  * beyond three quarters of the free device memory; no counterpart in the
