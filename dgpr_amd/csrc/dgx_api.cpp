@@ -54,18 +54,23 @@ int dgx::default_stage_waves(int p, int q)
 
 // Stage kernel and occupancy target of a context, where the caller has not
 // chosen them.  q = 1 in FP64: the state-reading tiled kernel at p = 1 and 3, at
-// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1313
-// against 2166 us per RK4 stage on the 64^3 p = 3 cube, 299 against 437 us on
-// the 64^3 p = 1 cube, 146 against 195 us on a 61x37x43 p = 1 channel.  The
+// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1105
+// against 1930 us per RK4 stage on the 64^3 p = 3 cube, 267 against 442 us on
+// the 64^3 p = 1 cube, 137 against 188 us on a 61x37x43 p = 1 channel.  At p = 2
+// its tile of 7 elements, a lane of which takes as long as three of the one-row
+// kernel's, needs more elements to fill the chip: one-row against tiled, affine:
+// 10120 elements 42.2 / 42.4 us, 15000 59.4 / 63.8, 32768 136 / 107; curved: 7220
+// 45.6 / 50.0, 8400 57.1 / 50.5, 15000 83.8 / 78.9, 20160 106 / 87.  The
 // mixed forms: the record-reading tiled kernel at p = 3, q = 1 (3 waves per
 // SIMD on affine meshes, 2 on curved ones, where 3 spills).  The general-order
 // kernel (tile 2) outside 1 <= p, q <= 3, the one-row kernel elsewhere.
 static void apply_defaults(dgx_ctx* c)
 {
-  const bool fp64 = c->prec == DGX_PREC_FP64;
+  const bool fp64  = c->prec == DGX_PREC_FP64;
+  const bool line2 = c->p == 2 && c->nelem >= (c->affine ? 16384 : 8192);
   if (!c->tile_chosen)
     c->stage_tile = general_order(c->p, c->q) ? 2
-                  : (c->q == 1 && (c->p == 3 || (c->p == 1 && fp64))) ? 1 : 0;
+                  : c->q == 1 && (c->p == 3 || (fp64 && (c->p == 1 || line2))) ? 1 : 0;
   if (!c->waves_chosen)
     c->stage_waves = c->stage_tile != 1 ? default_stage_waves(c->p, c->q)
                                         : (!fp64 && c->p == 3 && c->affine ? 3 : 2);
@@ -646,7 +651,8 @@ static hipError_t launch_step(dgx_ctx* c, int scheme, double dt, bool want_norm,
       if (!fused && (e = norm_partials_dispatch(c->p, c->q, mesh_args(c), f1, c->partial,
                                                 c->stream)) != hipSuccess)
         return e;
-      const int nb = fused ? tile_blocks(c->p, c->nelem) : norm_blocks(c->p, c->q, c->nelem);
+      const int nb = fused ? tile_blocks(c->p, c->nelem, c->prec != DGX_PREC_FP64, c->stage_waves)
+                           : norm_blocks(c->p, c->q, c->nelem);
       e = norm_dev ? norm_dispatch(c->partial, nb, 1.0 / (double)c->nstate, norm_dev, c->stream)
                    : sum_dispatch(c->partial, nb, c->sum, c->stream);
       if (e != hipSuccess)

@@ -776,10 +776,12 @@ hipError_t inviscid_rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph
 #undef CALL_INV
 }
 
-int tile_blocks(int p, int nelem)
+int tile_blocks(int p, int nelem, bool trace32, int waves)
 {
-  const int rows = tile_rows(p);
-  const int e = rows > 0 ? rows * (64 / ((p + 1) * (p + 1) * (p + 1))) : 1;
+  const int n = p + 1;
+  int e = 64 / (n * n);
+  if (trace32 || !line_tiled(p, nelem, waves))
+    e = tile_rows(p) > 0 ? tile_rows(p) * (64 / (n * n * n)) : 1;
   return (nelem + e - 1) / e;
 }
 

@@ -968,10 +968,11 @@ __device__ __forceinline__ void stage_body(const MeshArgs& mesh, const Phys& ph,
 
 #include "dgx_tile.hpp"
 #include "dgx_tile_state.hpp"
+#include "dgx_line_state.hpp"
 
 // The tiled stage kernel: the record-reading body with FP32 records (the
 // mixed forms, where a last-bit change of a trace can flip its rounding: the
-// records keep their arithmetic), the state-reading body in FP64.
+// records keep their arithmetic), a state-reading body in FP64.
 template <int P, int Q, int R, int W, typename TT, bool AFF, int CT = 0, bool NORM = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
 void dgx_tile_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
@@ -984,6 +985,15 @@ void dgx_tile_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* _
     tile_body_lds<P, Q, R, TT, AFF, CT, NORM>(mesh, ph, sa, lam, status, blockIdx.x, lds);
   else
     state_body<P, Q, R, AFF, NORM>(mesh, ph, sa, lam, status, blockIdx.x, lds);
+}
+
+template <int P, int W, bool AFF, bool NORM>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
+void dgx_line_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
+                           int* status)
+{
+  __shared__ __attribute__((aligned(16))) unsigned char lds[LineLds<P, AFF>::bytes];
+  line_body<P, AFF, NORM>(mesh, ph, sa, lam, status, blockIdx.x, lds);
 }
 
 }  // namespace dgx

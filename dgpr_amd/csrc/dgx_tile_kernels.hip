@@ -92,26 +92,37 @@ hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const dou
   return hipErrorInvalidValue;
 }
 
+template <int P, int Q, int W, typename TT, bool AFF, int CT, bool NORM>
+static void launch_tile_w(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
+                          int* status, hipStream_t st)
+{
+  constexpr bool FP64 = sizeof(TT) == sizeof(double);
+  const dim3 grid(tile_blocks(P, m.nelem, !FP64, W));
+  if constexpr (FP64 && line_order(P))
+    if (line_tiled(P, m.nelem, W))
+    {
+      hipLaunchKernelGGL((dgx_line_stage_kernel<P, W, AFF, NORM>), grid, dim3(64), 0, st, m, ph, sa,
+                         lam, status);
+      return;
+    }
+  if constexpr (!FP64 || P != 2)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, tile_rows(P), W, TT, AFF, CT, NORM>), grid,
+                       dim3(64), 0, st, m, ph, sa, lam, status);
+}
+
 template <int P, int Q, typename TT, bool AFF, int CT>
 static hipError_t launch_tile_ct(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
-                          const double* lam, int* status, int waves, hipStream_t st)
+                                 const double* lam, int* status, int waves, hipStream_t st)
 {
-  constexpr int R = tile_rows(P);
-  constexpr int E = TileDims<P, R>::E;
-  int nblk = (m.nelem + E - 1) / E;
   const bool norm = sa.normp != nullptr;
   if (waves == 2 && norm)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT, true>), dim3(nblk),
-                       dim3(64), 0, st, m, ph, sa, lam, status);
+    launch_tile_w<P, Q, 2, TT, AFF, CT, true>(m, ph, sa, lam, status, st);
   else if (waves == 2)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 2, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
-                       st, m, ph, sa, lam, status);
+    launch_tile_w<P, Q, 2, TT, AFF, CT, false>(m, ph, sa, lam, status, st);
   else if (waves == 3 && norm)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT, true>), dim3(nblk),
-                       dim3(64), 0, st, m, ph, sa, lam, status);
+    launch_tile_w<P, Q, 3, TT, AFF, CT, true>(m, ph, sa, lam, status, st);
   else if (waves == 3)
-    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, Q, R, 3, TT, AFF, CT>), dim3(nblk), dim3(64), 0,
-                       st, m, ph, sa, lam, status);
+    launch_tile_w<P, Q, 3, TT, AFF, CT, false>(m, ph, sa, lam, status, st);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

@@ -9,11 +9,12 @@
 // Cache hits mostly: every element is read once as own and six times as a
 // neighbour) leaves the state arrays; the traces of the new state need not be
 // produced, only the states of inflow and outflow boundary faces.  What bounds
-// this kernel is FP64 issue (about 2300 FP64 and 160 matrix instructions per
-// wavefront of 128 nodes).  Per RK4 stage, 64^3 p = 3 cube: 1313 us against
-// 1698 us (traffic 5.1 against 7.5 GB); 64^3 p = 1 cube: 299 us against
-// 369 us (one-row record kernel: 437); per TVD-RK3 stage, 48x24x24 p = 3
-// curved channel: 177 us against 227 us.
+// this kernel is FP64 issue (about 2150 FP64 and 160 matrix instructions per
+// wavefront of 128 nodes).  It runs p = 1 and, below the size where the tiles of
+// dgx_line_state.hpp fill the chip, p = 3.  Per RK4 stage, 64^3 p = 3 cube: 1266 us
+// against 1698 us (traffic 5.1 against 7.5 GB); 64^3 p = 1 cube: 267 us against
+// 369 us (one-row record kernel: 442); 61x37x43 p = 1 curved channel 137 us
+// against 188 us one-row.
 // Included by dgx_stage.hpp inside namespace dgx, after dgx_tile.hpp.
 #pragma once
 
@@ -47,12 +48,12 @@ __device__ __forceinline__ void phase_fence()
 }
 
 // Ends the live ranges of one step of a face subpass before the next begins:
-// what follows reads i (an index) or x only after v[0..2] exist.  Without
-// these ties the two sides' traces, tractions and the face physics are
-// interleaved into one block that needs over 240 registers.
-__device__ __forceinline__ void order_after(double* v, int& i)
+// what follows (a later such tie, or a read of x or y) comes after v[0..2]
+// exist.  Without these ties the two sides' traces, tractions and the face
+// physics are interleaved into one block that needs over 240 registers.
+__device__ __forceinline__ void order_after(double* v)
 {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(i));
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
 }
 __device__ __forceinline__ void order_after(double* v, double& x, double& y)
 {
@@ -150,21 +151,18 @@ __device__ __forceinline__ void line_traces(const double (&x)[5][N], const doubl
   }
 }
 
-// Gradient traction tau(grad u).n of one side of face point (a, b): its trace
-// U with velocity u and reciprocal density ir, normal derivative dn, inverse
-// Jacobian Ji with mc[c] = Ji[c] . n, and the traces of the face's other points
-// in s ([4][64], this face's points from fbase), or at p = 3 (lane = a + 4
-// face + 16 b) on the matrix cores.  The sums of grad_traction, scaled by mu/rho
+// Gradient traction tau(grad u).n of one side of a face point normal to D: its
+// trace U with velocity u and reciprocal density ir, normal derivative dn,
+// tangential derivatives tan(c, r) of variable r along direction c, inverse
+// Jacobian Ji with mc[c] = Ji[c] . n.  The sums of grad_traction, scaled by mu/rho
 // once, one reference direction after the other, so that four derivatives
 // are live at a time instead of twelve.
-template <int P, int D>
-__device__ __forceinline__ void face_traction(const PTab& pt, const MfTabs& mf, const double* s,
-                                              int fbase, int a, int b, const double* U,
-                                              const double* u, double ir, const double* dn,
-                                              const double Ji[3][3], const double* n,
-                                              const double* mc, double mu, double* vg)
+template <int D, typename Tan>
+__device__ __forceinline__ void face_traction(Tan tan, const double* U, const double* u, double ir,
+                                              const double* dn, const double Ji[3][3],
+                                              const double* n, const double* mc, double mu,
+                                              double* vg)
 {
-  constexpr int N = P + 1;
   double A[3] = {0.0, 0.0, 0.0}, tr = 0.0;
 #pragma unroll
   for (int c = 0; c < 3; ++c)
@@ -172,24 +170,7 @@ __device__ __forceinline__ void face_traction(const PTab& pt, const MfTabs& mf, 
     double g[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-    {
-      if (c == D)
-      {
-        g[r] = dn[r];
-        continue;
-      }
-      if constexpr (P == 3)
-      {
-        g[r] = (c == Tang<D>::T1) ? mf_lo(mf.one, mf.dg, U[r], 0.0) : mf_hi(mf.dg, U[r], 0.0);
-        continue;
-      }
-      double d = 0.0;
-#pragma unroll
-      for (int m = 0; m < N; ++m)
-        d += (c == Tang<D>::T1) ? pt.Dg[a][m] * s[r * 64 + fbase + m + N * b]
-                                : pt.Dg[b][m] * s[r * 64 + fbase + a + N * m];
-      g[r] = d;
-    }
+      g[r] = (c == D) ? dn[r] : tan(c, r);
     // rho d u / d xi_c
     const double dv[3] = {g[1] - g[0] * u[0], g[2] - g[0] * u[1], g[3] - g[0] * u[2]};
     const double kc = dv[0] * n[0] + dv[1] * n[1] + dv[2] * n[2];
@@ -199,7 +180,7 @@ __device__ __forceinline__ void face_traction(const PTab& pt, const MfTabs& mf, 
       A[i] += dv[i] * mc[c] + Ji[c][i] * kc;
       tr += dv[i] * Ji[c][i];
     }
-    order_after(A, fbase);
+    order_after(A);
   }
   const double k = mu * ir, t = (2.0 / 3.0) * tr;
 #pragma unroll
@@ -229,6 +210,105 @@ __device__ __forceinline__ double nbr_geo_load(const MeshArgs& mesh, int en, int
   const int lo = (c & 1) * t1 + (c >> 1) * t2;
   const double* X = mesh.nodes + (size_t)en * 24;
   return X[3 * (lo + hi) + d] - X[3 * lo + d];
+}
+
+// Physics of one face point from both sides' traces (UL, Ub) and normal
+// derivatives (dL, dR) with tangential derivatives tanL, tanR: the flux G and
+// the test-function fluxes hc, as face_point_fp64.  X, g, h: geometry of the
+// own element (nodes or record) and of the neighbour (NbrGeo); en, bt: neighbour
+// and boundary code; w: the point's quadrature weight.  next() starts the loads
+// that follow, when the registers of the tractions are free.
+template <int P, int Q, int D, bool AFF, typename TanL, typename TanR, typename Next>
+__device__ __forceinline__ void face_states(const MeshArgs& mesh, const Phys& ph, const QTab& qt,
+                                            const double* __restrict__ Tin, const double* X,
+                                            const double* g, const double* h, int en, int bt,
+                                            int hi, int a, int b, double w, double* UL,
+                                            const double* dL, double* Ub, const double* dR,
+                                            double lamL, double lamR, TanL tanL, TanR tanR,
+                                            Next next, double* G, double (&hc)[3][4])
+{
+  constexpr int N = P + 1, NF = N * N;
+  int gi[3];
+  gi[D]           = 0;
+  gi[Tang<D>::T1] = a;
+  gi[Tang<D>::T2] = b;
+  double J[3][3], JiL[3][3], nv[3], fJ, vgL[3], vgR[3];
+  if constexpr (AFF)
+    fJ = face_geometry<Q, AFF>(qt, X, g, D, hi, gi[0], gi[1], gi[2], JiL, nv);
+  else
+  {
+    double det;
+    geometry_at<Q, false>(qt, X, g, D, hi, gi[0], gi[1], gi[2], J, JiL, det);
+    fJ = face_normal(J, D, hi, nv);
+  }
+  double uL[3], uR[3], mcL[3];
+  const double irL = rcp(UL[0]), irR = rcp(Ub[0]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+  {
+    uL[i]  = UL[1 + i] * irL;
+    uR[i]  = Ub[1 + i] * irR;
+    mcL[i] = JiL[i][0] * nv[0] + JiL[i][1] * nv[1] + JiL[i][2] * nv[2];
+  }
+  face_traction<D>(tanL, UL, uL, irL, dL, JiL, nv, mcL, ph.mu, vgL);
+  order_after(vgL);
+  {
+    double JiR[3][3];
+    if constexpr (AFF)
+    {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          JiR[i][j] = h[3 * i + j];
+    }
+    else
+    {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        J[i][D] = 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+      {
+        const double s = qt.Bq[a][c & 1] * qt.Bq[b][c >> 1];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          J[i][D] += s * h[3 * c + i];
+      }
+      inv3(J, det3(J), JiR);
+    }
+    double mcR[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      mcR[i] = JiR[i][0] * nv[0] + JiR[i][1] * nv[1] + JiR[i][2] * nv[2];
+    face_traction<D>(tanR, Ub, uR, irR, dR, JiR, nv, mcR, ph.mu, vgR);
+  }
+  order_after(vgR, UL[0], Ub[0]);
+  next();
+  double irB = irR;
+  if (en < 0)
+  {
+    if (characteristic_bc(bt))
+    {
+      // written with Vin
+      const double* B =
+          Tin + (size_t)mesh.nelem * 6 * 8 * NF + (size_t)(-1 - en) * 5 * NF + a + N * b;
+#pragma unroll
+      for (int r = 0; r < 5; ++r)
+        Ub[r] = B[r * NF];
+    }
+    else
+      wall_state(bt, UL, nv, ph, Ub);
+    irB = rcp(Ub[0]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+      uR[i]  = Ub[1 + i] * irB;
+      vgR[i] = 0.0;
+    }
+  }
+  face_point_fp64(en >= 0, UL, uL, irL, Ub, uR, irB, vgL, vgR, nv, JiL, mcL, lamL, lamR, fJ * w,
+                  ph, G, hc);
 }
 
 // This lane's face point in subpass S of a tile (S = NSUB D + the subpass of
@@ -330,92 +410,22 @@ __device__ __forceinline__ void state_face_subpass(
   }
   double G[5], hn[4], hc[3][4];
   {
-    int gi[3];
-    gi[D]  = 0;
-    gi[T1] = a;
-    gi[T2] = b;
-    double J[3][3], JiL[3][3], nv[3], fJ, vgL[3], vgR[3];
-    if constexpr (AFF)
-      fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], D, hi, gi[0], gi[1], gi[2], JiL, nv);
-    else
-    {
-      double det;
-      geometry_at<Q, false>(qt, sX[l], sG[l], D, hi, gi[0], gi[1], gi[2], J, JiL, det);
-      fJ = face_normal(J, D, hi, nv);
-    }
-    double uL[3], uR[3], mcL[3];
-    const double irL = rcp(UL[0]), irR = rcp(Ub[0]);
+    auto tan = [&](const double* U, const double* s, int c, int r) __attribute__((always_inline)) {
+      if constexpr (P == 3)
+        return (c == T1) ? mf_lo(mf.one, mf.dg, U[r], 0.0) : mf_hi(mf.dg, U[r], 0.0);
+      double d = 0.0;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-    {
-      uL[i]  = UL[1 + i] * irL;
-      uR[i]  = Ub[1 + i] * irR;
-      mcL[i] = JiL[i][0] * nv[0] + JiL[i][1] * nv[1] + JiL[i][2] * nv[2];
-    }
-    face_traction<P, D>(pt, mf, sR, fbase, a, b, UL, uL, irL, dL, JiL, nv, mcL, ph.mu, vgL);
-    int fbR = fbase;
-    order_after(vgL, fbR);
-    {
-      double JiR[3][3];
-      const double* h = sH[6 * l + f];
-      if constexpr (AFF)
-      {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int j = 0; j < 3; ++j)
-            JiR[i][j] = h[3 * i + j];
-      }
-      else
-      {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          J[i][D] = 0.0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-        {
-          const double w = qt.Bq[a][c & 1] * qt.Bq[b][c >> 1];
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            J[i][D] += w * h[3 * c + i];
-        }
-        inv3(J, det3(J), JiR);
-      }
-      double mcR[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        mcR[i] = JiR[i][0] * nv[0] + JiR[i][1] * nv[1] + JiR[i][2] * nv[2];
-      face_traction<P, D>(pt, mf, sR + 4 * 64, fbR, a, b, Ub, uR, irR, dR, JiR, nv, mcR, ph.mu,
-                          vgR);
-    }
-    order_after(vgR, UL[0], Ub[0]);
-    next();
-    double irB = irR;
-    if (en < 0)
-    {
-      const int bt = sBt[l][f];
-      if (characteristic_bc(bt))
-      {
-        // written with Vin
-        const double* B =
-            Tin + (size_t)mesh.nelem * 6 * 8 * NF + (size_t)(-1 - en) * 5 * NF + a + N * b;
-#pragma unroll
-        for (int r = 0; r < 5; ++r)
-          Ub[r] = B[r * NF];
-      }
-      else
-        wall_state(bt, UL, nv, ph, Ub);
-      irB = rcp(Ub[0]);
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-      {
-        uR[i]  = Ub[1 + i] * irB;
-        vgR[i] = 0.0;
-      }
-    }
-    const double sc = fJ * pt.w[a] * pt.w[b];
-    face_point_fp64(en >= 0, UL, uL, irL, Ub, uR, irB, vgL, vgR, nv, JiL, mcL, lamL, lamR, sc, ph,
-                    G, hc);
+      for (int m = 0; m < N; ++m)
+        d += (c == T1) ? pt.Dg[a][m] * s[r * 64 + fbase + m + N * b]
+                       : pt.Dg[b][m] * s[r * 64 + fbase + a + N * m];
+      return d;
+    };
+    face_states<P, Q, D, AFF>(
+        mesh, ph, qt, Tin, sX[l], sG[l], sH[6 * l + f], en, sBt[l][f], hi, a, b,
+        pt.w[a] * pt.w[b], UL, dL, Ub, dR, lamL, lamR,
+        [&](int c, int r) __attribute__((always_inline)) { return tan(UL, sR, c, r); },
+        [&](int c, int r) __attribute__((always_inline)) { return tan(Ub, sR + 4 * 64, c, r); },
+        next, G, hc);
   }
   // T = G - Dg^T(t1) h_t1 - Dg^T(t2) h_t2 (the mass row has no viscous part)
 #pragma unroll
@@ -815,13 +825,7 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
   subpass(Const<0>{});
   subpass(Const<1>{});
   subpass(Const<2>{});
-  if constexpr (TD::NSUB == 2)
-  {
-    subpass(Const<3>{});
-    subpass(Const<4>{});
-    subpass(Const<5>{});
-  }
-  static_assert(TD::NSUB <= 2, "subpasses per direction");
+  static_assert(TD::NSUB == 1, "one subpass per direction");
 
   // ---- form f_g and the RK epilogue, one row at a time; with NORM, each
   // row's R = -B3^T W f_g in sR (three passes) and the lane's running sum of
