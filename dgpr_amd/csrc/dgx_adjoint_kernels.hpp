@@ -65,7 +65,7 @@ void dgx_adj_main_kernel(MeshArgs mesh, Phys ph, const double* __restrict__ V,
   if (vact)
   {
     double J[3][3], det;
-    geometry_at<Q, AFF>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
+    geometry_at<Q, AFF, true>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
     wJ = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]] * det;
     const double iwJ = rcp(wJ);
 #pragma unroll
@@ -261,7 +261,7 @@ void dgx_adj_main_kernel(MeshArgs mesh, Phys ph, const double* __restrict__ V,
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
       double J[3][3], JiL[3][3], detL;
-      geometry_at<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, J, JiL, detL);
+      geometry_at<Q, AFF, true>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, J, JiL, detL);
       double nv[3];
       const double fJ = face_normal(J, nd, hi, nv);
       const double lamL = lam[((size_t)ee * 6 + f) * NF + fpt];
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(64) void dgx_adj_boundary_kernel(MeshArgs mesh, Phy
   const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
   const int gi2 = (nd == 2) ? 0 : b;
   double J[3][3];
-  jac_at<Q>(c_qtab[P - 1][Q - 1], mesh.nodes + (size_t)e * NG * 3, nd, hi, gi0, gi1, gi2, J);
+  jac_at<Q, true>(c_qtab[P - 1][Q - 1], mesh.nodes + (size_t)e * NG * 3, nd, hi, gi0, gi1, gi2, J);
   double nv[3];
   face_normal(J, nd, hi, nv);
   const double* To = Tin + ((size_t)e * 6 + f) * 8 * NF + fpt;
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(64) void dgx_adj_trace_kernel(MeshArgs mesh, Phys p
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
       double J[3][3], Ji[3][3], det;
-      geometry_at<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, J, Ji, det);
+      geometry_at<Q, AFF, true>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, J, Ji, det);
       double nv[3];
       face_normal(J, nd, hi, nv);
       double gr[3][4];
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(64) void dgx_kinetic_energy_kernel(MeshArgs mesh,
   {
     const int i = nd0 % N, j = (nd0 / N) % N, kk = nd0 / (N * N);
     double J[3][3];
-    jac_at<Q>(qt, mesh.nodes + (size_t)e * NG * 3, -1, 0, i, j, kk, J);
+    jac_at<Q, true>(qt, mesh.nodes + (size_t)e * NG * 3, -1, 0, i, j, kk, J);
     const double wJ = pt.w[i] * pt.w[j] * pt.w[kk] * det3(J);
     double s[5];
 #pragma unroll

@@ -193,6 +193,46 @@ __device__ __forceinline__ void form_now(double (&acc)[N][5])
       asm volatile("" : "+v"(acc[k][r]));
 }
 
+// J = d x / d xi along the lane's line of nodes of a trilinear element: the z
+// column is constant on it and the others are linear in z.
+struct LineGeo
+{
+  double x0[3], dx[3], y0[3], dy[3], z[3];
+  __device__ __forceinline__ LineGeo(const double* X, double ga, double gb)
+  {
+    const double fa = 1.0 - ga, fb = 1.0 - gb;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+      double n[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        n[c] = X[3 * c + i];
+      x0[i] = fb * (n[1] - n[0]) + gb * (n[3] - n[2]);
+      y0[i] = fa * (n[2] - n[0]) + ga * (n[3] - n[1]);
+      dx[i] = fb * (n[5] - n[4]) + gb * (n[7] - n[6]) - x0[i];
+      dy[i] = fa * (n[6] - n[4]) + ga * (n[7] - n[5]) - y0[i];
+      z[i]  = fb * (fa * (n[4] - n[0]) + ga * (n[5] - n[1])) +
+             gb * (fa * (n[6] - n[2]) + ga * (n[7] - n[3]));
+    }
+  }
+  __device__ __forceinline__ void at(double g, double J[3][3]) const
+  {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+      J[i][0] = x0[i] + g * dx[i];
+      J[i][1] = y0[i] + g * dy[i];
+      J[i][2] = z[i];
+    }
+  }
+};
+
+struct AffineLine
+{
+  __device__ __forceinline__ AffineLine(const double*, double, double) {}
+};
+
 // Subpass S: local face S of every element of the tile: both sides' traces and
 // gradient tractions from the states (own from LDS, neighbour in fd), the face
 // point physics, the tangential (T) phase and the gather into the nodes'
@@ -207,7 +247,7 @@ __device__ __forceinline__ void line_face_subpass(
     double (&acc)[P + 1][5], FaceData<P>& fd, Next next)
 {
   using LD = LineDims<P>;
-  constexpr int N = LD::N, NF = LD::NF, JS = LD::JS, D = S >> 1, hi = S & 1, f = S;
+  constexpr int N = LD::N, JS = LD::JS, D = S >> 1, hi = S & 1, f = S;
   constexpr int T1 = Tang<D>::T1, T2 = Tang<D>::T2;
   const LineLane<P> ln(mesh, e0);
   const int tid = ln.tid, a = ln.a, b = ln.b, l = ln.l;
@@ -374,7 +414,7 @@ __device__ __forceinline__ void line_state_traces(const MeshArgs& mesh, const Ph
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
       double Ji[3][3], nv[3];
-      face_geometry<1, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
+      face_geometry<1, AFF, true>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
       if (records)
       {
         double gr[3][4];
@@ -508,13 +548,23 @@ __device__ __forceinline__ void line_body(const MeshArgs& mesh, const Phys& ph, 
 #pragma unroll
     for (int r = 0; r < 5; ++r)
       acc[k][r] = 0.0;
+  std::conditional_t<AFF, AffineLine, LineGeo> geo(sX[l], qt.Bq[a][1], qt.Bq[b][1]);
+  const QTab& cq = c_qtab[P - 1][0];
   // volume, one z row at a time: velocity gradient, flux, divergence
 #pragma unroll
   for (int k = 0; k < N; ++k)
   {
-    double J[3][3], Ji[3][3], det, H[3][5], gr[3][4], Fo[2][5];
-    geometry_at<1, AFF>(qt, sX[l], sG[l], -1, 0, a, b, k, J, Ji, det);
-    wJ[k] = wab * ct.w[k] * det;
+    double F[3][5], gr[3][4];
+    NodeGeo ng;
+    if constexpr (AFF)
+      ng.inverse(sG[l] + 10, wab * ct.w[k] * sG[l][9], ph.mu);
+    else
+    {
+      double J[3][3];
+      geo.at(cq.Bq[k][1], J);
+      ng.curved(J, wab * ct.w[k], ph.mu);
+    }
+    wJ[k] = ng.wJ;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
     {
@@ -534,32 +584,28 @@ __device__ __forceinline__ void line_body(const MeshArgs& mesh, const Phys& ph, 
         g2 += ct.Dg[k][m] * v[m][r];
       gr[2][r] = g2;
     }
-    volume_flux(v[k], gr, Ji, ph.gamma, ph.mu, H);
+    volume_flux_fp64(v[k], gr, ng.B, ng.kv, ng.A, ph.gamma, F);
 #pragma unroll
     for (int r = 0; r < 5; ++r)
     {
-      double F[3];
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-        F[c] = wJ[k] * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
       if constexpr (P == 3)
-        acc[k][r] = mf_hi(mf.dgt, F[1], mf_lo(mf.one, mf.dgt, F[0], acc[k][r]));
+        acc[k][r] = mf_hi(mf.dgt, F[1][r], mf_lo(mf.one, mf.dgt, F[0][r], acc[k][r]));
       else
       {
-        sR[r * 64 + tid]       = Fo[0][r] = F[0];
-        sR[(5 + r) * 64 + tid] = Fo[1][r] = F[1];
+        sR[r * 64 + tid]       = F[0][r];
+        sR[(5 + r) * 64 + tid] = F[1][r];
       }
 #pragma unroll
       for (int m = 0; m < N; ++m)
-        acc[m][r] += ct.Dg[k][m] * F[2];
+        acc[m][r] += ct.Dg[k][m] * F[2][r];
     }
     if constexpr (P != 3)
     {
       phase_fence();
 #pragma unroll
       for (int r = 0; r < 5; ++r)
-        acc[k][r] = row_sum(lt.tb, lt.nb, sR + (5 + r) * 64, Fo[1][r],
-                            row_sum(lt.ta, lt.na, sR + r * 64, Fo[0][r], acc[k][r]));
+        acc[k][r] = row_sum(lt.tb, lt.nb, sR + (5 + r) * 64, F[1][r],
+                            row_sum(lt.ta, lt.na, sR + r * 64, F[0][r], acc[k][r]));
     }
     form_now<N>(acc);
     phase_fence();

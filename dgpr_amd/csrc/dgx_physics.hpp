@@ -179,6 +179,9 @@ __device__ __forceinline__ void face_point_physics(bool interior, const T* UL, c
 //   hc[c][r] sc Ji[c] . dcQ, the contravariant dual-consistency flux, whose
 //            stress tau(a (x) n) gives  mu ((Ji[c].a) n + mc a - 2/3 (a.n) Ji[c])
 //            with a = s dmL, without forming the stress.
+// D >= 0: the face is known to be normal to reference direction D, whose
+// Ji[D] = mc[D] n (the row itself is not read).
+template <int D = -1>
 __device__ __forceinline__ void face_point_fp64(bool interior, const double* UL, const double* uL,
                                                 double irL, const double* Ub, const double* uB,
                                                 double irB, const double* vgL, const double* vgR,
@@ -231,10 +234,20 @@ __device__ __forceinline__ void face_point_fp64(bool interior, const double* UL,
 #pragma unroll
   for (int c = 0; c < 3; ++c)
   {
-    const double k = Ji[c][0] * a[0] + Ji[c][1] * a[1] + Ji[c][2] * a[2];
+    if (c == D)
+    {
+      const double k = (1.0 / 3.0) * al * dnL;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      hc[c][i] = k * n[i] + mc[c] * a[i] - t * Ji[c][i];
+      for (int i = 0; i < 3; ++i)
+        hc[c][i] = mc[c] * (a[i] + k * n[i]);
+    }
+    else
+    {
+      const double k = Ji[c][0] * a[0] + Ji[c][1] * a[1] + Ji[c][2] * a[2];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        hc[c][i] = k * n[i] + mc[c] * a[i] - t * Ji[c][i];
+    }
     hc[c][3] = uL[0] * hc[c][0] + uL[1] * hc[c][1] + uL[2] * hc[c][2];
   }
 }
@@ -316,6 +329,101 @@ __device__ __forceinline__ void volume_flux(const T* Vq, const G gr[3][4], const
         H[d][1 + i] -= p;
     }
     H[d][4] = u[0] * tau[0] + u[1] * tau[1] + u[2] * tau[2] - md * Ht;
+  }
+}
+
+// Geometry of a Gauss node for volume_flux_fp64, from J^-1 and w det J or from J
+// (w: the node's quadrature weight).
+struct NodeGeo
+{
+  double B[3][3], A[3][3], kv, wJ;
+  __device__ __forceinline__ void inverse(const double* Ji, double wdet, double mu)
+  {
+    wJ = wdet;
+    kv = mu;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+      {
+        B[c][d] = Ji[3 * c + d];
+        A[c][d] = wJ * B[c][d];
+      }
+  }
+  __device__ __forceinline__ void curved(const double J[3][3], double w, double mu)
+  {
+    // rows of det J Ji: cross products of the columns of J
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+      {
+        const int c1 = (c + 1) % 3, c2 = (c + 2) % 3, d1 = (d + 1) % 3, d2 = (d + 2) % 3;
+        B[c][d] = J[d1][c1] * J[d2][c2] - J[d2][c1] * J[d1][c2];
+        A[c][d] = w * B[c][d];
+      }
+    const double det = J[0][0] * B[0][0] + J[1][0] * B[0][1] + J[2][0] * B[0][2];
+    wJ = w * det;
+    kv = mu * rcp(det);
+  }
+};
+
+// Contravariant volume flux F[c] = A[c] . H (H of volume_flux) of the FP64
+// state-reading kernels: A[c] = w det J Ji[c], and the gradient is formed with
+// rows B = Ji (kv = mu) or the adjugate det J Ji (kv = mu / det J):
+//   A.(tau - u m - p) = S A - (A.m) u  with  S = tau - p I,  and the energy row
+//   u.(S A) - (E/rho) (A.m)
+// (VISC false: the inviscid part, tau = 0, gr and B not read),
+// 130 operations where H, then A H, take 175 (64^3 p = 3 cube 1161 -> 1150 us per
+// RK4 stage with the factor n of Ji[D] taken out in face_traction and
+// face_point_fp64: 3 % fewer FP64 operations).
+template <bool VISC = true>
+__device__ __forceinline__ void volume_flux_fp64(const double* Vq, const double gr[3][4],
+                                                 const double B[3][3], double kv,
+                                                 const double A[3][3], double gamma,
+                                                 double F[3][5])
+{
+  const double ir = rcp(Vq[0]);
+  const double u[3] = {Vq[1] * ir, Vq[2] * ir, Vq[3] * ir};
+  const double p = (gamma - 1.0) *
+                   (Vq[4] - 0.5 * (Vq[1] * u[0] + Vq[2] * u[1] + Vq[3] * u[2]));
+  double S[6] = {-p, -p, -p, 0.0, 0.0, 0.0};
+  if constexpr (VISC)
+  {
+    double L[3][3];  // rho d u_i / d x_d
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+      {
+        const double dv = gr[c][1 + i] - gr[c][0] * u[i];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          L[d][i] = (c == 0) ? B[c][d] * dv : L[d][i] + B[c][d] * dv;
+      }
+    const double k = kv * ir, k2 = 2.0 * k;
+    const double t = -(2.0 / 3.0) * k * (L[0][0] + L[1][1] + L[2][2]) - p;
+    S[0] = k2 * L[0][0] + t;
+    S[1] = k2 * L[1][1] + t;
+    S[2] = k2 * L[2][2] + t;
+    S[3] = k * (L[0][1] + L[1][0]);
+    S[4] = k * (L[0][2] + L[2][0]);
+    S[5] = k * (L[1][2] + L[2][1]);
+  }
+  const double e = Vq[4] * ir;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+  {
+    const double* a = A[c];
+    const double m  = a[0] * Vq[1] + a[1] * Vq[2] + a[2] * Vq[3];
+    const double s0 = VISC ? S[0] * a[0] + S[3] * a[1] + S[4] * a[2] : S[0] * a[0];
+    const double s1 = VISC ? S[3] * a[0] + S[1] * a[1] + S[5] * a[2] : S[1] * a[1];
+    const double s2 = VISC ? S[4] * a[0] + S[5] * a[1] + S[2] * a[2] : S[2] * a[2];
+    F[c][0] = -m;
+    F[c][1] = s0 - m * u[0];
+    F[c][2] = s1 - m * u[1];
+    F[c][3] = s2 - m * u[2];
+    F[c][4] = u[0] * s0 + u[1] * s1 + u[2] * s2 - m * e;
   }
 }
 

@@ -31,6 +31,7 @@
 // neighbour's gradient.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 #include "dgx_physics.hpp"
@@ -126,6 +127,33 @@ __device__ __forceinline__ void inv3(const double J[3][3], double det, double Ji
   Ji[2][2] = id * (J[0][0] * J[1][1] - J[0][1] * J[1][0]);
 }
 
+// jacobian of a trilinear element (q = 1, d* = -1 and 1) from the edge vectors:
+// 84 operations instead of 96, and the rounding of the edges instead of the
+// coordinates.  The FP64 kernels use it (DIFF below); the mixed forms keep the
+// sums (a last-bit change can flip the rounding of an FP32 record).
+__device__ __forceinline__ void jacobian_diff(const double* X, const double* vx, const double* vy,
+                                              const double* vz, double J[3][3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    J[d][0] = J[d][1] = J[d][2] = 0.0;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+    {
+      const double w0 = vy[a] * vz[b], w1 = vx[a] * vz[b], w2 = vx[a] * vy[b];
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+      {
+        const double* x = X + d;
+        J[d][0] += w0 * (x[3 * (2 * a + 4 * b + 1)] - x[3 * (2 * a + 4 * b)]);
+        J[d][1] += w1 * (x[3 * (a + 4 * b + 2)] - x[3 * (a + 4 * b)]);
+        J[d][2] += w2 * (x[3 * (a + 2 * b + 4)] - x[3 * (a + 2 * b)]);
+      }
+    }
+}
+
 // Geometry-basis 1D values for the three directions of a volume node (i,j,k)
 // or a face point (end e on direction nd, Gauss indices elsewhere).
 __device__ __forceinline__ void geo_vals(const QTab& qt, int nd, int e, int i, int j, int k,
@@ -148,14 +176,17 @@ __device__ __forceinline__ void geo_vals(const QTab& qt, int nd, int e, int i, i
   }
 }
 
-template <int Q>
+template <int Q, bool DIFF = false>
 __device__ __forceinline__ void jac_at(const QTab& qt, const double* X, int nd, int e, int i,
                                        int j, int k, double J[3][3])
 {
   const double* v[3];
   const double* d[3];
   geo_vals(qt, nd, e, i, j, k, v, d);
-  jacobian<Q>(X, v[0], d[0], v[1], d[1], v[2], d[2], J);
+  if constexpr (DIFF && Q == 1)
+    jacobian_diff(X, v[0], v[1], v[2], J);
+  else
+    jacobian<Q>(X, v[0], d[0], v[1], d[1], v[2], d[2], J);
 }
 
 
@@ -232,7 +263,7 @@ __device__ __forceinline__ void affine_record(const double* __restrict__ nodes, 
 // J, J^-1 and det J at a point: from the affine record in the affine
 // instantiation (AFF, q = 1 only), else from the geometry basis.  The two
 // are separate kernels: the general one is unchanged by the affine path.
-template <int Q, bool AFF>
+template <int Q, bool AFF, bool DIFF = false>
 __device__ __forceinline__ void geometry_at(const QTab& qt, const double* X, const double* g,
                                             int nd, int e, int i, int j, int k, double J[3][3],
                                             double Ji[3][3], double& det)
@@ -250,7 +281,7 @@ __device__ __forceinline__ void geometry_at(const QTab& qt, const double* X, con
     det = g[9];
     return;
   }
-  jac_at<Q>(qt, X, nd, e, i, j, k, J);
+  jac_at<Q, DIFF>(qt, X, nd, e, i, j, k, J);
   det = det3(J);
   inv3(J, det, Ji);
 }
@@ -259,7 +290,7 @@ __device__ __forceinline__ void geometry_at(const QTab& qt, const double* X, con
 // local face (nd, hi): from the affine record in the affine instantiation
 // (the face_normal of the element's constant J, bitwise), else from the
 // geometry basis at the point.
-template <int Q, bool AFF>
+template <int Q, bool AFF, bool DIFF = false>
 __device__ __forceinline__ double face_geometry(const QTab& qt, const double* X, const double* g,
                                                 int nd, int hi, int i, int j, int k,
                                                 double Ji[3][3], double* nv)
@@ -279,7 +310,7 @@ __device__ __forceinline__ double face_geometry(const QTab& qt, const double* X,
     return n[3];
   }
   double J[3][3], det;
-  geometry_at<Q, false>(qt, X, g, nd, hi, i, j, k, J, Ji, det);
+  geometry_at<Q, false, DIFF>(qt, X, g, nd, hi, i, j, k, J, Ji, det);
   return face_normal(J, nd, hi, nv);
 }
 
@@ -459,6 +490,7 @@ __device__ __forceinline__ void produce_traces(const MeshArgs& mesh, const Phys&
                                                int* status)
 {
   using FD = FaceDims<P>;
+  constexpr bool FP64 = sizeof(TT) == sizeof(double);
   constexpr int N = FD::N, NF = FD::NF;
   TT* Tb = Tout + (size_t)mesh.nelem * 6 * 8 * NF;
   const int tid = threadIdx.x;
@@ -508,7 +540,7 @@ __device__ __forceinline__ void produce_traces(const MeshArgs& mesh, const Phys&
       if constexpr (STO)
         stored_face_geometry<NF>(mesh, ee, f, fpt, Ji, nv);
       else
-        face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
+        face_geometry<Q, AFF, FP64>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
       double gr[3][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -631,7 +663,7 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
   constexpr int NG = (Q + 1) * (Q + 1) * (Q + 1);
   // the short form of the face physics; where the q > 1 kernel evaluates the
   // geometry basis and spills, it measured 1-5 % slower
-  constexpr bool FAST = (Q == 1 || STO) && sizeof(TT) == sizeof(double);
+  constexpr bool FP64 = sizeof(TT) == sizeof(double), FAST = (Q == 1 || STO) && FP64;
 
   auto sV  = reinterpret_cast<double(*)[5][NB]>(lds + SL::oV);
   auto sX  = reinterpret_cast<double(*)[NG * 3]>(lds + SL::oX);      // own geometry nodes
@@ -669,24 +701,45 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
   double wJ = 1.0;
   double acc[5] = {0, 0, 0, 0, 0};
   double Ji[3][3];
-  double H[3][5];  // physical flux Q - F at this node
+  // physical flux Q - F at this node; CONTRA: its contravariant form
+  constexpr bool CONTRA = FAST;
+  double H[3][5];
 
   // ---- volume: velocity gradient, fluxes ----
   if (vact)
   {
+    NodeGeo ng;
     if constexpr (STO)
+    {
       wJ = stored_volume_geometry<NB>(mesh, e, nd0, Ji);
+      ng.inverse(&Ji[0][0], wJ, ph.mu);
+    }
+    else if constexpr (CONTRA)
+    {
+      const double w = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]];
+      if constexpr (AFF)
+        ng.inverse(sG[le] + 10, w * sG[le][9], ph.mu);
+      else
+      {
+        double J[3][3];
+        jac_at<Q, true>(qt, sX[le], -1, 0, idx[0], idx[1], idx[2], J);
+        ng.curved(J, w, ph.mu);
+      }
+      wJ = ng.wJ;
+    }
     else
     {
       double J[3][3], det;
-      geometry_at<Q, AFF>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
+      geometry_at<Q, AFF, FP64>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
       wJ = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]] * det;
     }
     double Vq[5];
 #pragma unroll
     for (int r = 0; r < 5; ++r)
       Vq[r] = sV[le][r][nd0];
-    if constexpr (INV)
+    if constexpr (INV && CONTRA)
+      volume_flux_fp64<false>(Vq, nullptr, ng.B, 0.0, ng.A, ph.gamma, H);
+    else if constexpr (INV)
       euler_volume_flux(Vq, ph.gamma, H);
     else
     {
@@ -706,7 +759,10 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
         gr[1][r] = g1;
         gr[2][r] = g2;
       }
-      volume_flux(Vq, gr, Ji, ph.gamma, ph.mu, H);
+      if constexpr (CONTRA)
+        volume_flux_fp64(Vq, gr, ng.B, ng.kv, ng.A, ph.gamma, H);
+      else
+        volume_flux(Vq, gr, Ji, ph.gamma, ph.mu, H);
     }
   }
 
@@ -718,7 +774,9 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
     {
 #pragma unroll
       for (int r = 0; r < 5; ++r)
-        sR[(le * 5 + r) * NB + nd0] = wJ * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
+        sR[(le * 5 + r) * NB + nd0] =
+            CONTRA ? H[c][r]
+                   : wJ * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
     }
     __syncthreads();
     if (vact)
@@ -784,7 +842,7 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       if constexpr (STO)
         fJ = stored_face_geometry<NF>(mesh, ee, f, fpt, JiL, nv);
       else
-        fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
+        fJ = face_geometry<Q, AFF, FP64>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
       if (en >= 0 && FAST)
         roe_flux_fp64(UL, Ub, nv, ph.gamma, fpo.G);
       else if (en >= 0)
@@ -822,7 +880,7 @@ __device__ __forceinline__ void stage_body_lds(const MeshArgs& mesh, const Phys&
       if constexpr (STO)
         fJ = stored_face_geometry<NF>(mesh, ee, f, fpt, JiL, nv);
       else
-        fJ = face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
+        fJ = face_geometry<Q, AFF, FP64>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, JiL, nv);
       // affine meshes: the face's constant coefficient
       const double lamL =
           AFF ? mesh.lamf[(size_t)ee * 6 + f] : lam[((size_t)ee * 6 + f) * NF + fpt];

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64) void dgx_boundary_kernel(MeshArgs mesh, Phys ph
   const int gi0 = (nd == 0) ? 0 : a;
   const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
   const int gi2 = (nd == 2) ? 0 : b;
-  face_geometry<1, AFF>(c_qtab[P - 1][0], mesh.nodes + e * 24, AFF ? mesh.arec + e * GREC : nullptr,
+  face_geometry<1, AFF, true>(c_qtab[P - 1][0], mesh.nodes + e * 24, AFF ? mesh.arec + e * GREC : nullptr,
                         nd, hi, gi0, gi1, gi2, Ji, nv);
   if (!boundary_state(bt, U, nv, ph, Ub))
     atomicOr(status, 1);

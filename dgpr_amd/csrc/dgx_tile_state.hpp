@@ -154,9 +154,9 @@ __device__ __forceinline__ void line_traces(const double (&x)[5][N], const doubl
 // Gradient traction tau(grad u).n of one side of a face point normal to D: its
 // trace U with velocity u and reciprocal density ir, normal derivative dn,
 // tangential derivatives tan(c, r) of variable r along direction c, inverse
-// Jacobian Ji with mc[c] = Ji[c] . n.  The sums of grad_traction, scaled by mu/rho
-// once, one reference direction after the other, so that four derivatives
-// are live at a time instead of twelve.
+// Jacobian Ji with mc[c] = Ji[c] . n (Ji[D] = mc[D] n is not read).  The sums of
+// grad_traction, scaled by mu/rho once, one reference direction after the other,
+// so that four derivatives are live at a time instead of twelve.
 template <int D, typename Tan>
 __device__ __forceinline__ void face_traction(Tan tan, const double* U, const double* u, double ir,
                                               const double* dn, const double Ji[3][3],
@@ -174,11 +174,22 @@ __device__ __forceinline__ void face_traction(Tan tan, const double* U, const do
     // rho d u / d xi_c
     const double dv[3] = {g[1] - g[0] * u[0], g[2] - g[0] * u[1], g[3] - g[0] * u[2]};
     const double kc = dv[0] * n[0] + dv[1] * n[1] + dv[2] * n[2];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
+    if (c == D)
     {
-      A[i] += dv[i] * mc[c] + Ji[c][i] * kc;
-      tr += dv[i] * Ji[c][i];
+      const double k = mc[c] * kc;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        A[i] += dv[i] * mc[c] + k * n[i];
+      tr += k;
+    }
+    else
+    {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+      {
+        A[i] += dv[i] * mc[c] + Ji[c][i] * kc;
+        tr += dv[i] * Ji[c][i];
+      }
     }
     order_after(A);
   }
@@ -186,6 +197,30 @@ __device__ __forceinline__ void face_traction(Tan tan, const double* U, const do
 #pragma unroll
   for (int i = 0; i < 3; ++i)
     vg[i] = k * (A[i] - t * n[i]);
+}
+
+// The two tangential rows of J^-1 and mc[c] = Ji[c] . n (see face_traction) at a
+// face point normal to D, from the normal column of J, the tangential ones t1
+// and t2 (t1, t2 = columns D+1 and D+2, cyclic), the normal n and sg = +-1 / |t1 x t2|:
+// det J = (J_D . n) / sg, so that Ji[D] = n / (J_D . n).
+template <int D>
+__device__ __forceinline__ void face_inverse(const double* jd, const double* t1, const double* t2,
+                                             const double* n, double sg, double Ji[3][3],
+                                             double* mc)
+{
+  constexpr int c1 = (D + 1) % 3, c2 = (D + 2) % 3;
+  mc[D] = rcp(jd[0] * n[0] + jd[1] * n[1] + jd[2] * n[2]);
+  const double id = mc[D] * sg;
+  const double b[3] = {id * jd[0], id * jd[1], id * jd[2]};
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+  {
+    const int j = (i + 1) % 3, k = (i + 2) % 3;
+    Ji[c1][i] = t2[j] * b[k] - t2[k] * b[j];
+    Ji[c2][i] = b[j] * t1[k] - b[k] * t1[j];
+  }
+  mc[c1] = Ji[c1][0] * n[0] + Ji[c1][1] * n[1] + Ji[c1][2] * n[2];
+  mc[c2] = Ji[c2][0] * n[0] + Ji[c2][1] * n[1] + Ji[c2][2] * n[2];
 }
 
 // Geometry a tile keeps per element face about the element across it: on
@@ -212,6 +247,37 @@ __device__ __forceinline__ double nbr_geo_load(const MeshArgs& mesh, int en, int
   return X[3 * (lo + hi) + d] - X[3 * lo + d];
 }
 
+// The columns of J = d x / d xi at point (a, b) of face (D, hi) of a trilinear
+// element with nodes X (x fastest): j[c], with ga and gb the point's coordinates
+// along the face, and the bilinear weights w4 of the face's corners.  The face's
+// columns follow from its own four nodes and the normal one from the four
+// edges that leave it: 52 operations, half of the sums over 8 nodes of the
+// general form (jac_at).  With face_inverse and LineGeo, per stage: 48x24x24 p = 3
+// channel 157 -> 138 us (TVD-RK3), 61x37x43 p = 1 139 -> 133, 30x24x28 p = 2 88 -> 83 (RK4).
+template <int D>
+__device__ __forceinline__ void trilinear_face(const double* X, int hi, double ga, double gb,
+                                               double (&w4)[4], double j[3][3])
+{
+  constexpr int T1 = Tang<D>::T1, T2 = Tang<D>::T2, s1 = 3 << T1, s2 = 3 << T2, sn = 3 << D;
+  const double fa = 1.0 - ga, fb = 1.0 - gb;
+  w4[0] = fa * fb;
+  w4[1] = ga * fb;
+  w4[2] = fa * gb;
+  w4[3] = ga * gb;
+  const double* F = X + hi * sn;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+  {
+    const double a0 = F[s1 + i] - F[i], a1 = F[s1 + s2 + i] - F[s2 + i];
+    const double b0 = F[s2 + i] - F[i], b1 = F[s1 + s2 + i] - F[s1 + i];
+    j[T1][i] = fb * a0 + gb * a1;
+    j[T2][i] = fa * b0 + ga * b1;
+    j[D][i]  = w4[0] * (X[sn + i] - X[i]) + w4[1] * (X[sn + s1 + i] - X[s1 + i]) +
+              w4[2] * (X[sn + s2 + i] - X[s2 + i]) +
+              w4[3] * (X[sn + s1 + s2 + i] - X[s1 + s2 + i]);
+  }
+}
+
 // Physics of one face point from both sides' traces (UL, Ub) and normal
 // derivatives (dL, dR) with tangential derivatives tanL, tanR: the flux G and
 // the test-function fluxes hc, as face_point_fp64.  X, g, h: geometry of the
@@ -228,59 +294,63 @@ __device__ __forceinline__ void face_states(const MeshArgs& mesh, const Phys& ph
                                             Next next, double* G, double (&hc)[3][4])
 {
   constexpr int N = P + 1, NF = N * N;
-  int gi[3];
-  gi[D]           = 0;
-  gi[Tang<D>::T1] = a;
-  gi[Tang<D>::T2] = b;
-  double J[3][3], JiL[3][3], nv[3], fJ, vgL[3], vgR[3];
+  double j[3][3], w4[4];                // curved: columns of the own J, corner weights
+  double JiL[3][3], nv[3], mcL[3], fJ, sg = 0.0;
   if constexpr (AFF)
-    fJ = face_geometry<Q, AFF>(qt, X, g, D, hi, gi[0], gi[1], gi[2], JiL, nv);
+  {
+    fJ = face_geometry<Q, AFF>(qt, X, g, D, hi, 0, 0, 0, JiL, nv);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      mcL[i] = JiL[i][0] * nv[0] + JiL[i][1] * nv[1] + JiL[i][2] * nv[2];
+  }
   else
   {
-    double det;
-    geometry_at<Q, false>(qt, X, g, D, hi, gi[0], gi[1], gi[2], J, JiL, det);
-    fJ = face_normal(J, D, hi, nv);
+    trilinear_face<D>(X, hi, qt.Bq[a][1], qt.Bq[b][1], w4, j);
+    const double *t1 = j[(D + 1) % 3], *t2 = j[(D + 2) % 3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      nv[i] = t1[(i + 1) % 3] * t2[(i + 2) % 3] - t1[(i + 2) % 3] * t2[(i + 1) % 3];
+    const double n2 = nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2], r = rsq(n2);
+    fJ = n2 * r;
+    sg = hi ? r : -r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      nv[i] *= sg;
+    face_inverse<D>(j[D], t1, t2, nv, sg, JiL, mcL);
   }
-  double uL[3], uR[3], mcL[3];
+  double uL[3], uR[3], vgL[3], vgR[3];
   const double irL = rcp(UL[0]), irR = rcp(Ub[0]);
 #pragma unroll
   for (int i = 0; i < 3; ++i)
   {
-    uL[i]  = UL[1 + i] * irL;
-    uR[i]  = Ub[1 + i] * irR;
-    mcL[i] = JiL[i][0] * nv[0] + JiL[i][1] * nv[1] + JiL[i][2] * nv[2];
+    uL[i] = UL[1 + i] * irL;
+    uR[i] = Ub[1 + i] * irR;
   }
   face_traction<D>(tanL, UL, uL, irL, dL, JiL, nv, mcL, ph.mu, vgL);
   order_after(vgL);
   {
-    double JiR[3][3];
+    double JiR[3][3], mcR[3];
     if constexpr (AFF)
     {
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+      for (int c = 0; c < 3; ++c)
+      {
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          JiR[i][j] = h[3 * i + j];
+        for (int i = 0; i < 3; ++i)
+          JiR[c][i] = h[3 * c + i];
+        mcR[c] = JiR[c][0] * nv[0] + JiR[c][1] * nv[1] + JiR[c][2] * nv[2];
+      }
     }
     else
     {
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        J[i][D] = 0.0;
+      double jd[3] = {0.0, 0.0, 0.0};
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-      {
-        const double s = qt.Bq[a][c & 1] * qt.Bq[b][c >> 1];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-          J[i][D] += s * h[3 * c + i];
-      }
-      inv3(J, det3(J), JiR);
+          jd[i] += w4[c] * h[3 * c + i];
+      face_inverse<D>(jd, j[(D + 1) % 3], j[(D + 2) % 3], nv, sg, JiR, mcR);
     }
-    double mcR[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      mcR[i] = JiR[i][0] * nv[0] + JiR[i][1] * nv[1] + JiR[i][2] * nv[2];
     face_traction<D>(tanR, Ub, uR, irR, dR, JiR, nv, mcR, ph.mu, vgR);
   }
   order_after(vgR, UL[0], Ub[0]);
@@ -307,7 +377,7 @@ __device__ __forceinline__ void face_states(const MeshArgs& mesh, const Phys& ph
       vgR[i] = 0.0;
     }
   }
-  face_point_fp64(en >= 0, UL, uL, irL, Ub, uR, irB, vgL, vgR, nv, JiL, mcL, lamL, lamR, fJ * w,
+  face_point_fp64<D>(en >= 0, UL, uL, irL, Ub, uR, irB, vgL, vgR, nv, JiL, mcL, lamL, lamR, fJ * w,
                   ph, G, hc);
 }
 
@@ -556,7 +626,7 @@ __device__ __forceinline__ void state_traces(const MeshArgs& mesh, const Phys& p
       const int gi1 = (nd == 1) ? 0 : ((nd == 0) ? a : b);
       const int gi2 = (nd == 2) ? 0 : b;
       double Ji[3][3], nv[3];
-      face_geometry<Q, AFF>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
+      face_geometry<Q, AFF, true>(qt, sX[l], sG[l], nd, hi, gi0, gi1, gi2, Ji, nv);
       if (records)
       {
         double gr[3][4];
@@ -706,13 +776,20 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
     for (int r = 0; r < 5; ++r)
       acc[rr][r] = 0.0;
     wJ[rr] = 1.0;
-    double Ji[3][3];
-    double H[3][5];
+    double F[3][5];
     if (P == 3 || vact)
     {
-      double J[3][3], det;
-      geometry_at<Q, AFF>(qt, sX[le], sG[le], -1, 0, idx[0], idx[1], idx[2], J, Ji, det);
-      wJ[rr] = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]] * det;
+      NodeGeo ng;
+      const double w = pt.w[idx[0]] * pt.w[idx[1]] * pt.w[idx[2]];
+      if constexpr (AFF)
+        ng.inverse(sG[le] + 10, w * sG[le][9], ph.mu);
+      else
+      {
+        double J[3][3];
+        jac_at<Q, true>(qt, sX[le], -1, 0, idx[0], idx[1], idx[2], J);
+        ng.curved(J, w, ph.mu);
+      }
+      wJ[rr] = ng.wJ;
       double Vq[5], gr[3][4];
 #pragma unroll
       for (int r = 0; r < 5; ++r)
@@ -740,7 +817,7 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
         gr[1][r] = g1;
         gr[2][r] = g2;
       }
-      volume_flux(Vq, gr, Ji, ph.gamma, ph.mu, H);
+      volume_flux_fp64(Vq, gr, ng.B, ng.kv, ng.A, ph.gamma, F);
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -749,19 +826,15 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
       {
 #pragma unroll
         for (int r = 0; r < 5; ++r)
-        {
-          const double F =
-              wJ[rr] * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
-          acc[rr][r] = (c == 0) ? mf_lo(mf.one, mf.dgt, F, acc[rr][r]) : mf_hi(mf.dgt, F, acc[rr][r]);
-        }
+          acc[rr][r] = (c == 0) ? mf_lo(mf.one, mf.dgt, F[c][r], acc[rr][r])
+                                : mf_hi(mf.dgt, F[c][r], acc[rr][r]);
         continue;
       }
       if (P == 3 || vact)
       {
 #pragma unroll
         for (int r = 0; r < 5; ++r)
-          sR[r * 64 + tid] =
-              wJ[rr] * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
+          sR[r * 64 + tid] = F[c][r];
       }
       phase_fence();
       if (P == 3 || vact)
