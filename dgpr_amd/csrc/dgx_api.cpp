@@ -76,6 +76,12 @@ static void apply_defaults(dgx_ctx* c)
                                         : (!fp64 && c->p == 3 && c->affine ? 3 : 2);
 }
 
+// the mixed forms convert states with the arithmetic their records were rounded from
+static bool mixed_basis(const dgx_ctx* c)
+{
+  return c->prec != DGX_PREC_FP64;
+}
+
 static void derive_phys(const dgx_params& p, Phys& ph)
 {
   // total conditions of the reference state (solve.cpp:167-175)
@@ -433,7 +439,7 @@ dgx_status dgx_set_state_device(dgx_ctx* c, const double* U_dev)
 {
   if (!c || !U_dev)
     return DGX_ERR_INVALID;
-  HIPCHK(c, basis_dispatch(c->p, U_dev, c->U, c->nelem, 0, c->stream));
+  HIPCHK(c, basis_dispatch(c->p, U_dev, c->U, c->nelem, 0, c->stream, mixed_basis(c)));
   drop_traces(c);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return DGX_OK;
@@ -454,7 +460,7 @@ dgx_status dgx_set_state(dgx_ctx* c, const double* U_host)
     return DGX_ERR_INVALID;
   HIPCHK(c, hipMemcpyAsync(c->Ua, U_host, c->nstate * sizeof(double), hipMemcpyHostToDevice,
                            c->stream));
-  HIPCHK(c, basis_dispatch(c->p, c->Ua, c->U, c->nelem, 0, c->stream));
+  HIPCHK(c, basis_dispatch(c->p, c->Ua, c->U, c->nelem, 0, c->stream, mixed_basis(c)));
   drop_traces(c);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return DGX_OK;
@@ -545,7 +551,7 @@ dgx_status dgx_residual_device(dgx_ctx* c, const double* U_dev, double* R_dev, d
 {
   if (!c || !U_dev || !f_dev)
     return DGX_ERR_INVALID;
-  HIPCHK(c, basis_dispatch(c->p, U_dev, c->Ua, c->nelem, 0, c->stream));
+  HIPCHK(c, basis_dispatch(c->p, U_dev, c->Ua, c->nelem, 0, c->stream, mixed_basis(c)));
   const bool t32 = c->prec != DGX_PREC_FP64;
   if (reads_states(c))
     HIPCHK(c, boundary_dispatch(c->p, mesh_args(c), c->phys, c->Ua, c->TUa, c->status, c->stream));

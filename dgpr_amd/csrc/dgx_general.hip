@@ -717,7 +717,9 @@ __device__ __forceinline__ void gen_apply_dir(double (*s)[N * N * N], const doub
 
 // Basis conversions of one element per workgroup (modes as dgx_basis_kernel:
 // 0 V = B3 U, 1 U = B3^-1 V, 2 G = B3^T g, 3 g = B3^-T G), in double-double.
-template <int P>
+// MIX: by dd_fma.  The coefficients in LDS: 20^3 p = 5 116 -> 86 us, 19x13x17
+// p = 4 35 -> 27 us against lane-dependent loads from the tables.
+template <int P, bool MIX>
 __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const double* in, double* out,
                                                                     int mode)
 {
@@ -725,21 +727,21 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
   const GenTab& t = g_gtab[P * 8];
   __shared__ double sh[5][NB];
   __shared__ double sl[5][NB];
+  __shared__ DD sM[N][N];  // coefficient of input m in output i: [m][i]
   const int node = threadIdx.x;
   const size_t e = blockIdx.x;
   const bool act = node < NB;
+  const bool inv = (mode == 1 || mode == 3);
+  for (int x = node; x < N * N; x += GDims<P>::BT)
+  {
+    const int m = x / N, i = x % N, u = (mode >= 2) ? m : i, v = (mode >= 2) ? i : m;
+    sM[m][i] = inv ? DD{t.Binv[u][v], t.Binvlo[u][v]} : DD{t.B[u][v], t.Blo[u][v]};
+  }
   if (act)
 #pragma unroll
     for (int r = 0; r < 5; ++r)
-    {
       sh[r][node] = in[(e * 5 + r) * NB + node];
-      sl[r][node] = 0.0;
-    }
   __syncthreads();
-  const bool inv = (mode == 1 || mode == 3);
-  const double(*M)[GMAXN]  = inv ? t.Binv : t.B;
-  const double(*Ml)[GMAXN] = inv ? t.Binvlo : t.Blo;
-  const bool tr = (mode >= 2);
   const int i0 = node % N, i1 = (node / N) % N, i2 = node / (N * N);
 #pragma unroll
   for (int d = 0; d < 3; ++d)
@@ -748,20 +750,27 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
     if (act)
     {
       const int id = pick3i(d, i0, i1, i2);
+      const int b0 = (d == 0) ? nid<N>(0, i1, i2) : ((d == 1) ? nid<N>(i0, 0, i2) : nid<N>(i0, i1, 0));
+      constexpr int st[3] = {1, N, N * N};
+      auto c = [&](int m) { return sM[m][id]; };
 #pragma unroll
       for (int r = 0; r < 5; ++r)
-      {
-        DD acc = {0.0, 0.0};
-#pragma unroll
-        for (int m = 0; m < N; ++m)
+        if constexpr (MIX)
         {
-          const int src = (d == 0) ? nid<N>(m, i1, i2) : ((d == 1) ? nid<N>(i0, m, i2) : nid<N>(i0, i1, m));
-          const double c  = tr ? M[m][id] : M[id][m];
-          const double cl = tr ? Ml[m][id] : Ml[id][m];
-          acc = dd_fma({sh[r][src], sl[r][src]}, c, cl, acc);
+          o[r] = {0.0, 0.0};
+#pragma unroll
+          for (int m = 0; m < N; ++m)
+          {
+            const DD k = c(m);
+            o[r] = dd_fma({sh[r][b0 + m * st[d]], d == 0 ? 0.0 : sl[r][b0 + m * st[d]]}, k.hi, k.lo,
+                          o[r]);
+          }
         }
-        o[r] = acc;
-      }
+        else if (d == 0)
+          o[r] = dd_dot<N, false>([&](int m) { return DD{sh[r][b0 + m], 0.0}; }, c);
+        else
+          o[r] = dd_dot<N, true>(
+              [&](int m) { return DD{sh[r][b0 + m * st[d]], sl[r][b0 + m * st[d]]}; }, c);
     }
     __syncthreads();
     if (act)
@@ -782,7 +791,9 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
 // From f_g of the epb elements from blockIdx.x * epb: f = B3^-1 f_g,
 // R = -B3^T W f_g (either may be null) and, with partial,
 // partial[blockIdx.x] = sum of R^2 over those elements (waves summed in a
-// fixed order: deterministic).
+// fixed order: deterministic).  The tables in LDS and w det J from the element's
+// record or the stored geometry, as in the stage: the norm of a 20^3 p = 5 cube
+// 78 -> 48 us, of a 19x13x17 p = 4 q = 2 channel 37 -> 16 us.
 template <int P>
 __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_resid_out_kernel(MeshArgs mesh,
                                                                         const double* fg,
@@ -792,21 +803,17 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_resid_out_kernel(MeshArg
 {
   using D = GDims<P>;
   constexpr int N = D::N, NB = D::NB, BT = D::BT, EPB = D::EPB;
-  const GenTab& t = g_gtab[P * 8 + q - 1];
   __shared__ double s[EPB][5][NB];
   __shared__ double red[BT / 64];
-  extern __shared__ double sX[];  // [epb][(q+1)^3 * 3]
-  const int tid = threadIdx.x, nq = q + 1, n3 = nq * nq * nq * 3;
+  __shared__ GenTab t;
+  extern __shared__ double sX[];  // [epb][(q+1)^3 * 3], [epb][GREC] or nothing
+  const int tid = threadIdx.x, nq = q + 1;
   const int e0 = blockIdx.x * epb;
   const int le = tid / NB, node = tid % NB;
   const size_t e = (size_t)e0 + le;
   const bool act = le < epb && e < (size_t)mesh.nelem;
   double (*se)[NB] = s[act ? le : 0];
-  for (int x = tid; x < epb * n3; x += BT)
-  {
-    const int l = x / n3;
-    sX[x] = (e0 + l < mesh.nelem) ? mesh.nodes[(size_t)(e0 + l) * n3 + (x - l * n3)] : 0.0;
-  }
+  gen_load_tables_nodes<P>(mesh, q, e0, epb, &t, sX);
   double fgv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (act)
 #pragma unroll
@@ -833,9 +840,8 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_resid_out_kernel(MeshArg
     const int i0 = node % N, i1 = (node / N) % N, i2 = node / (N * N);
     if (act)
     {
-      double J[3][3];
-      gen_jac_at(t, sX + le * n3, nq, -1, 0, i0, i1, i2, J);
-      const double wJ = t.w[i0] * t.w[i1] * t.w[i2] * det3(J);
+      double Ji[3][3], wJ;
+      gen_volume_geometry<NB>(mesh, t, sX, nq, e, le, node, i0, i1, i2, Ji, wJ);
 #pragma unroll
       for (int r = 0; r < 5; ++r)
         se[r][node] = -wJ * fgv[r];
@@ -1058,9 +1064,10 @@ template <int P>
 static hipError_t launch_gen_resid_out(int q, const MeshArgs& m, const double* fg, double* f,
                                        double* R, double* partial, hipStream_t st)
 {
+  // (the number of blocks sizes the partial sums: see resid_out_blocks)
   const int epb = gen_epb_of(GDims<P>::EPB, q);
   hipLaunchKernelGGL((dgx_gen_resid_out_kernel<P>), dim3((m.nelem + epb - 1) / epb),
-                     dim3(GDims<P>::BT), gen_node_lds(q, epb), st, m, fg, f, R, partial, q, epb);
+                     dim3(GDims<P>::BT), gen_geo_lds(m, q, epb), st, m, fg, f, R, partial, q, epb);
   return hipGetLastError();
 }
 
@@ -1075,20 +1082,24 @@ hipError_t gen_resid_out_dispatch(int p, int q, const MeshArgs& m, const double*
 }
 
 template <int P>
-static hipError_t launch_gen_basis(const double* in, double* out, int nelem, int mode,
+static hipError_t launch_gen_basis(const double* in, double* out, int nelem, int mode, bool mix,
                                    hipStream_t st)
 {
-  hipLaunchKernelGGL((dgx_gen_basis_kernel<P>), dim3(nelem), dim3(GDims<P>::BT), 0, st, in, out,
-                     mode);
+  if (mix)
+    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, true>), dim3(nelem), dim3(GDims<P>::BT), 0, st, in,
+                       out, mode);
+  else
+    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, false>), dim3(nelem), dim3(GDims<P>::BT), 0, st, in,
+                       out, mode);
   return hipGetLastError();
 }
 
-hipError_t gen_basis_dispatch(int p, const double* in, double* out, int nelem, int mode,
+hipError_t gen_basis_dispatch(int p, const double* in, double* out, int nelem, int mode, bool mix,
                               hipStream_t st)
 {
   if (nelem < 1 || mode < 0 || mode > 3)
     return hipErrorInvalidValue;
-#define CALL_GB(P) launch_gen_basis<P>(in, out, nelem, mode, st)
+#define CALL_GB(P) launch_gen_basis<P>(in, out, nelem, mode, mix, st)
   DGX_GEN_DISPATCH_P(p, CALL_GB)
 #undef CALL_GB
 }

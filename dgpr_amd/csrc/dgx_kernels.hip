@@ -186,67 +186,81 @@ __device__ __forceinline__ void apply_dir(double (*s)[5][NB], const double (*M)[
 // mode 1: U = B3^-1 V   (Gauss-nodal -> reference basis)
 // mode 2: G = B3^T g    (a gradient with respect to V -> with respect to U)
 // mode 3: g = B3^-T G   (a gradient with respect to U -> with respect to V)
+// A lane has a line of nodes along z (elements and lanes as LineLane): that
+// direction is done first, in registers and with x.lo = 0; the other two go
+// through LDS.  What bounds it is FP64 issue: 64^3 p = 3 cube (1.3 GB moved) 580 ->
+// 360 us against one node per lane, all directions through LDS and dd_fma.
 template <int P>
 __global__ __launch_bounds__(64) void dgx_basis_kernel(const double* in, double* out, int nelem,
                                                        int mode)
 {
-  constexpr int N = P + 1, NB = N * N * N, EPW = 64 / NB;
+  constexpr int N = P + 1, NF = N * N, NB = N * NF, E = 64 / NF;
   const PTab& pt = c_ptab[P - 1];
-  __shared__ double sh[EPW][5][NB];
-  __shared__ double sl[EPW][5][NB];
-  int tid = threadIdx.x, le = tid / NB, node = tid % NB;
-  int e = blockIdx.x * EPW + le;
-  bool act = le < EPW && e < nelem;
-  if (act)
-#pragma unroll
-    for (int r = 0; r < 5; ++r)
-    {
-      sh[le][r][node] = in[((size_t)e * 5 + r) * NB + node];
-      sl[le][r][node] = 0.0;
-    }
-  __syncthreads();
-  const bool inv = (mode == 1 || mode == 3);
-  const double(*M)[MAXN]  = inv ? pt.Binv : pt.B;
-  const double(*Ml)[MAXN] = inv ? pt.Binvlo : pt.Blo;
-  const bool tr = (mode >= 2);
-  int idx[3] = {node % N, (node / N) % N, node / (N * N)};
-#pragma unroll
-  for (int d = 0; d < 3; ++d)
+  __shared__ DD sM[N][N];           // coefficient of input m in output i: [m][i]
+  __shared__ double sh[5][64], sl[5][64];
+  const int tid = threadIdx.x;
   {
-    DD o[5];
-    if (act)
+    const bool inv = (mode == 1 || mode == 3);
+    const double(*M)[MAXN]  = inv ? pt.Binv : pt.B;
+    const double(*Ml)[MAXN] = inv ? pt.Binvlo : pt.Blo;
+    if (tid < NF)
     {
-#pragma unroll
-      for (int r = 0; r < 5; ++r)
-      {
-        DD acc = {0.0, 0.0};
-#pragma unroll
-        for (int m = 0; m < N; ++m)
-        {
-          int id2[3] = {idx[0], idx[1], idx[2]};
-          id2[d] = m;
-          int src = (id2[2] * N + id2[1]) * N + id2[0];
-          const double c  = tr ? M[m][idx[d]] : M[idx[d]][m];
-          const double cl = tr ? Ml[m][idx[d]] : Ml[idx[d]][m];
-          acc = dd_fma({sh[le][r][src], sl[le][r][src]}, c, cl, acc);
-        }
-        o[r] = acc;
-      }
+      const int m = tid / N, i = tid % N;
+      sM[m][i] = (mode >= 2) ? DD{M[m][i], Ml[m][i]} : DD{M[i][m], Ml[i][m]};
     }
-    __syncthreads();
-    if (act)
-#pragma unroll
-      for (int r = 0; r < 5; ++r)
-      {
-        sh[le][r][node] = o[r].hi;
-        sl[le][r][node] = o[r].lo;
-      }
-    __syncthreads();
   }
-  if (act)
+  const int t = min(tid, E * NF - 1), l = t / NF, a = t % N, b = (t / N) % N;
+  const int e = min((int)blockIdx.x * E + l, nelem - 1);
+  const bool act = tid < E * NF && (int)blockIdx.x * E + l < nelem;
+  const size_t base = (size_t)e * 5 * NB + b * N + a;
+  double x[N][5];
+#pragma unroll
+  for (int r = 0; r < 5; ++r)
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      x[k][r] = in[base + r * NB + k * NF];
+  __syncthreads();
+  DD ca[N], cb[N];
+#pragma unroll
+  for (int m = 0; m < N; ++m)
+  {
+    ca[m] = sM[m][a];
+    cb[m] = sM[m][b];
+  }
+  const int ba = l * NF + b * N, bb = l * NF + a;
+#pragma unroll 1
+  for (int k = 0; k < N; ++k)
+  {
+    DD z[5];
 #pragma unroll
     for (int r = 0; r < 5; ++r)
-      out[((size_t)e * 5 + r) * NB + node] = sh[le][r][node] + sl[le][r][node];
+      z[r] = dd_dot<N, false>([&](int m) { return DD{x[m][r], 0.0}; },
+                              [&](int m) { return sM[m][k]; });
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+    {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 5; ++r)
+      {
+        sh[r][tid] = z[r].hi;
+        sl[r][tid] = z[r].lo;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 5; ++r)
+        z[r] = dd_dot<N, true>(
+            [&](int m) {
+              const int s = d == 0 ? ba + m : bb + m * N;
+              return DD{sh[r][s], sl[r][s]};
+            },
+            [&](int m) { return d == 0 ? ca[m] : cb[m]; });
+    }
+    if (act)
+#pragma unroll
+      for (int r = 0; r < 5; ++r)
+        out[base + r * NB + k * NF] = z[r].hi + z[r].lo;
+  }
 }
 
 // From f_g (Gauss-nodal): f = B3^-1 f_g, R = -M f = -B3^T W f_g.  Either
@@ -358,7 +372,9 @@ __global__ __launch_bounds__(256) void dgx_norm_kernel(MeshArgs mesh, const doub
     for (int x = tid; x < (int)(sizeof(QTab) / 8); x += 256)
       d[x] = c[x];
   }
-  for (int x = tid; x < EPB * NG * 3; x += 256)
+  // uniform: w detJ read instead of formed (30x14x11 p = 2 q = 2: 9.3 -> 5.6 us)
+  const bool stored = Q > 1 && mesh.geov;
+  for (int x = tid; x < (stored ? 0 : EPB * NG * 3); x += 256)
   {
     const int l = x / (NG * 3), ee = e0 + l;
     sX[l][x % (NG * 3)] = (ee < mesh.nelem) ? mesh.nodes[(size_t)ee * NG * 3 + x % (NG * 3)] : 0.0;
@@ -372,9 +388,18 @@ __global__ __launch_bounds__(256) void dgx_norm_kernel(MeshArgs mesh, const doub
   const int ni = node % N, nj = (node / N) % N, nk = node / (N * N);
   if (act)
   {
-    double J[3][3];
-    jac_at<Q>(sQT, sX[le], -1, 0, ni, nj, nk, J);
-    const double wJ = sPT.w[ni] * sPT.w[nj] * sPT.w[nk] * det3(J);
+    double wJ;
+    if (stored)
+    {
+      double Ji[3][3];
+      wJ = stored_volume_geometry<NB>(mesh, e, node, Ji);
+    }
+    else
+    {
+      double J[3][3];
+      jac_at<Q>(sQT, sX[le], -1, 0, ni, nj, nk, J);
+      wJ = sPT.w[ni] * sPT.w[nj] * sPT.w[nk] * det3(J);
+    }
 #pragma unroll
     for (int r = 0; r < 5; ++r)
       s[le][r][node] = -wJ * fgv[r];
@@ -661,8 +686,8 @@ hipError_t launch_lift_coef(const MeshArgs& m, double* lam, hipStream_t st)
 template <int P>
 hipError_t launch_basis(const double* in, double* out, int nelem, int mode, hipStream_t st)
 {
-  constexpr int EPW = 64 / ((P + 1) * (P + 1) * (P + 1));
-  int nblk = (nelem + EPW - 1) / EPW;
+  constexpr int E = 64 / ((P + 1) * (P + 1));
+  int nblk = (nelem + E - 1) / E;
   hipLaunchKernelGGL((dgx_basis_kernel<P>), dim3(nblk), dim3(64), 0, st, in, out, nelem, mode);
   return hipGetLastError();
 }
@@ -910,15 +935,18 @@ hipError_t resid_out_dispatch(int p, int q, const MeshArgs& m, const double* fg,
 }
 
 hipError_t basis_dispatch(int p, const double* in, double* out, int nelem, int mode,
-                          hipStream_t st)
+                          hipStream_t st, bool mix)
 {
-  switch (p)
+  // lines of nodes from one wavefront per SIMD; below that a node per lane is
+  // quicker (2574 elements p = 3: 9.7 against 14.4 us, 512 p = 2: 5.2 against 7.1)
+  const bool lines = !mix && (long)nelem * (p + 1) * (p + 1) >= 64 * 1024;
+  switch (lines ? p : 0)
   {
     case 1: return launch_basis<1>(in, out, nelem, mode, st);
     case 2: return launch_basis<2>(in, out, nelem, mode, st);
     case 3: return launch_basis<3>(in, out, nelem, mode, st);
   }
-  return gen_basis_dispatch(p, in, out, nelem, mode, st);
+  return gen_basis_dispatch(p, in, out, nelem, mode, mix, st);
 }
 
 hipError_t sample_dispatch(int p, const double* V, int nelem, int Ns, int var, double gamma,

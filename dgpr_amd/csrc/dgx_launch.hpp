@@ -195,8 +195,9 @@ hipError_t lift_coef_dispatch(int p, int q, const MeshArgs& m, double* lam, hipS
 hipError_t lift_face_dispatch(int p, const double* lam, int nelem, double* lamf, hipStream_t st);
 hipError_t resid_out_dispatch(int p, int q, const MeshArgs& m, const double* fg, double* f,
                               double* R, double* partial, hipStream_t st);
+// mix: the conversion of the mixed forms (dd_fma)
 hipError_t basis_dispatch(int p, const double* in, double* out, int nelem, int mode,
-                          hipStream_t st);
+                          hipStream_t st, bool mix = false);
 // Sums of n per-workgroup partials (deterministic order).  Above
 // SUM_ONE_BLOCK partials the sum runs in two launches (chunks of SUM_CHUNK,
 // then the chunk sums): the partial buffer then holds sum_scratch(n) more
@@ -263,7 +264,7 @@ hipError_t gen_lift_coef_dispatch(int p, int q, const MeshArgs& m, double* lam, 
 hipError_t gen_resid_out_dispatch(int p, int q, const MeshArgs& m, const double* fg, double* f,
                                   double* R, double* partial, hipStream_t st);
 hipError_t gen_basis_dispatch(int p, const double* in, double* out, int nelem, int mode,
-                              hipStream_t st);
+                              bool mix, hipStream_t st);
 hipError_t gen_sample_dispatch(int p, const double* V, int nelem, int Ns, int var, double gamma,
                                double* out, hipStream_t st);
 
