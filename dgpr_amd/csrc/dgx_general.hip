@@ -404,6 +404,8 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_stage_kernel(MeshArgs me
   double wJ = 1.0;
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   double Ji[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+  // physical flux at the node; CONTRA: its contravariant form
+  constexpr bool CONTRA = sizeof(TT) == sizeof(double);
   double H[3][5];
   if (vact)
   {
@@ -428,7 +430,14 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_stage_kernel(MeshArgs me
       gr[1][r] = g1;
       gr[2][r] = g2;
     }
-    volume_flux(Vq, gr, Ji, ph.gamma, ph.mu, H);
+    if constexpr (CONTRA)
+    {
+      NodeGeo ng;
+      ng.inverse(&Ji[0][0], wJ, ph.mu);
+      volume_flux_fp64(Vq, gr, ng.B, ng.kv, ng.A, ph.gamma, H);
+    }
+    else
+      volume_flux(Vq, gr, Ji, ph.gamma, ph.mu, H);
   }
 
   // ---- volume divergence, one reference direction at a time ----
@@ -439,7 +448,8 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_stage_kernel(MeshArgs me
 #pragma unroll
       for (int r = 0; r < 5; ++r)
         sR[(le * 5 + r) * NB + nd0] =
-            wJ * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
+            CONTRA ? H[c][r]
+                   : wJ * (Ji[c][0] * H[0][r] + Ji[c][1] * H[1][r] + Ji[c][2] * H[2][r]);
     __syncthreads();
     if (vact)
     {

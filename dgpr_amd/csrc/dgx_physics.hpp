@@ -376,7 +376,8 @@ struct NodeGeo
 // (VISC false: the inviscid part, tau = 0, gr and B not read),
 // 130 operations where H, then A H, take 175 (64^3 p = 3 cube 1161 -> 1150 us per
 // RK4 stage with the factor n of Ji[D] taken out in face_traction and
-// face_point_fp64: 3 % fewer FP64 operations).
+// face_point_fp64: 3 % fewer FP64 operations; general-order kernel 20^3 p = 5 223.6 ->
+// 220.5 us).
 template <bool VISC = true>
 __device__ __forceinline__ void volume_flux_fp64(const double* Vq, const double gr[3][4],
                                                  const double B[3][3], double kv,
