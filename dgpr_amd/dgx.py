@@ -548,7 +548,8 @@ class Solver:
                          "Roe, inverse mass, RK in FP64",
     }
 
-    # rows per tile of the tiled stage kernel at p = 1, 2, 3
+    # rows per tile of the tiled stage kernel of the mixed forms, and of the FP64
+    # one at p = 1 and (below 12288 elements or at 3 waves) p = 3
     TILE_ROWS = {1: 1, 2: 3, 3: 2}
 
     def stage_kernel_name(self, waves=None, tile=None):
@@ -558,6 +559,9 @@ class Solver:
         t = self.tile if tile is None else tile
         if t == 2:
             return "dgx_gen_stage_kernel<%d,double>" % self.mesh.p
+        p, fp64 = self.mesh.p, self.precision == "fp64"
+        if t and fp64 and (p == 2 or (p == 3 and w == 2 and self.mesh.nelem >= 12288)):
+            return "dgx_line_stage_kernel<%d,%d>" % (p, w)
         if t:
             return "dgx_tile_stage_kernel<%d,%d,%d,%d>" % (self.mesh.p, self.mesh.q,
                                                            self.TILE_ROWS[self.mesh.p], w)

@@ -250,8 +250,8 @@ dgx_status dgx_ensemble_get_stream(dgx_ensemble* ens, void** stream);
 /* For each layout (1, 2, 0) times every launch group at each occupancy
  * target and, for the ensemble stage kernel,
  * each tile (one-row units: 64/(p+1)^3 elements per workgroup, one node per
- * lane; tiled units: 2, 6 or 8 elements per workgroup at p = 3, 2, 1, up to
- * 3 nodes per lane), with reps launches of the first stage (which writes
+ * lane; tiled units: 4, 7 or 8 elements per workgroup at p = 3, 2, 1, up to
+ * 4 nodes per lane), with reps launches of the first stage (which writes
  * stage buffers only), keeps the fastest per group, then keeps the layout
  * whose first stage over all members is fastest (a later
  * dgx_ensemble_set_layout overrides it).  Writes each member's
@@ -394,10 +394,11 @@ dgx_status dgx_autotune(dgx_ctx* ctx, int reps, int* chosen, double us_out[3]);
 /* Stage tile: 0 runs the stage kernel that maps one row of whole elements
  * (one element at p = 3, 2 at p = 2, 8 at p = 1) to a wavefront and mixes
  * the faces of all directions in each face pass; 1 runs the tiled kernel:
- * several rows per wavefront (2 at p = 3, 3 at p = 2, 1 at p = 1), each lane
- * owning one node per row, faces processed one reference direction at a
- * time in whole-face subpasses (compiled for q = 1 meshes at 2 and 3 waves
- * per SIMD; selecting it moves a target of 1 to 2; DGX_ERR_UNSUPPORTED for
+ * several elements per wavefront (FP64: 2, or on large meshes 4, at p = 3, 7
+ * at p = 2, 8 at p = 1; FP32 records: 2, 6, 8), one or more nodes per lane,
+ * faces processed one reference direction at a time in whole-face subpasses,
+ * in FP64 from the states instead of trace records (compiled for q = 1 meshes
+ * at 2 and 3 waves per SIMD; selecting it moves a target of 1 to 2; DGX_ERR_UNSUPPORTED for
  * q > 1); 2 runs the general-order kernel (one element, or several at
  * p <= 2, per workgroup, one Gauss node per lane; every order, and the only tile outside 1 <= p, q <= 3,
  * where 0 and 1 return DGX_ERR_UNSUPPORTED; occupancy targets do not apply).
