@@ -54,7 +54,7 @@ int dgx::default_stage_waves(int p, int q)
 
 // Stage kernel and occupancy target of a context, where the caller has not
 // chosen them.  q = 1 in FP64: the state-reading tiled kernel at p = 1 and 3, at
-// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1105
+// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1083
 // against 1930 us per RK4 stage on the 64^3 p = 3 cube, 267 against 442 us on
 // the 64^3 p = 1 cube, 137 against 188 us on a 61x37x43 p = 1 channel.  At p = 2
 // its tile of 7 elements, a lane of which takes as long as three of the one-row

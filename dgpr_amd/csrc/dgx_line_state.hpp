@@ -12,14 +12,16 @@
 //     element's ends and the z derivative come through the scalar cache.
 //   * LDS is read for the other points of a line only, a third less per node;
 //     faces normal to z need no gather.
-// What bounds it is FP64 issue at p = 3 (4100 FP64 and 324 matrix instructions
-// per wavefront of 256 nodes, 75 % of the cycles at 2 wavefronts per SIMD) and
-// at p = 2 issue and LDS in equal parts.  Per RK4 stage against the
-// 2-element tile of dgx_tile_state.hpp, 64^3 p = 3 cube: 1105 against 1266 us,
-// 48x24x24 p = 3 curved channel (TVD-RK3) 149 against 162; against the one-row
-// kernel, 32^3 p = 2 cube 107 against 136 us, 30x24x28 p = 2 curved channel 87
-// against 106.  One wavefront takes 20 us against 11 (p = 3) and 12 us (p = 2)
-// of the others, so small meshes keep those (line_tiled, apply_defaults).  At
+// What bounds it is FP64 issue at p = 3 (3900 FP64 and 324 matrix instructions
+// per wavefront of 256 nodes at 2 wavefronts per SIMD) together with the traffic
+// of the state arrays (64^3 cube: 4.55 GB per launch, 87 % of the rate of a large
+// copy), and at p = 2 issue and LDS in equal parts.  Per RK4 stage against the
+// 2-element tile of dgx_tile_state.hpp, 64^3 p = 3 cube: 1083 against 1266 us,
+// 48x24x24 p = 3 curved channel (TVD-RK3) 132 against 162 (both with the longer
+// geometry 149 against 162); against the one-row kernel, 32^3 p = 2 cube 107
+// against 136 us, 30x24x28 p = 2 curved channel 81 against 106.  One wavefront
+// takes 20 us against 11 (p = 3) and 12 us (p = 2) of the others, so small meshes
+// keep those (line_tiled, apply_defaults).  At
 // p = 1 the same layout measured 4 % slower (16 elements of 6 faces take 18 KB
 // of LDS).
 // Included by dgx_stage.hpp inside namespace dgx, after dgx_tile_state.hpp.
@@ -482,9 +484,11 @@ __device__ __forceinline__ void line_body(const MeshArgs& mesh, const Phys& ph, 
   using LD = LineDims<P>;
   using TL = LineLds<P, AFF>;
   constexpr int N = LD::N, NB = LD::NB, NF = LD::NF, E = LD::E, JS = LD::JS;
-  // base state and accumulator loaded during the last subpass; at p = 3 the 80
-  // registers are not there (14 spilled)
-  constexpr bool PREF = P != 3;
+  // z rows of the base state and accumulator loaded during the last subpass: all
+  // at p = 2; at p = 3 the registers of three are there (four spill).  Against
+  // none at p = 3: 64^3 cube 1104 -> 1083 us per RK4 stage, 32^3 144 -> 137,
+  // 48x24x24 channel 132.4 -> 131.6
+  constexpr int KP = P == 3 ? 3 : N;
 
   double* sV = reinterpret_cast<double*>(lds + TL::oV);
   auto sX  = reinterpret_cast<double(*)[24]>(lds + TL::oX);    // curved meshes
@@ -632,10 +636,10 @@ __device__ __forceinline__ void line_body(const MeshArgs& mesh, const Phys& ph, 
             if constexpr (S & 1)
               hg.load(mesh, sNb, (S + 1) / 2);
           }
-          else if (PREF && ln.act)
+          else if (ln.act)
           {
 #pragma unroll
-            for (int k = 0; k < N; ++k)
+            for (int k = 0; k < KP; ++k)
             {
               if (sa.Vout && sa.ca != 0.0)  // Vbase may be null without Vout
 #pragma unroll
@@ -662,10 +666,10 @@ __device__ __forceinline__ void line_body(const MeshArgs& mesh, const Phys& ph, 
   subpass(Const<5>{});
 
   double q[NORM ? N : 1][5];
-  if (!PREF && ln.act)
+  if (KP < N && ln.act)
   {
 #pragma unroll
-    for (int k = 0; k < N; ++k)
+    for (int k = KP; k < N; ++k)
     {
       if (sa.Vout && sa.ca != 0.0)  // Vbase may be null without Vout
 #pragma unroll
