@@ -53,7 +53,7 @@ int dgx::default_stage_waves(int p, int q)
 }
 
 // Stage kernel and occupancy target of a context, where the caller has not
-// chosen them.  q = 1 in FP64: the state-reading tiled kernel at p = 1 and 3, at
+// chosen them.  q = 1 in FP64, faces matched: the state-reading tiled kernel at p = 1 and 3, at
 // 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1083
 // against 1930 us per RK4 stage on the 64^3 p = 3 cube, 267 against 442 us on
 // the 64^3 p = 1 cube, 137 against 188 us on a 61x37x43 p = 1 channel.  At p = 2
@@ -61,16 +61,16 @@ int dgx::default_stage_waves(int p, int q)
 // kernel's, needs more elements to fill the chip: one-row against tiled, affine:
 // 10120 elements 42.2 / 42.4 us, 15000 59.4 / 63.8, 32768 136 / 107; curved: 7220
 // 45.6 / 50.0, 8400 57.1 / 50.5, 15000 83.8 / 78.9, 20160 106 / 87.  The
-// mixed forms: the record-reading tiled kernel at p = 3, q = 1 (3 waves per
-// SIMD on affine meshes, 2 on curved ones, where 3 spills).  The general-order
+// mixed forms and FP64 on unmatched faces: the record-reading tiled kernel at p =
+// 3, q = 1 (mixed on affine meshes 3 waves per SIMD, else 2, where 3 spills).  The general-order
 // kernel (tile 2) outside 1 <= p, q <= 3, the one-row kernel elsewhere.
 static void apply_defaults(dgx_ctx* c)
 {
-  const bool fp64  = c->prec == DGX_PREC_FP64;
+  const bool fp64  = c->prec == DGX_PREC_FP64, states = fp64 && c->matched;
   const bool line2 = c->p == 2 && c->nelem >= (c->affine ? 16384 : 8192);
   if (!c->tile_chosen)
     c->stage_tile = general_order(c->p, c->q) ? 2
-                  : c->q == 1 && (c->p == 3 || (fp64 && (c->p == 1 || line2))) ? 1 : 0;
+                  : c->q == 1 && (c->p == 3 || (states && (c->p == 1 || line2))) ? 1 : 0;
   if (!c->waves_chosen)
     c->stage_waves = c->stage_tile != 1 ? default_stage_waves(c->p, c->q)
                                         : (!fp64 && c->p == 3 && c->affine ? 3 : 2);
@@ -113,6 +113,7 @@ MeshArgs dgx::mesh_args(const dgx_ctx* c)
   for (int i = 0; i < 6; ++i)
     m.bounds[i] = c->bounds[i];
   m.affine = c->affine;
+  m.matched = c->matched;
   m.lamf   = c->lamf;
   m.arec   = c->arec;
   m.geov   = c->geo;
@@ -315,8 +316,8 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
     if ((e = hipMalloc(tbufs[i], tb)) != hipSuccess)
       return bail("hipMalloc(traces)", e);
   drop_traces(c);
-  c->prec = DGX_PREC_FP64;
-  apply_defaults(c);
+  c->prec    = DGX_PREC_FP64;
+  c->matched = 1;
   c->bytes = 5 * sb + 3 * tb +
              (nn + nlam +
               (c->affine ? (size_t)c->nelem * 6 + affine_record_doubles(c->nelem) : 0) + (size_t)c->npartial +
@@ -367,6 +368,21 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   }
   if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);
+  if (c->q == 1)
+  {
+    int bad = 0;
+    if ((e = matched_dispatch(mesh_args(c), c->status, c->stream)) != hipSuccess)
+      return bail("face check", e);
+    if ((e = hipMemcpyAsync(&bad, c->status, sizeof(int), hipMemcpyDeviceToHost, c->stream)) !=
+        hipSuccess)
+      return bail("hipMemcpy(face check)", e);
+    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess)
+      return bail("hipStreamSynchronize", e);
+    c->matched = !bad;
+    if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
+      return bail("hipMemset(status)", e);
+  }
+  apply_defaults(c);
   if ((e = hipStreamSynchronize(c->stream)) != hipSuccess)
     return bail("hipStreamSynchronize", e);
   *out = c;
@@ -657,7 +673,7 @@ static hipError_t launch_step(dgx_ctx* c, int scheme, double dt, bool want_norm,
       if (!fused && (e = norm_partials_dispatch(c->p, c->q, mesh_args(c), f1, c->partial,
                                                 c->stream)) != hipSuccess)
         return e;
-      const int nb = fused ? tile_blocks(c->p, c->nelem, c->prec != DGX_PREC_FP64, c->stage_waves)
+      const int nb = fused ? tile_blocks(c->p, c->nelem, !reads_states(c), c->stage_waves)
                            : norm_blocks(c->p, c->q, c->nelem);
       e = norm_dev ? norm_dispatch(c->partial, nb, 1.0 / (double)c->nstate, norm_dev, c->stream)
                    : sum_dispatch(c->partial, nb, c->sum, c->stream);
@@ -772,6 +788,14 @@ dgx_status dgx_set_tile(dgx_ctx* c, int tile)
   apply_defaults(c);
   if (!tile_valid(c->p, c->q, tile, c->stage_waves))
     c->stage_waves = 2;  // the tiled kernels are compiled for 2 and 3 waves per SIMD
+  return DGX_OK;
+}
+
+dgx_status dgx_faces_match(const dgx_ctx* c, int* match)
+{
+  if (!c || !match)
+    return DGX_ERR_INVALID;
+  *match = c->matched;
   return DGX_OK;
 }
 

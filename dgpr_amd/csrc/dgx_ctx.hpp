@@ -41,6 +41,7 @@ struct dgx_ctx
   bool tile_chosen, waves_chosen;  // by the caller (else the defaults)
   int prec;         // DGX_PREC_* (float trace records in the mixed forms)
   int affine;       // q = 1 and every element a parallelepiped
+  int matched;      // both elements at a face have the same face up to a translation (q = 1)
   double* mean;     // running mean (Gauss-nodal), allocated on first use
   double* adj_store;       // stored stages of the last dgx_adjoint_rk4 (kept:
   size_t adj_store_bytes;  // freeing tens of GB can take seconds)
@@ -66,7 +67,7 @@ hipError_t ensure_boundary(dgx_ctx* c);
 // whether the context's stages read states instead of trace records
 inline bool reads_states(const dgx_ctx* c)
 {
-  return c->stage_tile == 1 && c->prec == DGX_PREC_FP64;
+  return c->stage_tile == 1 && c->prec == DGX_PREC_FP64 && c->matched;
 }
 // the last stage of a step has written U and what the next stage reads
 inline void stage_outputs_valid(dgx_ctx* c)

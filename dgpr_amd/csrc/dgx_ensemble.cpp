@@ -42,6 +42,7 @@ struct EnsGroup
 {
   int p, q;      // p = 0 for a one-launch group of q = 1 members of any order
   int affine;    // every member an affine q = 1 mesh
+  int matched;   // unit_grid: every member's faces match (dgx_faces_match)
   bool unit_grid;  // the ensemble stage kernel (layouts 1, 2), else batched
   std::vector<int> members;
   int nblocks;   // grid blocks (batched) or work units (ensemble kernel)
@@ -277,14 +278,16 @@ dgx_status dgx_ensemble_create(int ncase, const dgx_mesh* meshes, const dgx_para
   }
   en->device = en->ctx[0]->device;
   en->layout = 1;
-  auto group_of = [&](bool unit_grid, int p, int q, int affine) -> EnsGroup& {
+  auto group_of = [&](bool unit_grid, int p, int q, int affine, int matched = 1) -> EnsGroup& {
     for (EnsGroup& x : en->groups)
-      if (x.unit_grid == unit_grid && x.p == p && x.q == q && x.affine == affine)
+      if (x.unit_grid == unit_grid && x.p == p && x.q == q && x.affine == affine &&
+          x.matched == matched)
         return x;
     EnsGroup ng;
     ng.p = p;
     ng.q = q;
     ng.affine = affine;
+    ng.matched = matched;
     ng.unit_grid = unit_grid;
     ng.nblocks = 0;
     ng.waves = unit_grid ? 3 : default_stage_waves(p, q);
@@ -295,9 +298,9 @@ dgx_status dgx_ensemble_create(int ncase, const dgx_mesh* meshes, const dgx_para
     en->groups.push_back(ng);
     return en->groups.back();
   };
-  // batched groups per (p, q, affine); one-launch groups per affine class of
-  // the q = 1 members, and per (order, affine class), largest members (most
-  // elements x nodes) first
+  // batched groups per (p, q, affine); one-launch groups per class (affine,
+  // matched faces) of the q = 1 members, and per (order, class), largest members
+  // (most elements x nodes) first
   for (int i = 0; i < ncase; ++i)
   {
     dgx_ctx* c = en->ctx[i];
@@ -314,8 +317,8 @@ dgx_status dgx_ensemble_create(int ncase, const dgx_mesh* meshes, const dgx_para
     dgx_ctx* c = en->ctx[i];
     if (c->q == 1 && !general_order(c->p, c->q))
     {
-      group_of(true, 0, 1, c->affine).members.push_back(i);
-      group_of(true, c->p, 1, c->affine).members.push_back(i);
+      group_of(true, 0, 1, c->affine, c->matched).members.push_back(i);
+      group_of(true, c->p, 1, c->affine, c->matched).members.push_back(i);
     }
   }
   auto bail = [&](const char* what, hipError_t e) {
@@ -489,7 +492,8 @@ dgx_status dgx_ensemble_autotune(dgx_ensemble* en, int scheme, const double* dt,
       int best_w = g.waves, best_t = g.tile;
       float best_ms = 0.0f;
       bool have = false;
-      for (int t = 0; t <= (g.unit_grid ? 1 : 0); ++t)
+      // the tiled units read states: not for members whose faces do not match
+      for (int t = 0; t <= (g.unit_grid && g.matched ? 1 : 0); ++t)
         for (int w = g.unit_grid ? 2 : 1; w <= 3; ++w)
         {
           g.waves = w;

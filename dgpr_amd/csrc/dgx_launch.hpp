@@ -71,6 +71,10 @@ struct MeshArgs
   // constant over a parallelepiped's face (fJ / det J times a table sum);
   // null otherwise
   const double* lamf;
+  // q = 1: both elements at a face have the same face up to a translation
+  // (matched_dispatch), so that the kernels that read the neighbour's state may
+  // take the face's geometry from their own side
+  int matched;
   // affine meshes: each element's constant geometry [e][GREC] (affine_record
   // in dgx_stage.hpp); null otherwise
   const double* arec;
@@ -109,7 +113,7 @@ struct StageArgs
               // matrix cores, 2 split-BF16 matrix cores (with trace32 set)
   // tiled kernel only (tile 1): when set, normp[block] receives the block's
   // sum of R^2, R = -B3^T W f (the residual norm of this stage's f), for
-  // tile_blocks(p, nelem, trace32, waves) blocks
+  // tile_blocks(p, nelem, records, waves) blocks
   double* normp = nullptr;
   // FP64 tiled kernel only: 0 writes just the boundary states of Vout's inflow
   // and outflow faces to Tout (all that its next stage reads); the other
@@ -139,8 +143,9 @@ struct BatchItem
 hipError_t rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
                         const double* lam, int* status, int waves, hipStream_t st, int tile = 0);
 bool tile_valid(int p, int q, int tile, int waves);
-// the tiled kernel (tile 1) of q = 1 meshes (dgx_tile_kernels.hip): in FP64 it
-// reads both sides' states, and of Tin only the boundary states of Vin
+// the tiled kernel (tile 1) of q = 1 meshes (dgx_tile_kernels.hip): in FP64 on
+// meshes of matched faces it reads both sides' states, and of Tin only the
+// boundary states of Vin
 hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const StageArgs& sa,
                              const double* lam, int* status, int waves, hipStream_t st);
 // boundary states of V (q = 1) into the boundary section of the record set
@@ -148,6 +153,9 @@ hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const Sta
 hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
                              double* Tout, int* status, hipStream_t st);
 hipError_t upload_tables_tile(const PTab* pt, const QTab* qt);
+// q = 1: *flag (device) becomes 1 if the two elements at some face, periodic
+// ones included, have faces that differ by more than a translation
+hipError_t matched_dispatch(const MeshArgs& m, int* flag, hipStream_t st);
 // affine meshes: arec (affine_record_doubles(nelem)) of every element
 size_t affine_record_doubles(int nelem);
 // geov and geof of the mesh (q > 1, or an order of the general kernels)
@@ -163,8 +171,9 @@ hipError_t rhs_batch_dispatch(int p, int q, const BatchItem* items_dev, int nite
                               int* status, int waves, bool affine, hipStream_t st);
 // grid blocks of one mesh in a stage launch
 int stage_blocks(int p, int nelem);
-// grid blocks of the tiled kernel (tile 1) on one mesh
-int tile_blocks(int p, int nelem, bool trace32, int waves);
+// grid blocks of the tiled kernel (tile 1) on one mesh; records: of the body that
+// reads trace records
+int tile_blocks(int p, int nelem, bool records, int waves);
 // fout = f(V; mu = 0), the inviscid right-hand side, from V and its trace
 // records Tin (written with any mu: their tractions are not read)
 hipError_t inviscid_rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, const double* V,

@@ -1028,15 +1028,16 @@ __device__ __forceinline__ void stage_body(const MeshArgs& mesh, const Phys& ph,
 #include "dgx_tile_state.hpp"
 #include "dgx_line_state.hpp"
 
-// The tiled stage kernel: the record-reading body with FP32 records (the
+// The tiled stage kernel: the record-reading body (REC) with FP32 records (the
 // mixed forms, where a last-bit change of a trace can flip its rounding: the
-// records keep their arithmetic), a state-reading body in FP64.
-template <int P, int Q, int R, int W, typename TT, bool AFF, int CT = 0, bool NORM = false>
+// records keep their arithmetic) and in FP64 on meshes whose faces do not match
+// (the neighbour's tractions are of its own geometry), else a state-reading body.
+template <int P, int Q, int R, int W, typename TT, bool AFF, int CT = 0, bool NORM = false,
+          bool REC = sizeof(TT) == sizeof(float)>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W)))
 void dgx_tile_stage_kernel(MeshArgs mesh, Phys ph, StageArgs sa, const double* __restrict__ lam,
                            int* status)
 {
-  constexpr bool REC = sizeof(TT) == sizeof(float);
   constexpr size_t LDS = REC ? TileLds<P, Q, R>::bytes : StateLds<P, Q, R, AFF>::bytes;
   __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
   if constexpr (REC)

@@ -92,6 +92,73 @@ hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const dou
   return hipErrorInvalidValue;
 }
 
+// One thread per element and direction: the element's high face against the low
+// face of the element across it, corner differences to a few roundings of the
+// coordinates.
+__global__ __launch_bounds__(256) void dgx_matched_kernel(MeshArgs mesh, int* flag)
+{
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= (size_t)mesh.nelem * 3)
+    return;
+  const int e = (int)(t / 3), d = (int)(t % 3);
+  const int ci = e % mesh.nx, cj = (e / mesh.nx) % mesh.ny, ck = e / (mesh.nx * mesh.ny);
+  int bt;
+  const int nb = neighbour(mesh, ci, cj, ck, 2 * d + 1, &bt);
+  if (nb < 0)
+    return;
+  // node strides along the face and across it
+  const int s1 = d == 0 ? 6 : 3, s2 = d == 2 ? 6 : 12;
+  const double* A = mesh.nodes + (size_t)e * 24 + (3 << d);
+  const double* B = mesh.nodes + (size_t)nb * 24;
+  double diff = 0.0, mag = 0.0;
+  bool same = true;
+  for (int c = 0; c < 4; ++c)
+  {
+    const int o = (c & 1) * s1 + (c >> 1) * s2;
+    for (int i = 0; i < 3; ++i)
+    {
+      const double x = (A[o + i] - A[i]) - (B[o + i] - B[i]);
+      same = same && x == x;
+      diff = fmax(diff, fabs(x));
+      mag  = fmax(mag, fmax(fabs(A[o + i]), fabs(B[o + i])));
+    }
+  }
+  if (!same || !(diff <= 8.0 * 2.220446049250313e-16 * mag))
+    atomicOr(flag, 1);
+}
+
+hipError_t matched_dispatch(const MeshArgs& m, int* flag, hipStream_t st)
+{
+  hipLaunchKernelGGL(dgx_matched_kernel, dim3((unsigned)(((size_t)m.nelem * 3 + 255) / 256)),
+                     dim3(256), 0, st, m, flag);
+  return hipGetLastError();
+}
+
+// the record-reading body in FP64 (meshes whose faces do not match)
+template <int P>
+static hipError_t launch_tile_rec(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
+                                  const double* lam, int* status, int waves, hipStream_t st)
+{
+  constexpr int R = tile_rows(P);
+  const dim3 grid(tile_blocks(P, m.nelem, true, waves)), block(64);
+  const bool norm = sa.normp != nullptr;
+  if (waves == 2 && norm)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, 1, R, 2, double, false, 0, true, true>), grid, block,
+                       0, st, m, ph, sa, lam, status);
+  else if (waves == 2)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, 1, R, 2, double, false, 0, false, true>), grid, block,
+                       0, st, m, ph, sa, lam, status);
+  else if (waves == 3 && norm)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, 1, R, 3, double, false, 0, true, true>), grid, block,
+                       0, st, m, ph, sa, lam, status);
+  else if (waves == 3)
+    hipLaunchKernelGGL((dgx_tile_stage_kernel<P, 1, R, 3, double, false, 0, false, true>), grid, block,
+                       0, st, m, ph, sa, lam, status);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
 template <int P, int Q, int W, typename TT, bool AFF, int CT, bool NORM>
 static void launch_tile_w(const MeshArgs& m, const Phys& ph, const StageArgs& sa, const double* lam,
                           int* status, hipStream_t st)
@@ -150,6 +217,8 @@ static hipError_t launch_tile(const MeshArgs& m, const Phys& ph, const StageArgs
   if (sa.trace32)
     return m.affine ? launch_tile_t<P, 1, float, true>(m, ph, sa, lam, status, waves, st)
                     : launch_tile_t<P, 1, float, false>(m, ph, sa, lam, status, waves, st);
+  if (!m.matched)
+    return launch_tile_rec<P>(m, ph, sa, lam, status, waves, st);
   return m.affine ? launch_tile_t<P, 1, double, true>(m, ph, sa, lam, status, waves, st)
                   : launch_tile_t<P, 1, double, false>(m, ph, sa, lam, status, waves, st);
 }

@@ -153,6 +153,7 @@ def lib():
         L.dgx_autotune.argtypes = [P_ctx, C.c_int, C.POINTER(C.c_int), PD]
         L.dgx_set_tile.argtypes = [P_ctx, C.c_int]
         L.dgx_get_tile.argtypes = [P_ctx, C.POINTER(C.c_int)]
+        L.dgx_faces_match.argtypes = [P_ctx, C.POINTER(C.c_int)]
         L.dgx_autotune_tiles.argtypes = [P_ctx, C.c_int, C.POINTER(C.c_int),
                                          C.POINTER(C.c_int), PD]
         for nm in ("dgx_create", "dgx_destroy", "dgx_set_params", "dgx_set_state",
@@ -165,7 +166,7 @@ def lib():
                    "dgx_write_dg", "dgx_read_dg_header", "dgx_read_dg", "dgx_set_tuning",
                    "dgx_mesh_is_affine",
                    "dgx_get_tuning", "dgx_autotune", "dgx_set_precision", "dgx_get_precision",
-                   "dgx_set_tile", "dgx_get_tile", "dgx_autotune_tiles",
+                   "dgx_set_tile", "dgx_get_tile", "dgx_faces_match", "dgx_autotune_tiles",
                    "dgx_sample_output",
                    "dgx_sample_output_device", "dgx_update_mean", "dgx_get_mean",
                    "dgx_set_mean", "dgx_write_dg_outputs", "dgx_read_dg_output_key",
@@ -559,13 +560,21 @@ class Solver:
         t = self.tile if tile is None else tile
         if t == 2:
             return "dgx_gen_stage_kernel<%d,double>" % self.mesh.p
-        p, fp64 = self.mesh.p, self.precision == "fp64"
-        if t and fp64 and (p == 2 or (p == 3 and w == 2 and self.mesh.nelem >= 12288)):
+        p, states = self.mesh.p, self.precision == "fp64" and self.faces_match
+        if t and states and (p == 2 or (p == 3 and w == 2 and self.mesh.nelem >= 12288)):
             return "dgx_line_stage_kernel<%d,%d>" % (p, w)
         if t:
             return "dgx_tile_stage_kernel<%d,%d,%d,%d>" % (self.mesh.p, self.mesh.q,
                                                            self.TILE_ROWS[self.mesh.p], w)
         return "dgx_rhs_stage_kernel<%d,%d,%d>" % (self.mesh.p, self.mesh.q, w)
+
+    @property
+    def faces_match(self):
+        """Whether both elements at every face have the same face up to a
+        translation (dgx_faces_match)."""
+        m = C.c_int()
+        _chk(lib().dgx_faces_match(self.ctx, C.byref(m)), self.ctx)
+        return bool(m.value)
 
     @property
     def tile(self):

@@ -405,6 +405,14 @@ dgx_status dgx_autotune(dgx_ctx* ctx, int reps, int* chosen, double us_out[3]);
  * Results agree to rounding. */
 dgx_status dgx_set_tile(dgx_ctx* ctx, int tile);
 dgx_status dgx_get_tile(const dgx_ctx* ctx, int* tile);
+/* Whether at every face between two elements, periodic ones included, both
+ * elements have the same face up to a translation, to 8 ulps of its largest
+ * coordinate (q = 1; 1 for q > 1, where it decides nothing; no counterpart in
+ * the reference, which stores each side's metrics).  Where it does not hold (the
+ * two sides of a periodic direction curved differently), every tile takes the
+ * neighbour's gradient with the neighbour's own geometry: the FP64 tiled kernel
+ * then reads trace records, and tile 0 is the default at p = 1 and 2. */
+dgx_status dgx_faces_match(const dgx_ctx* ctx, int* match);
 
 /* Times every (tile, occupancy target) pair on this context's mesh as
  * dgx_autotune does and keeps the fastest; us_out[3 * tile + waves - 1]
