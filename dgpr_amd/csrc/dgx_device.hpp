@@ -46,6 +46,17 @@ __device__ __forceinline__ double rsq(double x)
   return __builtin_fma(0.5 * y, e, y);
 }
 
+// x, negative also where y is: the sign that a quotient of two negatives loses.
+__device__ __forceinline__ double with_sign_of(double x, double y)
+{
+  unsigned long long a, b;
+  __builtin_memcpy(&a, &x, 8);
+  __builtin_memcpy(&b, &y, 8);
+  a |= b & 0x8000000000000000ull;
+  __builtin_memcpy(&x, &a, 8);
+  return x;
+}
+
 // Euler flux F[d][r] of conserved state U.
 __device__ __forceinline__ void euler_flux(const double* U, double gamma,
                                            double F[3][5])
@@ -141,8 +152,9 @@ __device__ __forceinline__ void roe_flux(const T* Ul, const T* Ur, const double*
 // records and tests follow).  ul, ur are the velocities and irl, irr the
 // reciprocal densities of the two states, which the caller needs too.  The Roe
 // weights come from one square root, wr = s / (1 + s) with s = sqrt(rr / rl); c and 1/c
-// from one reciprocal square root; 1/(2 eps) is 10/c.  Also returns the jumps
-// d = Ur - Ul.
+// from one reciprocal square root; 1/(2 eps) is 10/c.  A negative density on
+// either side, or on both, gives NaN as the square roots of the densities do.
+// Also returns the jumps d = Ur - Ul.
 __device__ __forceinline__ void roe_flux_fp64(const double* Ul, const double* ul, double irl,
                                               const double* Ur, const double* ur, double irr,
                                               const double* n, double g, double* f, double* d)
@@ -151,7 +163,7 @@ __device__ __forceinline__ void roe_flux_fp64(const double* Ul, const double* ul
   const double pl = gm1 * (Ul[4] - 0.5 * (Ul[1] * ul[0] + Ul[2] * ul[1] + Ul[3] * ul[2]));
   const double pr = gm1 * (Ur[4] - 0.5 * (Ur[1] * ur[0] + Ur[2] * ur[1] + Ur[3] * ur[2]));
   const double Hl = (Ul[4] + pl) * irl, Hr = (Ur[4] + pr) * irr;
-  const double x = Ur[0] * irl, s = x * rsq(x);
+  const double x = with_sign_of(Ur[0] * irl, Ul[0]), s = x * rsq(x);
   const double wr = s * rcp(1.0 + s);
   const double u[3] = {ul[0] + wr * (ur[0] - ul[0]), ul[1] + wr * (ur[1] - ul[1]),
                        ul[2] + wr * (ur[2] - ul[2])};
