@@ -65,7 +65,8 @@ class ResidualFunction(torch.autograd.Function):
         solver = ctx.solver
         _load_state(solver, U)
         if U.is_cuda:
-            w = g.detach().to(U.device, torch.float64).contiguous()
+            # the library reads the stored values: a lazily negated view is not one
+            w = g.detach().to(U.device, torch.float64).resolve_neg().contiguous()
             gU = torch.empty(U.shape, dtype=torch.float64, device=U.device)
             torch.cuda.current_stream(U.device).synchronize()
             solver.residual_vjp_device(w.data_ptr(), gU.data_ptr())
@@ -109,7 +110,7 @@ class KineticEnergyRK4(torch.autograd.Function):
             torch.cuda.current_stream(U0.device).synchronize()
             _, dmu = solver.adjoint_rk4_device(ctx.dt, ctx.nsteps, gU.data_ptr(), ctx.interval,
                                                want_mu=want_mu)
-            gU *= s.to(U0.device)
+            gU = gU * s.to(U0.device)  # (s may carry a batch under vmap)
         else:
             _, g, dmu = solver.adjoint_rk4(ctx.dt, ctx.nsteps, ctx.interval, want_mu=want_mu)
             gU = torch.from_numpy(g).view_as(U0) * s.to(U0.device)
