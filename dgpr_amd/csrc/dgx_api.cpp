@@ -62,7 +62,9 @@ int dgx::default_stage_waves(int p, int q)
 // 10120 elements 42.2 / 42.4 us, 15000 59.4 / 63.8, 32768 136 / 107; curved: 7220
 // 45.6 / 50.0, 8400 57.1 / 50.5, 15000 83.8 / 78.9, 20160 106 / 87.  The
 // mixed forms and FP64 on unmatched faces: the record-reading tiled kernel at p =
-// 3, q = 1 (mixed on affine meshes 3 waves per SIMD, else 2, where 3 spills).  The general-order
+// 3, q = 1 (mixed on affine meshes 3 waves per SIMD, else 2, where 3 spills).  A
+// target that the caller has chosen and the tiled kernel does not have (1) keeps
+// the one-row kernel.  The general-order
 // kernel (tile 2) outside 1 <= p, q <= 3, the one-row kernel elsewhere.
 static void apply_defaults(dgx_ctx* c)
 {
@@ -71,6 +73,8 @@ static void apply_defaults(dgx_ctx* c)
   if (!c->tile_chosen)
     c->stage_tile = general_order(c->p, c->q) ? 2
                   : c->q == 1 && (c->p == 3 || (states && (c->p == 1 || line2))) ? 1 : 0;
+  if (!c->tile_chosen && c->waves_chosen && !tile_valid(c->p, c->q, c->stage_tile, c->stage_waves))
+    c->stage_tile = 0;
   if (!c->waves_chosen)
     c->stage_waves = c->stage_tile != 1 ? default_stage_waves(c->p, c->q)
                                         : (!fp64 && c->p == 3 && c->affine ? 3 : 2);
@@ -761,10 +765,15 @@ dgx_status dgx_get_precision(const dgx_ctx* c, int* precision)
 
 dgx_status dgx_set_tuning(dgx_ctx* c, int stage_waves)
 {
-  if (!c || stage_waves < 1 || stage_waves > 3 || !tile_valid(c->p, c->q, c->stage_tile, stage_waves))
+  if (!c || stage_waves < 1 || stage_waves > 3)
+    return DGX_ERR_INVALID;
+  // at p = 1 and 2 the tile follows the target unless the caller has chosen it
+  const bool follows = !c->tile_chosen && c->stage_tile == 1 && c->p != 3;
+  if (!follows && !tile_valid(c->p, c->q, c->stage_tile, stage_waves))
     return DGX_ERR_INVALID;
   c->stage_waves  = stage_waves;
   c->waves_chosen = true;
+  apply_defaults(c);
   return DGX_OK;
 }
 
@@ -876,6 +885,7 @@ dgx_status dgx_autotune_tiles(dgx_ctx* c, int reps, int* tile_out, int* waves_ou
   if (!c || reps < 1)
     return DGX_ERR_INVALID;
   const int keep_tile = c->stage_tile, keep_waves = c->stage_waves;
+  const bool keep_chosen = c->waves_chosen;
   int best_tile = keep_tile, best_waves = keep_waves;
   double best_us = 0.0;
   bool have = false;
@@ -891,8 +901,9 @@ dgx_status dgx_autotune_tiles(dgx_ctx* c, int reps, int* tile_out, int* waves_ou
       dgx_status st = dgx_autotune(c, reps, &w, us);
       if (st != DGX_OK)
       {
-        c->stage_tile  = keep_tile;
-        c->stage_waves = keep_waves;
+        c->stage_tile   = keep_tile;
+        c->stage_waves  = keep_waves;
+        c->waves_chosen = keep_chosen;
         return st;
       }
       for (int k = 0; k < 3; ++k)

@@ -378,8 +378,11 @@ dgx_status dgx_get_precision(const dgx_ctx* ctx, int* precision);
  * fixed launch shapes, solve_cuda.cu:1235-1282) ---------------------------- */
 
 /* The stage kernel is compiled for occupancy targets of 1, 2 and 3 waves per
- * SIMD (register budgets of 512, 256 and 168 VGPRs).  dgx_create picks a
- * default per (p, q); these set or read the target used by later stages. */
+ * SIMD (register budgets of 512, 256 and 168 VGPRs); the tiled form (dgx_set_tile)
+ * for 2 and 3.  dgx_create picks a default per (p, q); these set or read the
+ * target used by later stages.  At p = 1 and 2, where no tile has been set, a
+ * target of 1 selects tile 0; with tile 1 set, and at p = 3 unless tile 0 is, it
+ * is refused. */
 dgx_status dgx_set_tuning(dgx_ctx* ctx, int stage_waves);
 dgx_status dgx_get_tuning(const dgx_ctx* ctx, int* stage_waves);
 
