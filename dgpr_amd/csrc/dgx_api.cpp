@@ -677,7 +677,7 @@ static hipError_t launch_step(dgx_ctx* c, int scheme, double dt, bool want_norm,
       if (!fused && (e = norm_partials_dispatch(c->p, c->q, mesh_args(c), f1, c->partial,
                                                 c->stream)) != hipSuccess)
         return e;
-      const int nb = fused ? tile_blocks(c->p, c->nelem, !reads_states(c), c->stage_waves)
+      const int nb = fused ? tile_blocks(c->p, c->nelem, !reads_states(c))
                            : norm_blocks(c->p, c->q, c->nelem);
       e = norm_dev ? norm_dispatch(c->partial, nb, 1.0 / (double)c->nstate, norm_dev, c->stream)
                    : sum_dispatch(c->partial, nb, c->sum, c->stream);

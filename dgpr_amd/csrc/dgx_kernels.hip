@@ -801,11 +801,11 @@ hipError_t inviscid_rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph
 #undef CALL_INV
 }
 
-int tile_blocks(int p, int nelem, bool records, int waves)
+int tile_blocks(int p, int nelem, bool records)
 {
   const int n = p + 1;
   int e = 64 / (n * n);
-  if (records || !line_tiled(p, nelem, waves))
+  if (records || !line_tiled(p, nelem))
     e = tile_rows(p) > 0 ? tile_rows(p) * (64 / (n * n * n)) : 1;
   return (nelem + e - 1) / e;
 }

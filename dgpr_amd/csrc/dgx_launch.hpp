@@ -113,7 +113,7 @@ struct StageArgs
               // matrix cores, 2 split-BF16 matrix cores (with trace32 set)
   // tiled kernel only (tile 1): when set, normp[block] receives the block's
   // sum of R^2, R = -B3^T W f (the residual norm of this stage's f), for
-  // tile_blocks(p, nelem, records, waves) blocks
+  // tile_blocks(p, nelem, records) blocks
   double* normp = nullptr;
   // FP64 tiled kernel only: 0 writes just the boundary states of Vout's inflow
   // and outflow faces to Tout (all that its next stage reads); the other
@@ -173,7 +173,7 @@ hipError_t rhs_batch_dispatch(int p, int q, const BatchItem* items_dev, int nite
 int stage_blocks(int p, int nelem);
 // grid blocks of the tiled kernel (tile 1) on one mesh; records: of the body that
 // reads trace records
-int tile_blocks(int p, int nelem, bool records, int waves);
+int tile_blocks(int p, int nelem, bool records);
 // fout = f(V; mu = 0), the inviscid right-hand side, from V and its trace
 // records Tin (written with any mu: their tractions are not read)
 hipError_t inviscid_rhs_dispatch(int p, int q, const MeshArgs& m, const Phys& ph, const double* V,

@@ -33,13 +33,12 @@ constexpr bool line_order(int p)
 }
 
 // Whether tile 1 in FP64 runs this kernel: always at p = 2; at p = 3 from three
-// wavefronts per SIMD (1024 SIMDs, 4 elements each) at the 2-wave target.  Per
-// RK4 stage, 2-element against 4-element tile: 5202 elements 35.4 against 39.7
+// wavefronts per SIMD (1024 SIMDs, 4 elements each).  Per RK4 stage, 2-element against 4-element tile: 5202 elements 35.4 against 39.7
 // us, 8000 45.5 / 45.7, 11132 61.8 / 63.1, 32768 160 / 145; curved 5202 41.6 /
 // 47.6, 11132 74.5 / 74.4, 27648 (TVD-RK3) 162 / 149.
-constexpr bool line_tiled(int p, int nelem, int waves)
+constexpr bool line_tiled(int p, int nelem)
 {
-  return p == 2 || (p == 3 && waves == 2 && nelem >= 12288);
+  return p == 2 || (p == 3 && nelem >= 12288);
 }
 
 template <int P>

@@ -140,7 +140,7 @@ static hipError_t launch_tile_rec(const MeshArgs& m, const Phys& ph, const Stage
                                   const double* lam, int* status, int waves, hipStream_t st)
 {
   constexpr int R = tile_rows(P);
-  const dim3 grid(tile_blocks(P, m.nelem, true, waves)), block(64);
+  const dim3 grid(tile_blocks(P, m.nelem, true)), block(64);
   const bool norm = sa.normp != nullptr;
   if (waves == 2 && norm)
     hipLaunchKernelGGL((dgx_tile_stage_kernel<P, 1, R, 2, double, false, 0, true, true>), grid, block,
@@ -164,9 +164,9 @@ static void launch_tile_w(const MeshArgs& m, const Phys& ph, const StageArgs& sa
                           int* status, hipStream_t st)
 {
   constexpr bool FP64 = sizeof(TT) == sizeof(double);
-  const dim3 grid(tile_blocks(P, m.nelem, !FP64, W));
+  const dim3 grid(tile_blocks(P, m.nelem, !FP64));
   if constexpr (FP64 && line_order(P))
-    if (line_tiled(P, m.nelem, W))
+    if (line_tiled(P, m.nelem))
     {
       hipLaunchKernelGGL((dgx_line_stage_kernel<P, W, AFF, NORM>), grid, dim3(64), 0, st, m, ph, sa,
                          lam, status);
@@ -181,17 +181,23 @@ template <int P, int Q, typename TT, bool AFF, int CT>
 static hipError_t launch_tile_ct(const MeshArgs& m, const Phys& ph, const StageArgs& sa,
                                  const double* lam, int* status, int waves, hipStream_t st)
 {
-  const bool norm = sa.normp != nullptr;
+  if (waves != 2 && waves != 3)
+    return hipErrorInvalidValue;
+  // a target of 3 runs the 2-wave instance of the state-reading bodies at p = 2
+  // and 3: with a third of the registers less they spill.  Per stage at 2 and at 3
+  // waves: 32^3 p = 2 90 / 220 us, 16^3 p = 3 23 / 41, 64^3 p = 3 978 / 2554,
+  // 48x24x24 p = 3 curved 128 / 253 (p = 1: 64^3 247 / 234)
+  constexpr bool FP64 = sizeof(TT) == sizeof(double);
+  constexpr int W3    = FP64 && P != 1 ? 2 : 3;
+  const bool norm     = sa.normp != nullptr;
   if (waves == 2 && norm)
     launch_tile_w<P, Q, 2, TT, AFF, CT, true>(m, ph, sa, lam, status, st);
   else if (waves == 2)
     launch_tile_w<P, Q, 2, TT, AFF, CT, false>(m, ph, sa, lam, status, st);
-  else if (waves == 3 && norm)
-    launch_tile_w<P, Q, 3, TT, AFF, CT, true>(m, ph, sa, lam, status, st);
-  else if (waves == 3)
-    launch_tile_w<P, Q, 3, TT, AFF, CT, false>(m, ph, sa, lam, status, st);
+  else if (norm)
+    launch_tile_w<P, Q, W3, TT, AFF, CT, true>(m, ph, sa, lam, status, st);
   else
-    return hipErrorInvalidValue;
+    launch_tile_w<P, Q, W3, TT, AFF, CT, false>(m, ph, sa, lam, status, st);
   return hipGetLastError();
 }
 

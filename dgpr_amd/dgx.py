@@ -550,7 +550,7 @@ class Solver:
     }
 
     # rows per tile of the tiled stage kernel of the mixed forms, and of the FP64
-    # one at p = 1 and (below 12288 elements or at 3 waves) p = 3
+    # one at p = 1 and (below 12288 elements) p = 3
     TILE_ROWS = {1: 1, 2: 3, 3: 2}
 
     def stage_kernel_name(self, waves=None, tile=None):
@@ -561,7 +561,9 @@ class Solver:
         if t == 2:
             return "dgx_gen_stage_kernel<%d,double>" % self.mesh.p
         p, states = self.mesh.p, self.precision == "fp64" and self.faces_match
-        if t and states and (p == 2 or (p == 3 and w == 2 and self.mesh.nelem >= 12288)):
+        if t and states and p > 1:
+            w = 2  # what a target of 3 runs too
+        if t and states and (p == 2 or (p == 3 and self.mesh.nelem >= 12288)):
             return "dgx_line_stage_kernel<%d,%d>" % (p, w)
         if t:
             return "dgx_tile_stage_kernel<%d,%d,%d,%d>" % (self.mesh.p, self.mesh.q,

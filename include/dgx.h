@@ -379,7 +379,7 @@ dgx_status dgx_get_precision(const dgx_ctx* ctx, int* precision);
 
 /* The stage kernel is compiled for occupancy targets of 1, 2 and 3 waves per
  * SIMD (register budgets of 512, 256 and 168 VGPRs); the tiled form (dgx_set_tile)
- * for 2 and 3.  dgx_create picks a default per (p, q); these set or read the
+ * for 2 and 3, in FP64 at p = 2 and 3 for 2, which a target of 3 runs too.  dgx_create picks a default per (p, q); these set or read the
  * target used by later stages.  At p = 1 and 2, where no tile has been set, a
  * target of 1 selects tile 0; with tile 1 set, and at p = 3 unless tile 0 is, it
  * is refused. */
