@@ -862,6 +862,8 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
   for (int k = 0; k < NH; ++k)
     if (tid + 64 * k < E * 6 * NbrGeo<AFF>::n)
       (&sH[0][0])[tid + 64 * k] = hg[k];
+  if constexpr (P == 3)  // at p = 1 the first subpass has a fence before it reads sH
+    phase_fence();
 
   // ---- faces, one reference direction at a time ----
   bool ok = true;
