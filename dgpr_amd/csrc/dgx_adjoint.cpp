@@ -39,6 +39,7 @@
 #include "../../include/dgx.h"
 #include "dgx_ctx.hpp"
 #include "dgx_launch.hpp"
+#include "dgx_pool.hpp"
 
 using namespace dgx;
 
@@ -71,46 +72,10 @@ dgx_status afail(dgx_ctx* c, dgx_status st, const char* fmt, ...)
       return afail((c), DGX_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));       \
   } while (0)
 
-hipError_t alloc(DevBuf& b, size_t ndouble)
+hipError_t alloc(const dgx_ctx* c, DevBuf& b, size_t ndouble)
 {
-  return hipMalloc(&b.p, ndouble * sizeof(double));
+  return pool_malloc((void**)&b.p, ndouble * sizeof(double), c->device);
 }
-
-// The temporaries of one adjoint call, cut from the context's workspace.  It
-// stays with the context (grown when a call needs more) until
-// dgx_adjoint_release or dgx_destroy: allocating and freeing a dozen buffers
-// took 1-3 ms a call, more than the kernels of a small residual adjoint.
-struct Workspace
-{
-  double* next = nullptr;
-  hipError_t open(dgx_ctx* c, size_t ndouble)
-  {
-    const size_t need = ndouble * sizeof(double);
-    if (c->adj_ws_bytes < need)
-    {
-      hipError_t e = hipStreamSynchronize(c->stream);
-      if (e == hipSuccess && c->adj_ws)
-        e = hipFree(c->adj_ws);
-      c->adj_ws       = nullptr;
-      c->adj_ws_bytes = 0;
-      if (e == hipSuccess)
-        e = hipMalloc(&c->adj_ws, need);
-      if (e != hipSuccess)
-        return e;
-      c->adj_ws_bytes = need;
-    }
-    next = c->adj_ws;
-    return hipSuccess;
-  }
-  // n doubles, at a multiple of 256 bytes (open() asks for `padded` sizes)
-  double* take(size_t n)
-  {
-    double* p = next;
-    next += padded(n);
-    return p;
-  }
-  static size_t padded(size_t n) { return (n + 31) & ~(size_t)31; }
-};
 
 // one stage kernel launch with explicit physics: Vout = Vbase + cf f(Vin)
 // (Vout may be null), fout = f(Vin) (may be null)
@@ -227,8 +192,8 @@ static dgx_status residual_vjp(dgx_ctx* c, const double* w, double* g, bool host
   if (st != DGX_OK)
     return st;
   const size_t n = c->nstate, tr = trace_doubles(c->p, c->nx, c->ny, c->nz);
-  Workspace ws;
-  AHIP(c, ws.open(c, 3 * Workspace::padded(n) + 2 * Workspace::padded(tr)));
+  Workspace ws(c);
+  AHIP(c, ws.open(3 * Workspace::padded(n) + 2 * Workspace::padded(tr)));
   double *pvol = ws.take(n), *a = ws.take(n), *b = ws.take(n);
   double *aown = ws.take(tr), *anbr = ws.take(tr);
   AHIP(c, ensure_traces(c));
@@ -322,9 +287,9 @@ static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t i
 
   const int ndot = 1024;
   const size_t nsum = dJdmu ? 4 * nsteps : 1;  // one dot product per reverse stage, read back once
-  Workspace ws;
-  AHIP(c, ws.open(c, (dJdmu ? 7 : 6) * Workspace::padded(n) + 2 * Workspace::padded(ntr) +
-                         Workspace::padded(ndot) + Workspace::padded(nsum)));
+  Workspace ws(c);
+  AHIP(c, ws.open((dJdmu ? 7 : 6) * Workspace::padded(n) + 2 * Workspace::padded(ntr) +
+                  Workspace::padded(ndot) + Workspace::padded(nsum)));
   double *lam = ws.take(n), *lk = ws.take(n), *acur = ws.take(n), *asum = ws.take(n);
   double *final_state = ws.take(n), *pvol = ws.take(n), *f0 = dJdmu ? ws.take(n) : nullptr;
   double *aown = ws.take(ntr), *anbr = ws.take(ntr), *dpart = ws.take(ndot), *dsum = ws.take(nsum);
@@ -348,9 +313,13 @@ static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t i
       return nullptr;
     if (c->adj_store && c->adj_store_bytes >= need)
       return c->adj_store;
-    size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) != hipSuccess ||
-        (double)need > 0.75 * ((double)fr + (double)c->adj_store_bytes))
+    auto fits = [&]() {
+      OnDevice on(c->device);
+      size_t fr = 0, tot = 0;
+      return hipMemGetInfo(&fr, &tot) == hipSuccess &&
+             (double)need <= 0.75 * ((double)fr + (double)c->adj_store_bytes);
+    };
+    if (!fits() && !(pool_reclaim(c->device) && fits()))
       return nullptr;
     if (hipStreamSynchronize(c->stream) != hipSuccess)
       return nullptr;
@@ -359,11 +328,8 @@ static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t i
     c->adj_store       = nullptr;
     c->adj_store_bytes = 0;
     double* p          = nullptr;
-    if (hipMalloc(&p, need) != hipSuccess)
-    {
-      (void)hipGetLastError();  // fall back to the next schedule
-      return nullptr;
-    }
+    if (pool_malloc((void**)&p, need, c->device) != hipSuccess)
+      return nullptr;  // fall back to the next schedule
     c->adj_store       = p;
     c->adj_store_bytes = need;
     return p;
@@ -426,7 +392,7 @@ static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t i
   const uint64_t nchk = store_all ? 0 : (nsteps + K - 1) / K;
   std::vector<DevBuf> chk(nchk);
   for (auto& b : chk)
-    AHIP(c, alloc(b, n));
+    AHIP(c, alloc(c, b, n));
   bool seg_store = false;
   if (!store_all)
   {
@@ -556,13 +522,13 @@ static dgx_status adjoint_rk4(dgx_ctx* c, double dt, uint64_t nsteps, uint64_t i
     // the stage states S0..S3 with their records and rhs k1..k4, reverse it
     std::vector<DevBuf> seg(K);
     for (auto& b : seg)
-      AHIP(c, alloc(b, n));
+      AHIP(c, alloc(c, b, n));
     DevBuf S[4], T[4], kf[4];
     for (int i = 0; i < 4; ++i)
     {
-      AHIP(c, alloc(S[i], n));
-      AHIP(c, alloc(T[i], ntr));
-      AHIP(c, alloc(kf[i], n));
+      AHIP(c, alloc(c, S[i], n));
+      AHIP(c, alloc(c, T[i], ntr));
+      AHIP(c, alloc(c, kf[i], n));
     }
     double* const Si[4] = {S[0].p, S[1].p, S[2].p, S[3].p};
     double* const Ti[4] = {T[0].p, T[1].p, T[2].p, T[3].p};
@@ -662,16 +628,14 @@ dgx_status dgx_adjoint_release(dgx_ctx* c)
 {
   if (!c)
     return DGX_ERR_INVALID;
-  if (c->adj_store || c->adj_ws)
-    AHIP(c, hipStreamSynchronize(c->stream));
   if (c->adj_store)
+  {
+    AHIP(c, hipStreamSynchronize(c->stream));
     AHIP(c, hipFree(c->adj_store));
+  }
   c->adj_store       = nullptr;
   c->adj_store_bytes = 0;
-  if (c->adj_ws)
-    AHIP(c, hipFree(c->adj_ws));
-  c->adj_ws       = nullptr;
-  c->adj_ws_bytes = 0;
+  workspace_release(c);
   return DGX_OK;
 }
 

@@ -18,6 +18,7 @@
 #include "../../include/dgx.h"
 #include "dgx_ctx.hpp"
 #include "dgx_launch.hpp"
+#include "dgx_pool.hpp"
 
 using namespace dgx;
 
@@ -289,6 +290,8 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   size_t nn = (size_t)c->nelem * (c->q + 1) * (c->q + 1) * (c->q + 1) * 3;
   c->npartial = resid_out_blocks(c->p, c->q, c->nelem);
 
+  pool_add(c);
+  auto alloc = [dev](auto** p, size_t bytes) { return pool_malloc((void**)p, bytes, dev); };
   auto bail = [&](const char* what, hipError_t e) {
     snprintf(g_create_err, sizeof(g_create_err), "%s failed: %s", what, hipGetErrorString(e));
     dgx_destroy(c);
@@ -300,24 +303,24 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   size_t sb = c->nstate * sizeof(double);
   double** bufs[5] = {&c->U, &c->Ua, &c->Ub, &c->acc, &c->fs};
   for (int i = 0; i < 5; ++i)
-    if ((e = hipMalloc(bufs[i], sb)) != hipSuccess)
+    if ((e = alloc(bufs[i], sb)) != hipSuccess)
       return bail("hipMalloc(state)", e);
-  if ((e = hipMalloc(&c->nodes, nn * sizeof(double))) != hipSuccess)
+  if ((e = alloc(&c->nodes, nn * sizeof(double))) != hipSuccess)
     return bail("hipMalloc(nodes)", e);
-  if ((e = hipMalloc(&c->partial, ((size_t)c->npartial + sum_scratch(c->npartial)) *
+  if ((e = alloc(&c->partial, ((size_t)c->npartial + sum_scratch(c->npartial)) *
                                        sizeof(double))) != hipSuccess)
     return bail("hipMalloc(partial)", e);
-  if ((e = hipMalloc(&c->sum, sizeof(double))) != hipSuccess)
+  if ((e = alloc(&c->sum, sizeof(double))) != hipSuccess)
     return bail("hipMalloc(sum)", e);
   size_t nlam = (size_t)c->nelem * 6 * (c->p + 1) * (c->p + 1);
-  if ((e = hipMalloc(&c->lam, nlam * sizeof(double))) != hipSuccess)
+  if ((e = alloc(&c->lam, nlam * sizeof(double))) != hipSuccess)
     return bail("hipMalloc(lam)", e);
-  if ((e = hipMalloc(&c->status, sizeof(int))) != hipSuccess)
+  if ((e = alloc(&c->status, sizeof(int))) != hipSuccess)
     return bail("hipMalloc(status)", e);
   size_t tb = trace_doubles(c->p, c->nx, c->ny, c->nz) * sizeof(double);
   double** tbufs[3] = {&c->TU, &c->TUa, &c->TUb};
   for (int i = 0; i < 3; ++i)
-    if ((e = hipMalloc(tbufs[i], tb)) != hipSuccess)
+    if ((e = alloc(tbufs[i], tb)) != hipSuccess)
       return bail("hipMalloc(traces)", e);
   drop_traces(c);
   c->prec    = DGX_PREC_FP64;
@@ -335,11 +338,11 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
     return bail("lifting coefficients", e);
   if (c->affine)
   {
-    if ((e = hipMalloc(&c->lamf, (size_t)c->nelem * 6 * sizeof(double))) != hipSuccess)
+    if ((e = alloc(&c->lamf, (size_t)c->nelem * 6 * sizeof(double))) != hipSuccess)
       return bail("hipMalloc(lamf)", e);
     if ((e = lift_face_dispatch(c->p, c->lam, c->nelem, c->lamf, c->stream)) != hipSuccess)
       return bail("face lifting coefficients", e);
-    if ((e = hipMalloc(&c->arec, affine_record_doubles(c->nelem) * sizeof(double))) != hipSuccess)
+    if ((e = alloc(&c->arec, affine_record_doubles(c->nelem) * sizeof(double))) != hipSuccess)
       return bail("hipMalloc(arec)", e);
     if ((e = affine_record_dispatch(c->nodes, c->nelem, c->arec, c->stream)) != hipSuccess)
       return bail("affine records", e);
@@ -397,6 +400,7 @@ dgx_status dgx_destroy(dgx_ctx* c)
 {
   if (!c)
     return DGX_OK;
+  pool_remove(c);
   if (c->stream)
     (void)hipStreamSynchronize(c->stream);
   double* bufs[16] = {c->U,   c->Ua,   c->Ub,   c->acc, c->fs, c->nodes, c->partial, c->sum,
@@ -944,7 +948,7 @@ dgx_status dgx_sample_output(dgx_ctx* c, int var, int N, double* out_host)
     return DGX_ERR_INVALID;
   size_t n = (size_t)c->nelem * (N + 1) * (N + 1) * (N + 1);
   double* d = nullptr;
-  HIPCHK(c, hipMalloc(&d, n * sizeof(double)));
+  HIPCHK(c, pool_malloc((void**)&d, n * sizeof(double), c->device));
   hipError_t e = sample_dispatch(c->p, c->U, c->nelem, N, var, c->params.gamma, d, c->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(out_host, d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
@@ -963,7 +967,7 @@ dgx_status dgx_update_mean(dgx_ctx* c, uint64_t time_step, uint64_t mean_start)
   size_t sb = c->nstate * sizeof(double);
   if (!c->mean)
   {
-    HIPCHK(c, hipMalloc(&c->mean, sb));
+    HIPCHK(c, pool_malloc((void**)&c->mean, sb, c->device));
     c->bytes += sb;
     HIPCHK(c, hipMemsetAsync(c->mean, 0, sb, c->stream));
   }
@@ -982,7 +986,7 @@ dgx_status dgx_set_mean(dgx_ctx* c, const double* mean_host)
   size_t sb = c->nstate * sizeof(double);
   if (!c->mean)
   {
-    HIPCHK(c, hipMalloc(&c->mean, sb));
+    HIPCHK(c, pool_malloc((void**)&c->mean, sb, c->device));
     c->bytes += sb;
   }
   HIPCHK(c, hipMemcpyAsync(c->Ua, mean_host, sb, hipMemcpyHostToDevice, c->stream));

@@ -48,6 +48,7 @@ struct dgx_ctx
   size_t adj_store_limit;  // most bytes that store may take (0: no limit)
   double* adj_ws;          // workspace of the adjoint calls, kept likewise
   size_t adj_ws_bytes;
+  int adj_busy;            // the workspace is in use (see dgx_pool.hpp)
   int* status;      // kernel-side error flags
   int npartial;
   size_t bytes;

@@ -33,6 +33,7 @@
 #include "../../include/dgx.h"
 #include "dgx_ctx.hpp"
 #include "dgx_launch.hpp"
+#include "dgx_pool.hpp"
 
 using namespace dgx;
 
@@ -331,9 +332,10 @@ dgx_status dgx_ensemble_create(int ncase, const dgx_mesh* meshes, const dgx_para
     return bail("hipStreamCreate", e);
   for (EnsGroup& g : en->groups)
     for (int s = 0; s < 4; ++s)
-      if ((e = hipMalloc(&g.items[s], sizeof(BatchItem) * g.members.size())) != hipSuccess)
+      if ((e = pool_malloc((void**)&g.items[s], sizeof(BatchItem) * g.members.size(),
+                           en->device)) != hipSuccess)
         return bail("hipMalloc(items)", e);
-  if ((e = hipMalloc(&en->status, sizeof(int))) != hipSuccess)
+  if ((e = pool_malloc((void**)&en->status, sizeof(int), en->device)) != hipSuccess)
     return bail("hipMalloc(status)", e);
   if ((e = hipMemsetAsync(en->status, 0, sizeof(int), en->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);

@@ -331,7 +331,9 @@ dgx_status dgx_adjoint_rk4_device(dgx_ctx* ctx, double dt, uint64_t nsteps, uint
 /* Frees what the adjoint calls keep on the context: the stored-stage buffer
  * of dgx_adjoint_rk4 and the workspace (3 to 7 states and 2 trace-record sets)
  * of dgx_adjoint_rk4 and dgx_residual_vjp (no counterpart in the reference,
- * which has no adjoint).  No-op when none is held. */
+ * which has no adjoint).  A workspace of more than 1 GiB is not kept, and one
+ * that no call is using is freed when the library cannot allocate otherwise.
+ * No-op when none is held. */
 dgx_status dgx_adjoint_release(dgx_ctx* ctx);
 /* Caps the stored-stage buffer of dgx_adjoint_rk4 at `bytes` (0: no cap
  * beyond three quarters of the free device memory; no counterpart in the

@@ -1,0 +1,47 @@
+"""Device memory that contexts keep and can do without (dgx_pool.cpp), on the
+CPU against a stand-in for the HIP runtime (tests/cpu/pool_check.cpp), and
+overlapping adjoint calls on one solver on the GPU."""
+import os
+import subprocess
+import threading
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_pool(tmp_path):
+    exe = str(tmp_path / "pool_check")
+    csrc = os.path.join(ROOT, "dgpr_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread",
+                    "-I" + os.path.join(ROOT, "tests", "cpu", "pool"), "-I" + csrc,
+                    "-I" + os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "cpu", "pool_check.cpp"),
+                    os.path.join(csrc, "dgx_pool.cpp"), "-o", exe], check=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_overlapping_products_of_one_solver():
+    """Vector-Jacobian products of four threads on one solver: each its own."""
+    from dgpr_amd import cases, dgx
+    c = cases.channel_case(6, 5, 4, p=2, seed=3, nsteps=1)
+    w = [np.random.default_rng(t).standard_normal(c.U0.size) for t in range(4)]
+    with dgx.Solver(c.mesh, c.params) as s:
+        s.set_state(c.U0)
+        ref = [s.residual_vjp(x) for x in w]
+        bad = []
+
+        def work(t):
+            for _ in range(20):
+                if not np.array_equal(s.residual_vjp(w[t]), ref[t]):
+                    bad.append(t)
+
+        threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad
