@@ -107,9 +107,9 @@ static void derive_phys(const dgx_params& p, Phys& ph)
   }
 }
 
-MeshArgs dgx::mesh_args(const dgx_ctx* c)
+dgx::MeshLease dgx::mesh_args(const dgx_ctx* c)
 {
-  MeshArgs m;
+  MeshArgs m{};
   m.nodes = c->nodes;
   m.nx = c->nx;
   m.ny = c->ny;
@@ -121,9 +121,7 @@ MeshArgs dgx::mesh_args(const dgx_ctx* c)
   m.matched = c->matched;
   m.lamf   = c->lamf;
   m.arec   = c->arec;
-  m.geov   = c->geo;
-  m.geof   = c->geo ? c->geo + (size_t)c->nelem * GEOV * c->nbf : nullptr;
-  return m;
+  return MeshLease(m, const_cast<dgx_ctx*>(c));
 }
 
 // True when q = 1 and every element's bilinear and trilinear node terms
@@ -197,6 +195,40 @@ static dgx_status ensure_tables(int device)
     return fail(nullptr, DGX_ERR_HIP, "table upload failed: %s", hipGetErrorString(e));
   g_tab_devices.push_back(device);
   return DGX_OK;
+}
+
+// Curved geometry of the q > 1 and general orders is stored once (80 bytes per
+// Gauss node and 104 per face point) where there is room for it; otherwise every
+// stage evaluates it from the nodes.
+static bool stores_geometry(const dgx_ctx* c)
+{
+  return !c->affine && (c->q > 1 || general_order(c->p, c->q));
+}
+
+static size_t geometry_bytes(const dgx_ctx* c)
+{
+  const size_t nf = (size_t)(c->p + 1) * (c->p + 1);
+  return (size_t)c->nelem * (GEOV * c->nbf + 6 * GEOF * nf) * sizeof(double);
+}
+
+static hipError_t store_geometry(dgx_ctx* c)
+{
+  OnDevice on(c->device);
+  hipError_t e = hipMalloc(&c->geo, geometry_bytes(c));
+  if (e != hipSuccess)
+  {
+    (void)hipGetLastError();
+    c->geo = nullptr;
+    return e;
+  }
+  c->geo_bytes = geometry_bytes(c);
+  if ((e = geometry_dispatch(c->p, c->q, mesh_args(c), c->geo,
+                             c->geo + (size_t)c->nelem * GEOV * c->nbf, c->stream)) != hipSuccess)
+    return e;
+  // launches of other streams (an ensemble's) may follow
+  if ((e = hipStreamSynchronize(c->stream)) == hipSuccess)
+    __atomic_store_n(&c->geo_users, 0, __ATOMIC_RELEASE);
+  return e;
 }
 
 extern "C" {
@@ -274,6 +306,7 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   dgx_ctx* c = new dgx_ctx();
   memset(c, 0, sizeof(*c));
   c->device = dev;
+  c->geo_users = -1;
   c->p = (int)mesh->p;
   c->q = (int)mesh->q;
   c->affine = mesh_is_affine(mesh) ? 1 : 0;
@@ -325,10 +358,6 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   drop_traces(c);
   c->prec    = DGX_PREC_FP64;
   c->matched = 1;
-  c->bytes = 5 * sb + 3 * tb +
-             (nn + nlam +
-              (c->affine ? (size_t)c->nelem * 6 + affine_record_doubles(c->nelem) : 0) + (size_t)c->npartial +
-              sum_scratch(c->npartial)) * sizeof(double) + 16;
   if ((e = hipMemcpyAsync(c->nodes, mesh->nodes, nn * sizeof(double), hipMemcpyHostToDevice,
                           c->stream)) != hipSuccess)
     return bail("hipMemcpy(nodes)", e);
@@ -342,36 +371,31 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
       return bail("hipMalloc(lamf)", e);
     if ((e = lift_face_dispatch(c->p, c->lam, c->nelem, c->lamf, c->stream)) != hipSuccess)
       return bail("face lifting coefficients", e);
-    if ((e = alloc(&c->arec, affine_record_doubles(c->nelem) * sizeof(double))) != hipSuccess)
-      return bail("hipMalloc(arec)", e);
-    if ((e = affine_record_dispatch(c->nodes, c->nelem, c->arec, c->stream)) != hipSuccess)
-      return bail("affine records", e);
-  }
-  // curved geometry of the q > 1 and general orders is stored once (80 bytes
-  // per Gauss node and 104 per face point) where it takes at most a quarter of
-  // the free memory, so that no mesh that fitted without it is refused;
-  // otherwise every stage evaluates it from the nodes
-  if (!c->affine && (c->q > 1 || general_order(c->p, c->q)))
-  {
-    const size_t nf = (size_t)(c->p + 1) * (c->p + 1);
-    const size_t gb = (size_t)c->nelem * (GEOV * c->nbf + 6 * GEOF * nf) * sizeof(double);
-    size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess && gb <= fr / 4)
+    if (alloc(&c->arec, affine_record_doubles(c->nelem) * sizeof(double)) == hipSuccess)
     {
-      if (hipMalloc(&c->geo, gb) != hipSuccess)
-      {
-        (void)hipGetLastError();
-        c->geo = nullptr;
-      }
-      else
-      {
-        const MeshArgs ma = mesh_args(c);
-        if ((e = geometry_dispatch(c->p, c->q, ma, c->geo, const_cast<double*>(ma.geof),
-                                   c->stream)) != hipSuccess)
-          return bail("stored geometry", e);
-        c->bytes += gb;
-      }
+      if ((e = affine_record_dispatch(c->nodes, c->nelem, c->arec, c->stream)) != hipSuccess)
+        return bail("affine records", e);
     }
+    else
+    {
+      // no room for the records: the kernels of curved elements do without
+      (void)hipFree(c->lamf);
+      c->lamf   = nullptr;
+      c->affine = 0;
+    }
+  }
+  c->bytes = 5 * sb + 3 * tb +
+             (nn + nlam +
+              (c->affine ? (size_t)c->nelem * 6 + affine_record_doubles(c->nelem) : 0) + (size_t)c->npartial +
+              sum_scratch(c->npartial)) * sizeof(double) + 16;
+  // stored where it takes at most a quarter of the free memory; what later
+  // needs the room gets it back (pool_reclaim)
+  if (stores_geometry(c))
+  {
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && geometry_bytes(c) <= fr / 4 &&
+        (e = store_geometry(c)) != hipSuccess && e != hipErrorOutOfMemory)
+      return bail("stored geometry", e);
   }
   if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);
@@ -439,7 +463,7 @@ dgx_status dgx_get_sizes(const dgx_ctx* c, uint64_t out[4])
   out[0] = (uint64_t)c->nelem;
   out[1] = (uint64_t)c->nbf;
   out[2] = (uint64_t)c->nstate;
-  out[3] = (uint64_t)c->bytes;
+  out[3] = (uint64_t)(c->bytes + c->geo_bytes);
   return DGX_OK;
 }
 
@@ -801,6 +825,40 @@ dgx_status dgx_set_tile(dgx_ctx* c, int tile)
   apply_defaults(c);
   if (!tile_valid(c->p, c->q, tile, c->stage_waves))
     c->stage_waves = 2;  // the tiled kernels are compiled for 2 and 3 waves per SIMD
+  return DGX_OK;
+}
+
+dgx_status dgx_set_stored_geometry(dgx_ctx* c, int on)
+{
+  if (!c)
+    return DGX_ERR_INVALID;
+  if (!on)
+  {
+    if (c->geo && !geometry_release(c))
+      return fail(c, DGX_ERR_INVALID, "the stored geometry is in use by a call, a captured graph "
+                                      "or an ensemble");
+    return DGX_OK;
+  }
+  if (c->geo)
+    return DGX_OK;
+  if (!stores_geometry(c))
+    return fail(c, DGX_ERR_UNSUPPORTED, "no geometry is stored for affine meshes and for q = 1 at "
+                                        "p = 1 to 3");
+  const hipError_t e = store_geometry(c);
+  if (e == hipSuccess)
+    return DGX_OK;
+  if (c->geo)
+    (void)hipFree(c->geo);
+  c->geo       = nullptr;
+  c->geo_bytes = 0;
+  return fail(c, DGX_ERR_HIP, "stored geometry: %s", hipGetErrorString(e));
+}
+
+dgx_status dgx_get_stored_geometry(const dgx_ctx* c, int* on)
+{
+  if (!c || !on)
+    return DGX_ERR_INVALID;
+  *on = c->geo != nullptr;
   return DGX_OK;
 }
 

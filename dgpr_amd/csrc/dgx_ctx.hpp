@@ -31,6 +31,8 @@ struct dgx_ctx
   double* lamf;     // affine meshes: one coefficient per element face [e][6]
   double* arec;     // affine meshes: each element's constant geometry
   double* geo;      // stored geometry (geov, then geof), or null
+  size_t geo_bytes;
+  int geo_users;    // launches and graphs that read geo; -1: none is to be read
   double* TU;       // face trace records of U, Ua, Ub [e][6][8][(p+1)^2]
   double* TUa;
   double* TUb;
@@ -58,7 +60,6 @@ struct dgx_ctx
 namespace dgx
 {
 // MeshArgs of the context's mesh
-MeshArgs mesh_args(const dgx_ctx* c);
 // trace records of U, recomputed when U was set from outside
 hipError_t ensure_traces(dgx_ctx* c);
 // what a stage of the context's kernel reads besides U: the boundary states

@@ -152,7 +152,14 @@ static dgx_status plan(dgx_ensemble* en, int scheme, const double* dt)
       for (int s = 0; s < ns; ++s)
       {
         BatchItem it;
-        it.mesh = mesh_args(c);
+        // (the table outlives the launch; the batched kernels read no stored geometry)
+        if (g.general)
+          it.mesh = mesh_args(c).keep();
+        else
+        {
+          it.mesh = mesh_args(c);
+          it.mesh.geov = it.mesh.geof = nullptr;
+        }
         it.ph = c->phys;
         it.sa = sa[s];
         it.sa.records = !(g.unit_grid && g.tile == 1);

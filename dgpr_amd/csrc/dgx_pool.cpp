@@ -69,11 +69,16 @@ bool pool_reclaim(int device)
   std::lock_guard<std::mutex> lk(g_mutex);
   bool any = false;
   for (dgx_ctx* c : g_contexts)
-    if (c->device == device && claim(&c->adj_busy))
+  {
+    if (c->device != device)
+      continue;
+    if (claim(&c->adj_busy))
     {
       any = free_workspace(c) || any;
       unclaim(&c->adj_busy);
     }
+    any = geometry_release(c) || any;
+  }
   return any;
 }
 
@@ -130,6 +135,48 @@ Workspace::~Workspace()
       free_workspace(c_);
     unclaim(&c_->adj_busy);
   }
+}
+
+MeshLease::MeshLease(const MeshArgs& m, dgx_ctx* c) : MeshArgs(m), c_(nullptr)
+{
+  geov = geof = nullptr;
+  int n = __atomic_load_n(&c->geo_users, __ATOMIC_RELAXED);
+  while (n >= 0 && !__atomic_compare_exchange_n(&c->geo_users, &n, n + 1, true, __ATOMIC_ACQUIRE,
+                                                __ATOMIC_RELAXED))
+    ;
+  if (n < 0)
+    return;
+  geov = c->geo;
+  geof = c->geo + (size_t)c->nelem * GEOV * c->nbf;
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &s) == hipSuccess && s == hipStreamCaptureStatusNone)
+    c_ = c;
+}
+
+MeshLease::~MeshLease()
+{
+  if (c_)
+    __atomic_fetch_sub(&c_->geo_users, 1, __ATOMIC_RELEASE);
+}
+
+bool geometry_release(dgx_ctx* c)
+{
+  int idle = 0;
+  if (!__atomic_compare_exchange_n(&c->geo_users, &idle, -1, false, __ATOMIC_ACQUIRE,
+                                   __ATOMIC_RELAXED))
+    return false;
+  OnDevice on(c->device);
+  // kernels of returned calls may still read it, on any stream
+  if (hipDeviceSynchronize() != hipSuccess)
+  {
+    (void)hipGetLastError();
+    __atomic_store_n(&c->geo_users, 0, __ATOMIC_RELEASE);
+    return false;
+  }
+  (void)hipFree(c->geo);
+  c->geo       = nullptr;
+  c->geo_bytes = 0;
+  return true;
 }
 
 void workspace_release(dgx_ctx* c)

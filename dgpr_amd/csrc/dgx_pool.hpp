@@ -1,7 +1,7 @@
 // dgx_pool.hpp -- device memory that a context keeps to be faster and can do
-// without: the workspace of the adjoint calls.  What an idle context holds of
-// it is freed when an allocation of the library fails, so that whatever fits
-// into the device's memory without it still does.
+// without: the workspace of the adjoint calls and the stored geometry.  What no
+// call is using of it is freed when an allocation of the library fails, so that
+// whatever fits into the device's memory without it still does.
 #pragma once
 
 #include "dgx_ctx.hpp"
@@ -63,5 +63,30 @@ class Workspace
 
 // Frees the context's workspace unless a call is using it.
 void workspace_release(dgx_ctx* c);
+
+// The context's mesh for one launch.  While it exists the stored geometry that
+// it points to is not freed; a launch recorded into a graph (the context's
+// stream is being captured), and keep(), hold it as long as the context lives.
+class MeshLease : public MeshArgs
+{
+ public:
+  MeshLease(const MeshArgs& m, dgx_ctx* c);
+  ~MeshLease();
+  MeshLease(const MeshLease&) = delete;
+  MeshLease& operator=(const MeshLease&) = delete;
+  MeshArgs keep()
+  {
+    c_ = nullptr;
+    return *this;
+  }
+
+ private:
+  dgx_ctx* c_;  // whose geometry goes back at the end
+};
+MeshLease mesh_args(const dgx_ctx* c);
+
+// Frees the context's stored geometry unless a launch or a graph may read it;
+// whether it did.
+bool geometry_release(dgx_ctx* c);
 
 }  // namespace dgx

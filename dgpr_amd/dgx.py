@@ -154,6 +154,8 @@ def lib():
         L.dgx_set_tile.argtypes = [P_ctx, C.c_int]
         L.dgx_get_tile.argtypes = [P_ctx, C.POINTER(C.c_int)]
         L.dgx_faces_match.argtypes = [P_ctx, C.POINTER(C.c_int)]
+        L.dgx_set_stored_geometry.argtypes = [P_ctx, C.c_int]
+        L.dgx_get_stored_geometry.argtypes = [P_ctx, C.POINTER(C.c_int)]
         L.dgx_autotune_tiles.argtypes = [P_ctx, C.c_int, C.POINTER(C.c_int),
                                          C.POINTER(C.c_int), PD]
         for nm in ("dgx_create", "dgx_destroy", "dgx_set_params", "dgx_set_state",
@@ -167,6 +169,7 @@ def lib():
                    "dgx_mesh_is_affine",
                    "dgx_get_tuning", "dgx_autotune", "dgx_set_precision", "dgx_get_precision",
                    "dgx_set_tile", "dgx_get_tile", "dgx_faces_match", "dgx_autotune_tiles",
+                   "dgx_set_stored_geometry", "dgx_get_stored_geometry",
                    "dgx_sample_output",
                    "dgx_sample_output_device", "dgx_update_mean", "dgx_get_mean",
                    "dgx_set_mean", "dgx_write_dg_outputs", "dgx_read_dg_output_key",
@@ -569,6 +572,19 @@ class Solver:
             return "dgx_tile_stage_kernel<%d,%d,%d,%d>" % (self.mesh.p, self.mesh.q,
                                                            self.TILE_ROWS[self.mesh.p], w)
         return "dgx_rhs_stage_kernel<%d,%d,%d>" % (self.mesh.p, self.mesh.q, w)
+
+    @property
+    def stored_geometry(self):
+        """Whether the context keeps the geometry of a curved mesh of q > 1 or of
+        an order outside 1 <= p <= 3; set False to free it, True to store it again
+        (dgx_set_stored_geometry)."""
+        on = C.c_int()
+        _chk(lib().dgx_get_stored_geometry(self.ctx, C.byref(on)), self.ctx)
+        return bool(on.value)
+
+    @stored_geometry.setter
+    def stored_geometry(self, on):
+        _chk(lib().dgx_set_stored_geometry(self.ctx, int(bool(on))), self.ctx)
 
     @property
     def faces_match(self):

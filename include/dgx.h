@@ -410,6 +410,17 @@ dgx_status dgx_autotune(dgx_ctx* ctx, int reps, int* chosen, double us_out[3]);
  * Results agree to rounding. */
 dgx_status dgx_set_tile(dgx_ctx* ctx, int tile);
 dgx_status dgx_get_tile(const dgx_ctx* ctx, int* tile);
+/* Stored geometry of curved meshes of q > 1 and of the orders outside 1 <= p <= 3
+ * (no counterpart in the reference, whose metrics are always stored): inverse
+ * Jacobians, normals and surface elements at every node and face point, 80 and 104
+ * bytes each, which the stages read instead of evaluating the geometry basis
+ * (1.7 to 2.8 times as long at q = 2).  dgx_create stores them where they take at most a
+ * quarter of the free memory; an allocation of the library that would fail frees
+ * those that no launch or captured graph may read.  on = 0 frees them for other
+ * uses of the memory, on = 1 stores them again (DGX_ERR_HIP without the room,
+ * DGX_ERR_UNSUPPORTED on other meshes).  Results agree to rounding. */
+dgx_status dgx_set_stored_geometry(dgx_ctx* ctx, int on);
+dgx_status dgx_get_stored_geometry(const dgx_ctx* ctx, int* on);
 /* Whether at every face between two elements, periodic ones included, both
  * elements have the same face up to a translation, to 8 ulps of its largest
  * coordinate (q = 1; 1 for q > 1, where it decides nothing; no counterpart in

@@ -37,6 +37,14 @@ inline hipError_t hipSetDevice(int d)
   return hipSuccess;
 }
 inline hipError_t hipGetLastError() { return hipSuccess; }
+// every stream is being captured while this is set
+inline bool g_capturing = false;
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone, hipStreamCaptureStatusActive };
+inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
+{
+  *s = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n)
@@ -60,5 +68,64 @@ inline hipError_t hipFree(void* p)
   g_hip.blocks.erase(it);
   std::free(p);
   ++g_hip.frees;
+  return hipSuccess;
+}
+template <typename T>
+hipError_t hipMalloc(T** p, size_t n)
+{
+  return hipMalloc((void**)p, n);
+}
+
+// the rest of what dgx_api.cpp calls: streams do nothing, copies are immediate
+#include <cstring>
+typedef int* hipEvent_t;
+enum hipMemcpyKind
+{
+  hipMemcpyHostToDevice,
+  hipMemcpyDeviceToHost,
+  hipMemcpyDeviceToDevice,
+  hipMemcpyDefault
+};
+constexpr unsigned hipStreamNonBlocking = 1;
+inline const char* hipGetErrorString(hipError_t e)
+{
+  return e == hipErrorOutOfMemory ? "out of memory" : "error";
+}
+inline hipError_t hipGetDeviceCount(int* n)
+{
+  *n = 2;
+  return hipSuccess;
+}
+inline hipError_t hipMemGetInfo(size_t* free, size_t* total)
+{
+  std::lock_guard<std::mutex> lk(g_hip.mx);
+  *total = g_hip.capacity[t_device];
+  *free  = *total - g_hip.used[t_device];
+  return hipSuccess;
+}
+inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
+{
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t)
+{
+  return hipMemcpy(d, s, n, k);
+}
+inline hipError_t hipMemset(void* d, int v, size_t n)
+{
+  std::memset(d, v, n);
+  return hipSuccess;
+}
+inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
+inline hipError_t hipStreamCreateWithFlags(hipStream_t*, unsigned) { return hipSuccess; }
+inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+inline hipError_t hipEventCreate(hipEvent_t*) { return hipSuccess; }
+inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t)
+{
+  *t = 1.0f;
   return hipSuccess;
 }

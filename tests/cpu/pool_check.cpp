@@ -2,7 +2,8 @@
 // runtime with two devices of limited memory: the adjoint's workspace is kept
 // and grown on the context's own device, is not shared by calls that overlap, is
 // given back when another allocation needs the room, and is not kept above its
-// bound.
+// bound; the stored geometry is given back likewise, but not under a launch, a
+// captured one or a table that keeps it.
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -27,7 +28,8 @@ static dgx_ctx* context(int device)
 {
   dgx_ctx* c = new dgx_ctx();
   std::memset(c, 0, sizeof(*c));
-  c->device = device;
+  c->device    = device;
+  c->geo_users = -1;
   pool_add(c);
   return c;
 }
@@ -37,6 +39,86 @@ static void destroy(dgx_ctx* c)
   pool_remove(c);
   workspace_release(c);
   delete c;
+}
+
+static void store(dgx_ctx* c, size_t bytes)
+{
+  CHECK(hipMalloc((void**)&c->geo, bytes) == hipSuccess);
+  c->geo_bytes = bytes;
+  c->nelem = c->nbf = 1;
+  __atomic_store_n(&c->geo_users, 0, __ATOMIC_RELEASE);
+}
+
+static void geometry()
+{
+  g_hip.capacity[0] = (size_t)100 << 20;
+  dgx_ctx *a = context(0), *b = context(0);
+  {
+    MeshLease m(MeshArgs{}, b);  // nothing stored
+    CHECK(!m.geov && !m.geof && b->geo_users == -1);
+  }
+  store(a, (size_t)30 << 20);
+  store(b, (size_t)30 << 20);
+  void* p = nullptr;
+  {
+    MeshLease m(MeshArgs{}, a);
+    CHECK(m.geov == a->geo && m.geof == a->geo + GEOV);
+    CHECK(pool_malloc(&p, (size_t)60 << 20, 0) == hipSuccess);  // b's goes, a's is being read
+    CHECK(a->geo && !b->geo && b->geo_users == -1 && b->geo_bytes == 0);
+    CHECK(!geometry_release(a));
+    MeshLease n(MeshArgs{}, b);
+    CHECK(!n.geov && !n.geof);
+    hipFree(p);
+  }
+  CHECK(a->geo_users == 0 && geometry_release(a) && !a->geo && !geometry_release(a));
+
+  // recorded into a graph, or kept in a table: held for good
+  for (int k = 0; k < 2; ++k)
+  {
+    dgx_ctx* c = context(0);
+    store(c, (size_t)30 << 20);
+    MeshArgs kept{};
+    g_capturing = k == 0;
+    {
+      MeshLease m(MeshArgs{}, c);
+      if (k == 1)
+        kept = m.keep();
+    }
+    g_capturing = false;
+    CHECK(k == 0 || kept.geov == c->geo);
+    CHECK(!pool_reclaim(0) && c->geo);
+    hipFree(c->geo);
+    destroy(c);
+  }
+
+  // threads that launch while others need the room
+  store(a, (size_t)1 << 20);
+  std::atomic<int> bad{0};
+  std::atomic<bool> stop{false};
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 4; ++t)
+    ts.emplace_back([&] {
+      while (!stop)
+      {
+        MeshLease m(MeshArgs{}, a);
+        std::lock_guard<std::mutex> lk(g_hip.mx);
+        if (m.geov && !g_hip.blocks.count((void*)m.geov))
+          ++bad;
+      }
+    });
+  for (int it = 0; it < 200; ++it)
+  {
+    while (!geometry_release(a))
+      std::this_thread::yield();
+    store(a, (size_t)1 << 20);
+  }
+  stop = true;
+  for (auto& t : ts)
+    t.join();
+  CHECK(bad == 0 && a->geo_users == 0 && geometry_release(a));
+  destroy(a);
+  destroy(b);
+  CHECK(g_hip.blocks.empty());
 }
 
 int main()
@@ -137,5 +219,7 @@ int main()
   destroy(a);
   destroy(b);
   CHECK(g_hip.blocks.empty() && g_hip.mallocs == g_hip.frees);
+
+  geometry();
   return g_failed ? 1 : 0;
 }

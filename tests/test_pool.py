@@ -1,5 +1,6 @@
 """Device memory that contexts keep and can do without (dgx_pool.cpp), on the
-CPU against a stand-in for the HIP runtime (tests/cpu/pool_check.cpp), and
+CPU against a stand-in for the HIP runtime (tests/cpu/pool_check.cpp, and
+tests/cpu/memory_limit_check.cpp with contexts at the limit of the memory), and
 overlapping adjoint calls on one solver on the GPU."""
 import os
 import subprocess
@@ -11,14 +12,19 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_pool(tmp_path):
-    exe = str(tmp_path / "pool_check")
+@pytest.mark.parametrize("program, sources", [
+    ("pool_check", ["dgx_pool"]),
+    ("memory_limit_check", ["dgx_pool", "dgx_api", "dgx_tables", "dgx_host"]),
+])
+def test_on_the_cpu(program, sources, tmp_path):
+    exe = str(tmp_path / program)
     csrc = os.path.join(ROOT, "dgpr_amd", "csrc")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread",
                     "-I" + os.path.join(ROOT, "tests", "cpu", "pool"), "-I" + csrc,
                     "-I" + os.path.join(ROOT, "include"),
-                    os.path.join(ROOT, "tests", "cpu", "pool_check.cpp"),
-                    os.path.join(csrc, "dgx_pool.cpp"), "-o", exe], check=True, timeout=300)
+                    os.path.join(ROOT, "tests", "cpu", program + ".cpp")]
+                   + [os.path.join(csrc, s + ".cpp") for s in sources] + ["-o", exe],
+                   check=True, timeout=300)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
 
