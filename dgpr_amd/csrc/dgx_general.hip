@@ -725,24 +725,27 @@ __device__ __forceinline__ void gen_apply_dir(double (*s)[N * N * N], const doub
   __syncthreads();
 }
 
-// Basis conversions of one element per workgroup (modes as dgx_basis_kernel:
+// Basis conversions of a workgroup's EPB elements (modes as dgx_basis_kernel:
 // 0 V = B3 U, 1 U = B3^-1 V, 2 G = B3^T g, 3 g = B3^-T G), in double-double.
 // MIX: by dd_fma.  The coefficients in LDS: 20^3 p = 5 116 -> 86 us, 19x13x17
 // p = 4 35 -> 27 us against lane-dependent loads from the tables.
+// Of p <= 2 as many elements as fill a wavefront: with one, whose lanes are then
+// mostly idle, a 64^3 p = 1 conversion of the mixed forms took 234 us instead of 49,
+// a 48^3 p = 2 one 147 instead of 90.
 template <int P, bool MIX>
 __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const double* in, double* out,
-                                                                    int mode)
+                                                                    int nelem, int mode)
 {
-  constexpr int N = P + 1, NB = N * N * N;
+  constexpr int N = P + 1, NB = N * N * N, EPB = GDims<P>::EPB;
   const GenTab& t = g_gtab[P * 8];
-  __shared__ double sh[5][NB];
-  __shared__ double sl[5][NB];
+  __shared__ double sh[5][EPB * NB];
+  __shared__ double sl[5][EPB * NB];
   __shared__ DD sM[N][N];  // coefficient of input m in output i: [m][i]
-  const int node = threadIdx.x;
-  const size_t e = blockIdx.x;
-  const bool act = node < NB;
+  const int tid = threadIdx.x, le = tid / NB, node = tid % NB;
+  const size_t e = (size_t)blockIdx.x * EPB + le;
+  const bool act = le < EPB && e < (size_t)nelem;
   const bool inv = (mode == 1 || mode == 3);
-  for (int x = node; x < N * N; x += GDims<P>::BT)
+  for (int x = tid; x < N * N; x += GDims<P>::BT)
   {
     const int m = x / N, i = x % N, u = (mode >= 2) ? m : i, v = (mode >= 2) ? i : m;
     sM[m][i] = inv ? DD{t.Binv[u][v], t.Binvlo[u][v]} : DD{t.B[u][v], t.Blo[u][v]};
@@ -750,7 +753,7 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
   if (act)
 #pragma unroll
     for (int r = 0; r < 5; ++r)
-      sh[r][node] = in[(e * 5 + r) * NB + node];
+      sh[r][tid] = in[(e * 5 + r) * NB + node];
   __syncthreads();
   const int i0 = node % N, i1 = (node / N) % N, i2 = node / (N * N);
 #pragma unroll
@@ -760,7 +763,8 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
     if (act)
     {
       const int id = pick3i(d, i0, i1, i2);
-      const int b0 = (d == 0) ? nid<N>(0, i1, i2) : ((d == 1) ? nid<N>(i0, 0, i2) : nid<N>(i0, i1, 0));
+      const int b0 = le * NB + ((d == 0) ? nid<N>(0, i1, i2)
+                                         : ((d == 1) ? nid<N>(i0, 0, i2) : nid<N>(i0, i1, 0)));
       constexpr int st[3] = {1, N, N * N};
       auto c = [&](int m) { return sM[m][id]; };
 #pragma unroll
@@ -787,15 +791,15 @@ __global__ __launch_bounds__(GDims<P>::BT) void dgx_gen_basis_kernel(const doubl
 #pragma unroll
       for (int r = 0; r < 5; ++r)
       {
-        sh[r][node] = o[r].hi;
-        sl[r][node] = o[r].lo;
+        sh[r][tid] = o[r].hi;
+        sl[r][tid] = o[r].lo;
       }
     __syncthreads();
   }
   if (act)
 #pragma unroll
     for (int r = 0; r < 5; ++r)
-      out[(e * 5 + r) * NB + node] = sh[r][node] + sl[r][node];
+      out[(e * 5 + r) * NB + node] = sh[r][tid] + sl[r][tid];
 }
 
 // From f_g of the epb elements from blockIdx.x * epb: f = B3^-1 f_g,
@@ -1095,12 +1099,11 @@ template <int P>
 static hipError_t launch_gen_basis(const double* in, double* out, int nelem, int mode, bool mix,
                                    hipStream_t st)
 {
+  const dim3 grid((nelem + GDims<P>::EPB - 1) / GDims<P>::EPB), block(GDims<P>::BT);
   if (mix)
-    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, true>), dim3(nelem), dim3(GDims<P>::BT), 0, st, in,
-                       out, mode);
+    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, true>), grid, block, 0, st, in, out, nelem, mode);
   else
-    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, false>), dim3(nelem), dim3(GDims<P>::BT), 0, st, in,
-                       out, mode);
+    hipLaunchKernelGGL((dgx_gen_basis_kernel<P, false>), grid, block, 0, st, in, out, nelem, mode);
   return hipGetLastError();
 }
 

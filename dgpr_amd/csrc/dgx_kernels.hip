@@ -937,9 +937,11 @@ hipError_t resid_out_dispatch(int p, int q, const MeshArgs& m, const double* fg,
 hipError_t basis_dispatch(int p, const double* in, double* out, int nelem, int mode,
                           hipStream_t st, bool mix)
 {
-  // lines of nodes from one wavefront per SIMD; below that a node per lane is
-  // quicker (2574 elements p = 3: 9.7 against 14.4 us, 512 p = 2: 5.2 against 7.1)
-  const bool lines = !mix && (long)nelem * (p + 1) * (p + 1) >= 64 * 1024;
+  // lines of nodes from 1.5 wavefronts per SIMD (1024 SIMDs), 3 at p = 3; below that a
+  // node per lane is as quick or quicker.  Node against line, with 9 us of the call:
+  // 24^3 p = 1 15.6 / 15.7 us, 30^3 18.0 / 17.5; 20^3 p = 2 19.9 / 20.9, 22^3 22.3 / 21.6, 24^3
+  // 24.4 / 22.8; 17^3 p = 3 23.3 / 26.5, 24^3 38.2 / 38.7, 28^3 50.0 / 48.5, 32^3 63.5 / 58.8
+  const bool lines = !mix && (long)nelem * (p + 1) * (p + 1) >= (p == 3 ? 192 : 96) * 1024;
   switch (lines ? p : 0)
   {
     case 1: return launch_basis<1>(in, out, nelem, mode, st);
