@@ -505,11 +505,22 @@ __host__ __device__ __forceinline__ bool characteristic_bc(int bt) { return bt =
 // non-negative root (the reference aborts there on the host).  T is double
 // in the residual kernels and a dual number in the adjoint's boundary-face
 // kernel (the same expressions, so the double instantiation is unchanged).
-template <typename T>
+// SPLIT: one copy of the short states per code.  Joined, they take the one-row
+// p = 1 kernel from 168 to 177 registers, and so its third wave per SIMD (six 24^3
+// cubes in ensemble units: 195 us per stage joined, 155 split); split, they
+// take the curved p = 2 one from 167 to 169 (30x20x16: 46 us joined, 54 split).
+template <bool SPLIT = false, typename T>
 __device__ __forceinline__ bool boundary_state(int bt, const T* UL, const double* n,
                                                const Phys& ph, T* Ub)
 {
   double gamma = ph.gamma, gm1 = gamma - 1.0;
+  if constexpr (SPLIT)
+    switch (bt)
+    {
+      case -3: wall_state(-3, UL, n, ph, Ub); return true;
+      case -4: wall_state(-4, UL, n, ph, Ub); return true;
+      case -7: wall_state(-7, UL, n, ph, Ub); return true;
+    }
   switch (bt)
   {
     case -3:

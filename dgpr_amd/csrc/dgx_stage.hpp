@@ -570,7 +570,7 @@ __device__ __forceinline__ void produce_traces(const MeshArgs& mesh, const Phys&
       if (nb < 0)
       {
         double Ub[5];
-        ok = boundary_state(sBt[l][f], U, nv, ph, Ub) && ok;
+        ok = boundary_state<P == 1>(sBt[l][f], U, nv, ph, Ub) && ok;
         TT* B = Tb + (size_t)(-1 - nb) * 5 * NF + fpt;
 #pragma unroll
         for (int r = 0; r < 5; ++r)
