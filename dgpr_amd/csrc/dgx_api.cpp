@@ -399,23 +399,22 @@ dgx_status dgx_create(const dgx_mesh* mesh, const dgx_params* params, dgx_ctx** 
   }
   if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
     return bail("hipMemset(status)", e);
-  if (c->q == 1)
+  // (the other orders have no kernel that shares a face's geometry)
+  int unmatched = 0;
+  if (c->q == 1 && !general_order(c->p, c->q))
   {
-    int bad = 0;
     if ((e = matched_dispatch(mesh_args(c), c->status, c->stream)) != hipSuccess)
       return bail("face check", e);
-    if ((e = hipMemcpyAsync(&bad, c->status, sizeof(int), hipMemcpyDeviceToHost, c->stream)) !=
-        hipSuccess)
+    if ((e = hipMemcpyAsync(&unmatched, c->status, sizeof(int), hipMemcpyDeviceToHost,
+                            c->stream)) != hipSuccess)
       return bail("hipMemcpy(face check)", e);
-    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess)
-      return bail("hipStreamSynchronize", e);
-    c->matched = !bad;
-    if ((e = hipMemsetAsync(c->status, 0, sizeof(int), c->stream)) != hipSuccess)
-      return bail("hipMemset(status)", e);
   }
-  apply_defaults(c);
   if ((e = hipStreamSynchronize(c->stream)) != hipSuccess)
     return bail("hipStreamSynchronize", e);
+  if (unmatched && (e = hipMemset(c->status, 0, sizeof(int))) != hipSuccess)
+    return bail("hipMemset(status)", e);
+  c->matched = !unmatched;
+  apply_defaults(c);
   *out = c;
   return DGX_OK;
 }

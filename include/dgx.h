@@ -423,8 +423,8 @@ dgx_status dgx_set_stored_geometry(dgx_ctx* ctx, int on);
 dgx_status dgx_get_stored_geometry(const dgx_ctx* ctx, int* on);
 /* Whether at every face between two elements, periodic ones included, both
  * elements have the same face up to a translation, to 8 ulps of its largest
- * coordinate (q = 1; 1 for q > 1, where it decides nothing; no counterpart in
- * the reference, which stores each side's metrics).  Where it does not hold (the
+ * coordinate (q = 1, p = 1 to 3; 1 otherwise, where it decides nothing; no
+ * counterpart in the reference, which stores each side's metrics).  Where it does not hold (the
  * two sides of a periodic direction curved differently), every tile takes the
  * neighbour's gradient with the neighbour's own geometry: the FP64 tiled kernel
  * then reads trace records, and tile 0 is the default at p = 1 and 2. */
