@@ -629,9 +629,9 @@ dgx_status dgx_residual(dgx_ctx* c, double* R_host, double* f_host)
 }  // extern "C"
 
 // Stage arguments of one step (time_distributed.cpp:46-102, classic RK4 with
-// an accumulator, Shu-Osher TVD-RK3).  Every stage writes the trace records
-// of its output state, so the next stage (and the next step) reads them
-// instead of recomputing.
+// an accumulator, Shu-Osher TVD-RK3).  Every stage writes what the next stage
+// (and the next step) reads besides its output state: the trace records, or of
+// the kernels that read states the boundary states of inflow and outflow.
 int dgx::stage_plan(const dgx_ctx* c, int scheme, double dt, StageArgs sa[4])
 {
   const int t32 = c->prec != DGX_PREC_FP64;

@@ -227,7 +227,7 @@ __device__ __forceinline__ void face_inverse(const double* jd, const double* t1,
 // affine meshes the neighbour's J^-1 (9), else the four edge vectors of the
 // neighbour along the face direction (12), from which the normal column of
 // its Jacobian follows at every face point; its tangential columns are the
-// own side's, the face being shared.
+// own side's, the face being shared up to a translation (MeshArgs::matched).
 template <bool AFF>
 struct NbrGeo
 {
@@ -381,27 +381,25 @@ __device__ __forceinline__ void face_states(const MeshArgs& mesh, const Phys& ph
                   ph, G, hc);
 }
 
-// This lane's face point in subpass S of a tile (S = NSUB D + the subpass of
-// direction D): face point (a, b) of local face f of tile element l, whose
-// element is e.  Every lane has one: lanes beyond the subpass's faces repeat
-// one of them, and faces of elements past the end of the mesh give values
-// that no node gathers.
-template <int P, int R, int S>
+// This lane's face point in subpass D of a tile, the tile's 2 E faces normal to
+// direction D: face point (a, b) of local face f of tile element l, whose
+// element is e.  Every lane has one (p = 1 and 3: 64 face points a subpass);
+// faces of elements past the end of the mesh give values that no node gathers.
+template <int P, int R, int D>
 struct FaceLane
 {
   using TD = TileDims<P, R>;
-  static constexpr int D = S / TD::NSUB, SP = S % TD::NSUB;
+  static_assert(2 * TD::E * TD::NF == 64, "one face point of the subpass per lane");
   int tid, slot, a, b, l, hi, f, e;
   __device__ __forceinline__ FaceLane(const MeshArgs& mesh, int e0)
   {
     tid  = opaque_tid();
-    slot = (P == 3) ? (tid >> 2) & 3 : min(tid / TD::NF, TD::FPS - 1);
-    const int g = min(SP * TD::FPS + slot, 2 * TD::E - 1);  // element g / 2, side g % 2
+    slot = (P == 3) ? (tid >> 2) & 3 : tid / TD::NF;  // element slot / 2, side slot % 2
     const int t = tid % TD::NF;
     a  = (P == 3) ? tid & 3 : t % TD::N;
     b  = (P == 3) ? tid >> 4 : t / TD::N;
-    l  = g >> 1;
-    hi = g & 1;
+    l  = slot >> 1;
+    hi = slot & 1;
     f  = 2 * D + hi;
     e  = min(e0 + l, mesh.nelem - 1);
   }
@@ -418,16 +416,16 @@ struct FaceData
   double lamL, lamR;
 };
 
-template <int P, int R, int S, bool AFF>
+template <int P, int R, int D, bool AFF>
 __device__ __forceinline__ void face_load(const MeshArgs& mesh, const double* __restrict__ Vin,
                                           const double* __restrict__ lam, const int (*sNb)[6],
                                           int e0, FaceData<P>& fd)
 {
   constexpr int NB = TileDims<P, R>::NB, NF = TileDims<P, R>::NF;
-  const FaceLane<P, R, S> fl(mesh, e0);
+  const FaceLane<P, R, D> fl(mesh, e0);
   // (a boundary face reads its own element here; those values are not used)
   const int nb = sNb[fl.l][fl.f], en = nb >= 0 ? nb : fl.e;
-  line_load<P, FaceLane<P, R, S>::D>(Vin + (size_t)en * 5 * NB, fl.a, fl.b, fd.x);
+  line_load<P, D>(Vin + (size_t)en * 5 * NB, fl.a, fl.b, fd.x);
   // affine meshes: the face's constant coefficient (48 B per element instead
   // of 6 (p+1)^2 doubles, read for the own and the neighbour side)
   const size_t iL = (size_t)fl.e * 6 + fl.f, iR = (size_t)en * 6 + (fl.f ^ 1);
@@ -436,11 +434,11 @@ __device__ __forceinline__ void face_load(const MeshArgs& mesh, const double* __
   fd.lamR = AFF ? mesh.lamf[iR] : lam[iR * NF + fpt];
 }
 
-// Subpass S: both sides' traces and gradient tractions from the states (own
-// from LDS, neighbour in fd), face point physics of whole faces of one
-// direction, the tangential (T) phase and the gather into the nodes'
+// Subpass D: both sides' traces and gradient tractions from the states (own
+// from LDS, neighbour in fd), face point physics of the faces normal to
+// direction D, the tangential (T) phase and the gather into the nodes'
 // accumulators.  next() starts the loads that follow.
-template <int P, int Q, int R, int S, bool AFF, typename Next>
+template <int P, int Q, int R, int D, bool AFF, typename Next>
 __device__ __forceinline__ void state_face_subpass(
     const MeshArgs& mesh, const Phys& ph, const PTab& pt, const QTab& qt,
     const double* __restrict__ Tin, const double (*sV)[5][TileDims<P, R>::NB],
@@ -449,10 +447,9 @@ __device__ __forceinline__ void state_face_subpass(
     const MfTabs& mf, int e0, double (&acc)[R][5], FaceData<P>& fd, Next next)
 {
   using TD = TileDims<P, R>;
-  using FL = FaceLane<P, R, S>;
-  constexpr int N = TD::N, NB = TD::NB, NF = TD::NF, EPR = TD::EPR, FPS = TD::FPS, D = FL::D;
+  constexpr int N = TD::N, NB = TD::NB, NF = TD::NF, EPR = TD::EPR;
   constexpr int T1 = Tang<D>::T1, T2 = Tang<D>::T2;
-  const FL fl(mesh, e0);
+  const FaceLane<P, R, D> fl(mesh, e0);
   const int tid = fl.tid, a = fl.a, b = fl.b, l = fl.l, hi = fl.hi, f = fl.f;
   const int fbase = fl.slot * NF;
 
@@ -539,7 +536,6 @@ __device__ __forceinline__ void state_face_subpass(
     sR[(5 + r) * 64 + tid] = hn[r];
   phase_fence();
   // gather: each node takes its element's low and high face of direction D
-  // when they belong to this subpass
 #pragma unroll
   for (int rr = 0; rr < R; ++rr)
   {
@@ -553,10 +549,8 @@ __device__ __forceinline__ void state_face_subpass(
       for (int h = 0; h < 2; ++h)
       {
         const int gg = 2 * le + h;
-        if (gg / FPS != FL::SP)
-          continue;
-        const int fp = (P == 3) ? idx[T1] + 4 * (gg % FPS) + 16 * idx[T2]
-                                : (gg % FPS) * NF + idx[T2] * N + idx[T1];
+        const int fp = (P == 3) ? idx[T1] + 4 * gg + 16 * idx[T2]
+                                : gg * NF + idx[T2] * N + idx[T1];
         acc[rr][0] += pt.L[h][m] * sR[fp];
 #pragma unroll
         for (int r = 1; r < 5; ++r)
@@ -686,16 +680,13 @@ struct StateLds
 };
 
 // The tiled stage: f_g of the tile's E elements (tile number `block`)
-// fused with the RK stage of StageArgs, then the trace records of the new
-// state (see stage_body_lds for the meaning of every argument; the
-// arithmetic per point is the same), in the LDS region lds
-// (StateLds<P, Q, R>::bytes, 16-byte aligned).
-// CT selects how the volume contractions are done: 0 in FP64 on the vector
-// ALUs; at p = 3, 1 in FP32 and 2 in split BF16 on the matrix cores
-// (dgx_mfma.hpp), the flux physics between them staying FP64.  NORM: the
-// instance that also writes the tile's sum of R^2 to sa.normp (the first
-// stage of a step with its residual norm); kept apart so that the other
-// stages run code without it.
+// fused with the RK stage of StageArgs, then of the new state the boundary
+// states of characteristic faces or, with sa.records, every face's trace record
+// (see stage_body_lds for the meaning of every argument; the arithmetic per
+// point is the same up to rounding), in the LDS region lds
+// (StateLds<P, Q, R, AFF>::bytes, 16-byte aligned).  NORM: the instance that also
+// writes the tile's sum of R^2 to sa.normp (the first stage of a step with its
+// residual norm); kept apart so that the other stages run code without it.
 template <int P, int Q, int R, bool AFF, bool NORM>
 __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
                                               const StageArgs& sa,
@@ -869,12 +860,12 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
   bool ok = true;
   double pbase[R][5], pacc[R][5];  // base state and accumulator, loaded ahead
   auto subpass = [&](auto sc) __attribute__((always_inline)) {
-    constexpr int S = decltype(sc)::value;
-    state_face_subpass<P, Q, R, S, AFF>(
+    constexpr int D = decltype(sc)::value;
+    state_face_subpass<P, Q, R, D, AFF>(
         mesh, ph, pt, qt, Tin, sV, sX, sG, sH, sNb, sBt, sR, mf, e0, acc, fd,
         [&]() __attribute__((always_inline)) {
-          if constexpr (S + 1 < 3 * TD::NSUB)
-            face_load<P, R, S + 1, AFF>(mesh, sa.Vin, lam, sNb, e0, fd);
+          if constexpr (D < 2)
+            face_load<P, R, D + 1, AFF>(mesh, sa.Vin, lam, sNb, e0, fd);
           else
           {
 #pragma unroll
@@ -900,7 +891,6 @@ __device__ __forceinline__ void state_body(const MeshArgs& mesh, const Phys& ph,
   subpass(Const<0>{});
   subpass(Const<1>{});
   subpass(Const<2>{});
-  static_assert(TD::NSUB == 1, "one subpass per direction");
 
   // ---- form f_g and the RK epilogue, one row at a time; with NORM, each
   // row's R = -B3^T W f_g in sR (three passes) and the lane's running sum of
