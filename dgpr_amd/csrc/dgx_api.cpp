@@ -54,19 +54,19 @@ int dgx::default_stage_waves(int p, int q)
 }
 
 // Stage kernel and occupancy target of a context, where the caller has not
-// chosen them.  q = 1 in FP64, faces matched: the state-reading tiled kernel at p = 1 and 3, at
-// 2 waves per SIMD (a 3-wave target spills); against the one-row kernel 1083
-// against 1930 us per RK4 stage on the 64^3 p = 3 cube, 267 against 442 us on
-// the 64^3 p = 1 cube, 137 against 188 us on a 61x37x43 p = 1 channel.  At p = 2
-// its tile of 7 elements, a lane of which takes as long as three of the one-row
-// kernel's, needs more elements to fill the chip: one-row against tiled, affine:
-// 10120 elements 42.2 / 42.4 us, 15000 59.4 / 63.8, 32768 136 / 107; curved: 7220
-// 45.6 / 50.0, 8400 57.1 / 50.5, 15000 83.8 / 78.9, 20160 106 / 87.  The
-// mixed forms and FP64 on unmatched faces: the record-reading tiled kernel at p =
-// 3, q = 1 (mixed on affine meshes 3 waves per SIMD, else 2, where 3 spills).  A
-// target that the caller has chosen and the tiled kernel does not have (1) keeps
-// the one-row kernel.  The general-order
-// kernel (tile 2) outside 1 <= p, q <= 3, the one-row kernel elsewhere.
+// chosen them.  q = 1 in FP64, faces matched: the state-reading tiled kernel at
+// p = 1 and 3, at 2 waves per SIMD (a 3-wave target spills); against the one-row
+// kernel 1083 against 1930 us per RK4 stage on the 64^3 p = 3 cube, 267 against
+// 442 us on the 64^3 p = 1 cube, 137 against 188 us on a 61x37x43 p = 1 channel.
+// At p = 2 its tile of 7 elements, a lane of which takes as long as three of the
+// one-row kernel's, needs more elements to fill the chip: one-row against tiled,
+// affine: 10120 elements 42.2 / 42.4 us, 15000 59.4 / 63.8, 32768 136 / 107;
+// curved: 7220 45.6 / 50.0, 8400 57.1 / 50.5, 15000 83.8 / 78.9, 20160 106 / 87.
+// The mixed forms and FP64 on unmatched faces: the record-reading tiled kernel
+// at p = 3, q = 1 (mixed on affine meshes 3 waves per SIMD, else 2, where 3
+// spills).  A target that the caller has chosen and the tiled kernel does not
+// have (1) keeps the one-row kernel.  The general-order kernel (tile 2) outside
+// 1 <= p, q <= 3, the one-row kernel elsewhere.
 static void apply_defaults(dgx_ctx* c)
 {
   const bool fp64  = c->prec == DGX_PREC_FP64, states = fp64 && c->matched;

@@ -14,11 +14,11 @@
 //     faces normal to z need no gather.
 // What bounds it is FP64 issue at p = 3 (3900 FP64 and 324 matrix instructions
 // per wavefront of 256 nodes at 2 wavefronts per SIMD) together with the traffic
-// of the state arrays (64^3 cube: 4.55 GB per launch, 87 % of the rate of a large
+// of the state arrays (64^3 cube: 4.09 GB per launch, 78 % of the rate of a large
 // copy), and at p = 2 issue and LDS in equal parts.  Per RK4 stage against the
-// 2-element tile of dgx_tile_state.hpp, 64^3 p = 3 cube: 1083 against 1266 us,
-// 48x24x24 p = 3 curved channel (TVD-RK3) 132 against 162 (both with the longer
-// geometry 149 against 162); against the one-row kernel, 32^3 p = 2 cube 107
+// 2-element tile of dgx_tile_state.hpp, 64^3 p = 3 cube: 1083 against 1266 us (1083
+// to 1140 from card to card), 48x24x24 p = 3 curved channel (TVD-RK3) 132 against
+// 162 (both with the longer geometry 149 against 162); against the one-row kernel, 32^3 p = 2 cube 107
 // against 136 us, 30x24x28 p = 2 curved channel 81 against 106.  One wavefront
 // takes 20 us against 11 (p = 3) and 12 us (p = 2) of the others, so small meshes
 // keep those (line_tiled, apply_defaults).  At
@@ -33,9 +33,12 @@ constexpr bool line_order(int p)
 }
 
 // Whether tile 1 in FP64 runs this kernel: always at p = 2; at p = 3 from three
-// wavefronts per SIMD (1024 SIMDs, 4 elements each).  Per RK4 stage, 2-element against 4-element tile: 5202 elements 35.4 against 39.7
-// us, 8000 45.5 / 45.7, 11132 61.8 / 63.1, 32768 160 / 145; curved 5202 41.6 /
-// 47.6, 11132 74.5 / 74.4, 27648 (TVD-RK3) 162 / 149.
+// wavefronts per SIMD (1024 SIMDs, 4 elements each), where it was the quicker one
+// before its epilogue's loads ran ahead.  With them, per RK4 stage, 2-element against
+// 4-element tile: 5202 elements 35.8 against 38.0 us, 8000 47.5 / 45.2, 11132 62.4 /
+// 60.9, 13824 74.4 / 72.9, 32768 163 / 143; curved (TVD-RK3) 5202 40.2 / 42.0, 8000
+// 52.8 / 48.0, 11132 71.9 / 67.2, 27648 154 / 135: from 8000 on it is 2 to 9 %
+// quicker below the line too.
 constexpr bool line_tiled(int p, int nelem)
 {
   return p == 2 || (p == 3 && nelem >= 12288);
