@@ -153,7 +153,7 @@ hipError_t tile_rhs_dispatch(int p, const MeshArgs& m, const Phys& ph, const Sta
 hipError_t boundary_dispatch(int p, const MeshArgs& m, const Phys& ph, const double* V,
                              double* Tout, int* status, hipStream_t st);
 hipError_t upload_tables_tile(const PTab* pt, const QTab* qt);
-// q = 1: *flag (device) becomes 1 if the two elements at some face, periodic
+// q = 1: *flag (device or pinned host memory) becomes 1 if the two elements at some face, periodic
 // ones included, have faces that differ by more than a translation
 hipError_t matched_dispatch(const MeshArgs& m, int* flag, hipStream_t st);
 // affine meshes: arec (affine_record_doubles(nelem)) of every element

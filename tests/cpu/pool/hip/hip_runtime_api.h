@@ -87,6 +87,12 @@ enum hipMemcpyKind
   hipMemcpyDefault
 };
 constexpr unsigned hipStreamNonBlocking = 1;
+constexpr unsigned hipHostMallocPortable = 1;
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned)
+{
+  *p = std::malloc(n);
+  return hipSuccess;
+}
 inline const char* hipGetErrorString(hipError_t e)
 {
   return e == hipErrorOutOfMemory ? "out of memory" : "error";
